@@ -30,6 +30,7 @@ HIP_SOURCES = [
     "set/assemble.hip",
     "set/batch.hip",
     "set/generic.hip",
+    "set/hex27.hip",
     "set/sideset.hip",
     "learned/lq_assemble.hip",
     "learned/mlp.hip",

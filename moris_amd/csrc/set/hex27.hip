@@ -1,0 +1,561 @@
+// hex27.hip -- element matrices of HEX27 IP cells on the generic path.
+//
+// The moment integrand of a box HEX27 cell, dN_a/dx_i dN_b/dx_j (two triquadratic factors, one
+// differentiated each), is a polynomial of degree <= 4 in each axis.  Its sum over a cell's
+// integration points (TET_35 on the XTK sub-tets, w* = w detJ, points with detJ < -1e-6 skipped,
+// cl_FEM_Element_Bulk.cpp:258-355; HEX_3x3x3 on whole cells) is therefore a fixed linear function of
+// the cell's 125 moments of degree <= 4 per axis, and factorises over the axes.
+// Both quadrature options take this route, in FP64 at either precision option: it is the point sum
+// in another order, and closer to that sum than a point-wise accumulation of M (K within 1.2e-16 ..
+// 2.9e-16 of sums in 80-bit long double, against 7.8e-16 .. 2.1e-15).  32^3 cut cells, elasticity, p = 2 (1.1M
+// sub-tets, 37.8M points): element kernels 11.8 ms with M accumulated point by point on 21 FP64 MFMA
+// tiles, 1.4 ms here.
+//
+//   k_hex27_moments    one wavefront per element: the 125 moments of a cut cell on FP64 MFMA, one
+//                      16 x 16 x 4 product per 4 points (whole cells: closed form).
+//   k_hex27_tensor     elements whose T is a tensor product of one 1D matrix per axis (nodal rows,
+//                      untruncated p = 2 B-splines): T folded into the 1D factor tables, so that K_e
+//                      comes straight from the moments; one block of 4 wavefronts per element.
+//   k_hex27_general    any other T (truncated hierarchical rows): K_p from the moments with the
+//                      Lagrange tables, K_e = T^T K_p T on FP64 MFMA.
+// K_e goes to the element's slot of the pool, or (scatter mode) is added into the CSR values.
+#include <hip/hip_runtime.h>
+
+#include "../common/fem_tables.hpp"
+#include "set_state.hpp"
+
+namespace mgpu {
+
+namespace {
+
+typedef double doublex4_t __attribute__((ext_vector_type(4)));
+
+// ------------------------------------------------------------------------------------------------
+// 1D tables.  The moments are taken in the basis {l_0, l_1, l_2, c, c x} of each axis: the quadratic
+// Lagrange functions of the nodes -1, 0, 1 and c = x^3 - x, which vanishes there.  A polynomial of degree
+// <= 4 is sum_n p(n - 1) l_n + p_3 c + p_4 c x, so the tables of the (dyadic) 1D functions below are
+// exact, and the basis is well conditioned.  Monomials cost 4e-15 on K of nodal rows; the degree-4
+// Lagrange basis through the Gauss-Legendre nodes, with rounded tables, is as accurate as this one but
+// takes three times the arithmetic per point.
+// kQuad1D: polynomial coefficients [function][power] of l_0 .. l_2 and of the uniform quadratic B-splines
+// of a cell (those of the T rows: vertex rows 1/2 1/2, mid rows 1/8 3/4 1/8, times l_0 .. l_2).
+// ------------------------------------------------------------------------------------------------
+constexpr double kQuad1D[2][3][3] = {
+    {{0.0, -0.5, 0.5}, {1.0, 0.0, -1.0}, {0.0, 0.5, 0.5}},
+    {{0.125, -0.25, 0.125}, {0.75, 0.0, -0.25}, {0.125, 0.25, 0.125}},
+};
+
+// v[kind][tau][3 alpha + beta][m]: coefficients of F_alpha F_beta in the basis; tau = 2 [alpha differentiated] +
+// [beta differentiated]; kind 0 Lagrange, 1 B-spline.
+struct AxisTables {
+    double v[2][4][9][5];
+    constexpr AxisTables() : v{} {
+        for (int kind = 0; kind < 2; ++kind)
+            for (int tau = 0; tau < 4; ++tau)
+                for (int al = 0; al < 3; ++al)
+                    for (int be = 0; be < 3; ++be) {
+                        double p[3] = {}, q[3] = {}, r[5] = {};
+                        for (int n = 0; n < 3; ++n) {
+                            if (tau & 2) { if (n > 0) p[n - 1] = n * kQuad1D[kind][al][n]; }
+                            else p[n] = kQuad1D[kind][al][n];
+                            if (tau & 1) { if (n > 0) q[n - 1] = n * kQuad1D[kind][be][n]; }
+                            else q[n] = kQuad1D[kind][be][n];
+                        }
+                        for (int a = 0; a < 3; ++a)
+                            for (int b = 0; b < 3; ++b) r[a + b] += p[a] * q[b];
+                        double* o = v[kind][tau][3 * al + be];
+                        o[0] = r[0] - r[1] + r[2] - r[3] + r[4];
+                        o[1] = r[0];
+                        o[2] = r[0] + r[1] + r[2] + r[3] + r[4];
+                        o[3] = r[3];
+                        o[4] = r[4];
+                    }
+    }
+};
+__constant__ const AxisTables kAxis{};
+// integrals of the basis over [-1, 1]
+__constant__ const double kBasisInt[5] = {1.0 / 3.0, 4.0 / 3.0, 1.0 / 3.0, 0.0, -4.0 / 15.0};
+
+// ------------------------------------------------------------------------------------------------
+// k_hex27_moments: mom[e][(i 5 + j) 5 + k] = sum_ip w* g_i(x) g_j(y) g_k(z), g the basis above.  64 points at
+// a time, a lane a point: mapped, its 15 row values w* g_i(x) l_n(y) and 10 column values g_k(z) {1, c(y)}
+// put in LDS 32 points at a time (stride 25 doubles: distinct banks; 6.4 KB, so that registers and not LDS
+// bound the wavefronts in flight), then 8 MFMA steps of 4 points with one 8-byte read per operand.
+// Splitting g_j over rows and columns lets one 16 x 16 tile hold all 125 moments (rows (i, j), columns k
+// would take two, 25 x 5 of 32 x 16 used): sum_n l_n = 1 and l_2 - l_0 = y give c and c y.  Bound by the FP64
+// units, MFMA and the per-point arithmetic together: 0.67 ms for 32^3 cut cells.
+// ------------------------------------------------------------------------------------------------
+constexpr int kMomPt = 25;
+__device__ inline void hex27_basis(double x, double* v) {
+    const double x2 = x * x;
+    v[0] = 0.5 * (x2 - x);
+    v[1] = 1.0 - x2;
+    v[2] = 0.5 * (x2 + x);
+    v[3] = -x * v[1];
+    v[4] = x * v[3];
+}
+__global__ __launch_bounds__(64) void k_hex27_moments(GenView g, double* mom) {
+    __shared__ double rec[32 * kMomPt];
+    const int e = g.order ? g.order[blockIdx.x] : (int)blockIdx.x;
+    const int lane = threadIdx.x;
+    double hh[3];
+    for (int d = 0; d < 3; ++d) hh[d] = g.ip_box[(size_t)e * 6 + 3 + d];
+    const int ig0 = g.ig_ptr[e], nsub = g.ig_ptr[e + 1] - ig0;
+    double* out = mom + (size_t)e * kHex27Moments;
+    if (nsub == 0) {
+        // whole cell: products of 1D integrals (HEX_3x3x3 integrates the basis exactly)
+        const double detJ = (0.5 * hh[0]) * (0.5 * hh[1]) * (0.5 * hh[2]);
+        for (int t = lane; t < kHex27Moments; t += 64) {
+            out[t] = detJ * (kBasisInt[t / 25] * kBasisInt[(t / 5) % 5] * kBasisInt[t % 5]);
+        }
+        return;
+    }
+    const int npts = nsub * kTet35Points;
+    const int r16 = lane & 15, kq = lane >> 4;
+    const int ao = kq * kMomPt + (r16 < 15 ? r16 : 0);
+    const int bo = kq * kMomPt + 15 + (r16 < 10 ? r16 : 0);
+    // summed per chunk (two chains), then over the chunks: shorter chains of rounded additions
+    doublex4_t tot = {0.0, 0.0, 0.0, 0.0}, acc0 = tot, acc1 = tot;
+    // the lane's point of the coming chunk: sub-tet vertices and rule (lanes past the end: point 0
+    // with weight 0), requested before the matrix work of the chunk before it
+    const double vol6 = (0.5 * hh[0]) * (0.5 * hh[1]) * (0.5 * hh[2]) / 6.0;
+    double X[12], bq[4];
+    auto request = [&](int p0) {
+        const int ip = p0 + lane, ipc = ip < npts ? ip : 0;
+        const int t = ipc / kTet35Points, q = ipc - kTet35Points * t;
+        const double2* X2 = reinterpret_cast<const double2*>(g.ig_xi + (size_t)(ig0 + t) * 12);
+#pragma unroll
+        for (int n = 0; n < 6; ++n) {
+            const double2 v = X2[n];
+            X[2 * n] = v.x;
+            X[2 * n + 1] = v.y;
+        }
+        bq[0] = kTet35Xi[q][0];
+        bq[1] = kTet35Xi[q][1];
+        bq[2] = kTet35Xi[q][2];
+        bq[3] = ip < npts ? kTet35W[q] : 0.0;
+    };
+    request(0);
+    for (int p0 = 0; p0 < npts; p0 += 64) {
+        // vertex 2 plus the rule's coordinates along the edges J to the others (the same affine map as
+        // the vertex weights (xi0, xi1, 1 - xi0 - xi1 - xi2, xi2))
+        double x[3], J[3][3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            J[0][d] = X[d] - X[6 + d];
+            J[1][d] = X[3 + d] - X[6 + d];
+            J[2][d] = X[9 + d] - X[6 + d];
+            x[d] = X[6 + d] + bq[0] * J[0][d] + bq[1] * J[1][d] + bq[2] * J[2][d];
+        }
+        const double detJ = (J[0][0] * (J[1][1] * J[2][2] - J[2][1] * J[1][2]) -
+                             J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
+                             J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0])) * vol6;
+        const double w = detJ < kDetJLowerLimit ? 0.0 : bq[3] * detJ;
+        double gx[5], gy[5], gz[5], av[15], cv[5];
+        hex27_basis(x[0], gx);
+        hex27_basis(x[1], gy);
+        hex27_basis(x[2], gz);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            const double wg = w * gx[i];
+#pragma unroll
+            for (int n = 0; n < 3; ++n) av[3 * i + n] = wg * gy[n];
+            cv[i] = gz[i] * gy[3];
+        }
+        request(p0 + 64);   // (past the last chunk: point 0, unused)
+        tot += acc0 + acc1;
+        acc0 = acc1 = doublex4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            __syncthreads();   // the previous records are read
+            if ((lane >> 5) == half) {
+                double* pp = rec + (lane & 31) * kMomPt;
+#pragma unroll
+                for (int n = 0; n < 15; ++n) pp[n] = av[n];
+#pragma unroll
+                for (int k = 0; k < 5; ++k) {
+                    pp[15 + 2 * k] = gz[k];
+                    pp[16 + 2 * k] = cv[k];
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < 8; s += 2) {
+                const double* ps = rec + 4 * s * kMomPt;
+                acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(ps[ao], ps[bo], acc0, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(ps[4 * kMomPt + ao], ps[4 * kMomPt + bo], acc1, 0, 0, 0);
+            }
+        }
+    }
+    // the tile through LDS: register n of a lane holds row lane / 16 + 4 n = 3 i + l, column lane % 16 =
+    // 2 k + [times c]; the last row and columns 10 .. 15 repeat others
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < 4; ++n) rec[(kq + 4 * n) * 17 + r16] = tot[n] + (acc0[n] + acc1[n]);
+    __syncthreads();
+    for (int t = lane; t < kHex27Moments; t += 64) {
+        const int i = t / 25, j = (t / 5) % 5, k = t % 5;
+        const double* D = rec + 3 * i * 17 + 2 * k + (j >= 3 ? 1 : 0);
+        out[t] = j < 3 ? D[17 * j] : (j == 3 ? (D[0] + D[17]) + D[34] : D[34] - D[0]);
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+// M from the moments, by sum factorisation over the axes: block p = (i, j), i <= j, of
+//   M[(i,a),(j,b)] = s_i s_j sum_{x,y,z <= 4} mom_xyz P_0(a_0,b_0; x) P_1(a_1,b_1; y) P_2(a_2,b_2; z),
+// s_i = 2 / h_i, contracted over z, y, x.  Wavefronts take whole tasks, so that the 1D tables are
+// scalar loads.  Result G[p][a][b] in LDS, a = (a_0 3 + a_1) 3 + a_2; NF == 1: the sum of the three
+// diagonal blocks only.  LDS: mom, Z[zt][x 5 + y][ab_2], Y[block][x][ab_1][ab_2], then G over Z and Y.
+// ------------------------------------------------------------------------------------------------
+template <int NF> struct Hex27Blocks;
+template <> struct Hex27Blocks<1> {
+    static constexpr int n = 3;
+    static constexpr int i[3] = {0, 1, 2}, j[3] = {0, 1, 2};
+};
+template <> struct Hex27Blocks<3> {
+    static constexpr int n = 6;
+    static constexpr int i[6] = {0, 0, 0, 1, 1, 2}, j[6] = {0, 1, 2, 1, 2, 2};
+};
+constexpr int kSfZ = 128, kSfY = kSfZ + 3 * 225;
+template <int NF>
+constexpr int sf_lds() {   // doubles
+    return NF == 3 ? 6 * 729 : kSfY + 3 * 405;
+}
+static_assert(kSfY + 6 * 405 <= 6 * 729, "the contraction stages fit the space of G");
+
+template <int NF>
+__device__ inline void sf_moments(const GenView& g, const double* mom, int e, int kind, double* lds) {
+    using B = Hex27Blocks<NF>;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    double* Z = lds + kSfZ;
+    double* Y = lds + kSfY;
+    if (tid < kHex27Moments) lds[tid] = mom[(size_t)e * kHex27Moments + tid];
+    double sc[3];
+    for (int d = 0; d < 3; ++d) sc[d] = 2.0 / g.ip_box[(size_t)e * 6 + 3 + d];
+    __syncthreads();
+    // z: task zt = wave, tau_2 = 0, 1, 3 (alpha alone is differentiated on axis 2 in no block i <= j)
+    if (wave < 3 && lane < 25) {
+        const double(*P)[5] = kAxis.v[kind][wave == 2 ? 3 : wave];
+        double m[5];
+#pragma unroll
+        for (int k = 0; k < 5; ++k) m[k] = lds[lane * 5 + k];
+#pragma unroll
+        for (int ab = 0; ab < 9; ++ab) {
+            double v = 0.0;
+#pragma unroll
+            for (int k = 0; k < 5; ++k) v += m[k] * P[ab][k];
+            Z[wave * 225 + lane * 9 + ab] = v;
+        }
+    }
+    __syncthreads();
+    // y: task block p, lane (x, ab_2)
+    for (int p = wave; p < B::n; p += 4) {
+        const int i = NF == 1 ? p : (p >= 3) + (p >= 5), j = NF == 1 ? p : (p < 3 ? p : (p < 5 ? p - 2 : 2));
+        const int tau1 = 2 * (i == 1) + (j == 1), tau2 = 2 * (i == 2) + (j == 2);
+        const double(*P)[5] = kAxis.v[kind][tau1];
+        if (lane < 45) {
+            const int x = lane / 9, ab2 = lane - 9 * x;
+            const double* Zp = Z + (tau2 == 3 ? 2 : tau2) * 225 + x * 45 + ab2;
+            double z[5];
+#pragma unroll
+            for (int y = 0; y < 5; ++y) z[y] = Zp[9 * y];
+#pragma unroll
+            for (int ab1 = 0; ab1 < 9; ++ab1) {
+                double v = 0.0;
+#pragma unroll
+                for (int y = 0; y < 5; ++y) v += z[y] * P[ab1][y];
+                Y[p * 405 + x * 81 + ab1 * 9 + ab2] = v;
+            }
+        }
+    }
+    __syncthreads();
+    // x: task (p, half), lane ab_12; the results stay in registers until Y is read by every task
+    constexpr int NT = NF == 3 ? 3 : 1;
+    double r[NT][9];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+#pragma unroll
+        for (int q = 0; q < 9; ++q) r[n][q] = 0.0;
+        const int task = wave + 4 * n;
+        if (NF == 1 && task >= 2) continue;
+        const int ab12 = (task & 1) * 64 + lane;
+        if (ab12 >= 81) continue;
+#pragma unroll
+        for (int pp = 0; pp < (NF == 3 ? 1 : 3); ++pp) {
+            const int p = NF == 3 ? task >> 1 : pp;
+            const int i = NF == 1 ? p : (p >= 3) + (p >= 5), j = NF == 1 ? p : (p < 3 ? p : (p < 5 ? p - 2 : 2));
+            const int tau0 = 2 * (i == 0) + (j == 0);
+            const double(*P)[5] = kAxis.v[kind][tau0];
+            const double s2 = (i == 0 ? sc[0] : (i == 1 ? sc[1] : sc[2])) * (j == 0 ? sc[0] : (j == 1 ? sc[1] : sc[2]));
+            double y[5];
+#pragma unroll
+            for (int x = 0; x < 5; ++x) y[x] = s2 * Y[p * 405 + x * 81 + ab12];
+#pragma unroll
+            for (int ab0 = 0; ab0 < 9; ++ab0)
+#pragma unroll
+                for (int x = 0; x < 5; ++x) r[n][ab0] += y[x] * P[ab0][x];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int task = wave + 4 * n;
+        if (NF == 1 && task >= 2) continue;
+        const int ab12 = (task & 1) * 64 + lane;
+        if (ab12 >= 81) continue;
+        const int p = NF == 3 ? task >> 1 : 0;
+        const int a12 = (ab12 / 27) * 3 + (ab12 / 3) % 3, b12 = ((ab12 / 9) % 3) * 3 + ab12 % 3;
+#pragma unroll
+        for (int ab0 = 0; ab0 < 9; ++ab0) lds[p * 729 + ((ab0 / 3) * 9 + a12) * 27 + (ab0 % 3) * 9 + b12] = r[n][ab0];
+    }
+    __syncthreads();
+}
+
+// Entry (f, a), (h, b) of K as a sum of three coefficients times entries of G:
+//   f == h: c0 M_ff[a,b] + cs (M_ii + M_jj)[a,b];  f != h: c1 M_fh[a,b] + cs M_hf[a,b], M_hf[a,b] = M_fh[b,a]
+// (isotropic D, block (f, h) of B^T D B; diffusion: the material times the summed diagonal blocks).
+// The three entries sit at base[n] + a sa[n] + b sb[n].
+struct KTerms {
+    double c[3];
+    int base[3], sa[3], sb[3];
+};
+template <int NF>
+__device__ inline KTerms k_terms(int f, int h, double c0, double c1, double cs) {
+    KTerms k;
+    if (NF == 1) {
+        k.c[0] = c0;
+        k.c[1] = k.c[2] = 0.0;
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            k.base[n] = 0;
+            k.sa[n] = 27;
+            k.sb[n] = 1;
+        }
+        return k;
+    }
+    // block index of (i, j), i <= j: 0 (0,0) 1 (0,1) 2 (0,2) 3 (1,1) 4 (1,2) 5 (2,2)
+    const int lo = min(f, h), hi = max(f, h);
+    const int pf = f == 0 ? 0 : (f == 1 ? 3 : 5);
+    const int pfh = lo == 0 ? hi : (lo == 1 ? hi + 2 : 5);
+    const bool dg = f == h, up = f < h;
+    k.c[0] = dg ? c0 : c1;
+    k.c[1] = cs;
+    k.c[2] = dg ? cs : 0.0;
+    k.base[0] = 729 * (dg ? pf : pfh);
+    k.base[1] = 729 * (dg ? (f == 0 ? 3 : 0) : pfh);
+    k.base[2] = 729 * (dg ? (f == 2 ? 3 : 5) : pfh);
+    k.sa[0] = dg || up ? 27 : 1;
+    k.sb[0] = dg || up ? 1 : 27;
+    k.sa[1] = dg || !up ? 27 : 1;
+    k.sb[1] = dg || !up ? 1 : 27;
+    k.sa[2] = k.sa[0];
+    k.sb[2] = k.sb[0];
+    return k;
+}
+
+template <int NF>
+__device__ inline void hex27_material(const GenView& g, int e, double& c0, double& c1, double& cs) {
+    if (NF == 1) {
+        c0 = g.material[e];
+        c1 = cs = 0.0;
+    } else {
+        double D[6][6];
+        elastic_D<3>(g.material[2 * e], g.material[2 * e + 1], D);
+        c0 = D[0][0];
+        c1 = D[0][1];
+        cs = D[5][5];
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+// k_hex27_tensor: K_e of elements whose T is a tensor product (t_perm[e][27] = 1 nodal, 2 B-spline;
+// t_perm[e][y] the tensor index of the element's adof y).  Threads 0 .. 3 NA - 1 hold a column of K_e and
+// write NF rows' worth of consecutive values per step (stores of whole lines).  Without the products by T
+// and their LDS space four blocks instead of two fit a CU: 0.74 ms for 32^3 elements of 81 x 81 (1.7 GB
+// written), against 1.9 ms on the general path.
+// ------------------------------------------------------------------------------------------------
+template <int NF, bool SCATTER>
+__global__ __launch_bounds__(256) void k_hex27_tensor(GenView g, const int32_t* els, const double* mom, double* vals) {
+    constexpr int NA = NF * 27;
+    constexpr int RPS = NF == 3 ? 3 : 9;   // rows per step; divides 27
+    static_assert(RPS * NA <= 256 && 27 % RPS == 0, "a step's rows lie in one field block");
+    __shared__ double lds[sf_lds<NF>()];
+    __shared__ int perm[27];
+    const int e = els[blockIdx.x];
+    const int tid = threadIdx.x;
+    const uint8_t* pm = g.t_perm + (size_t)e * kHex27PermStride;
+    if (tid < 27) perm[tid] = pm[tid];
+    sf_moments<NF>(g, mom, e, __builtin_amdgcn_readfirstlane((int)pm[27]) - 1, lds);
+    double c0, c1, cs;
+    hex27_material<NF>(g, e, c0, c1, cs);
+    if (tid >= RPS * NA) return;
+    const int rs = tid / NA, col = tid - NA * rs, h = col / 27, y = col - 27 * h;
+    const int b = perm[y];
+    double* ke = SCATTER ? nullptr : g.ke + g.ke_off[e];
+    const int32_t* rows = SCATTER ? g.topo + g.topo_ptr[e] : nullptr;
+    const uint16_t* rk = SCATTER ? g.rank + g.rank_off[e] : nullptr;
+    for (int f = 0; f < NF; ++f) {
+        const KTerms k = k_terms<NF>(f, h, c0, c1, cs);
+        const double* G0 = lds + k.base[0] + b * k.sb[0];
+        const double* G1 = lds + k.base[1] + b * k.sb[1];
+        const double* G2 = lds + k.base[2] + b * k.sb[2];
+#pragma unroll 3
+        for (int n = 0; n < 27 / RPS; ++n) {
+            const int x = RPS * n + rs, a = perm[x];
+            double v = k.c[0] * G0[a * k.sa[0]];
+            if (NF > 1) v += k.c[1] * G1[a * k.sa[1]] + k.c[2] * G2[a * k.sa[2]];
+            if constexpr (SCATTER) {
+                const int32_t row = rows[f * 27 + x], r0 = g.row_ptr[row], len = (g.row_ptr[row + 1] - r0) / NF;
+                unsafeAtomicAdd(vals + r0 + h * len + rk[x * 27 + y], v);
+            } else {
+                ke[(f * 27 + RPS * n) * NA + tid] = v;
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+// k_hex27_general: K_e = T^T K_p T per (f, h) block on FP64 MFMA (16 x 16 tiles, k in steps of 4, operands
+// from LDS; A: row lane % 16, k = lane / 16; B: k = lane / 16, column lane % 16; result register j of a
+// lane: row lane / 16 + 4 j, column lane % 16): W = K_p[f][h] T (27 x na_t), its K_p operand formed
+// from G, then T^T W.  K_e being symmetric only the blocks h >= f are computed, block (h, f) is their
+// mirror image.
+// In scatter mode entry (x, y) of block (f, h) sits in row topo[f na_t + x], field block h of that row,
+// at the rank of adof y among the row adof's neighbours.  No other element of the colour touches
+// the row, so the adds are hardware FP64 atomics without return (no old value travels to the CU)
+// that still reach every value in colour order: the same sums on every call.
+// ------------------------------------------------------------------------------------------------
+template <int NF, bool SCATTER>
+__global__ __launch_bounds__(256) void k_hex27_general(GenView g, const int32_t* els, const double* mom, double* vals) {
+    constexpr int NB = 27;
+    constexpr int SF = sf_lds<NF>();
+    __shared__ double lds[SF + 2 * NB * kHex27MaxAdofsPerType];
+    const int e = els[blockIdx.x];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int col16 = lane & 15, kq = lane >> 4;
+    // dense element-local T (27 x na_t, the same for every dof type)
+    double* Tt = lds + SF;
+    double* W = Tt + NB * kHex27MaxAdofsPerType;
+    const int na_t = g.na_t[e];
+    const int NA = NF * na_t;
+    for (int idx = tid; idx < NB * na_t; idx += 256) Tt[idx] = 0.0;
+    __syncthreads();
+    if (tid < NB)
+        for (int q = g.t_ptr[e * NB + tid]; q < g.t_ptr[e * NB + tid + 1]; ++q) Tt[tid * na_t + g.t_col[q]] += g.t_w[q];
+    sf_moments<NF>(g, mom, e, 0, lds);
+    double c0, c1, cs;
+    hex27_material<NF>(g, e, c0, c1, cs);
+    // HEX27 basis of row / column operand n of a tile -> its tensor index in G
+    auto half = [&](int a) { return (kHex27Half[a][0] * 3 + kHex27Half[a][1]) * 3 + kHex27Half[a][2]; };
+    int ah[2], bh[(NB + 3) / 4];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) ah[mt] = half(min(mt * 16 + col16, NB - 1));
+#pragma unroll
+    for (int ks = 0; ks < (NB + 3) / 4; ++ks) bh[ks] = half(min(4 * ks + kq, NB - 1));
+    double* ke = SCATTER ? nullptr : g.ke + g.ke_off[e];
+    const int32_t* rows = SCATTER ? g.topo + g.topo_ptr[e] : nullptr;
+    const uint16_t* rk = SCATTER ? g.rank + g.rank_off[e] : nullptr;
+    const int n_nt = (na_t + 15) / 16;   // 16-column tiles of T, W and K_e
+    for (int f = 0; f < NF; ++f)
+        for (int hb = f; hb < NF; ++hb) {
+            const KTerms kt = k_terms<NF>(f, hb, c0, c1, cs);
+            for (int tile = wave; tile < 2 * n_nt; tile += 4) {
+                const int mt = tile / n_nt, nt = tile - n_nt * (tile / n_nt);
+                const int arow = mt * 16 + col16, bcol = nt * 16 + col16;   // a; y
+                const int a = mt ? ah[1] : ah[0];
+                doublex4_t c4 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int ks = 0; ks < (NB + 3) / 4; ++ks) {
+                    const int k = 4 * ks + kq;   // b
+                    double av = kt.c[0] * lds[kt.base[0] + a * kt.sa[0] + bh[ks] * kt.sb[0]];
+                    if (NF > 1)
+                        av += kt.c[1] * lds[kt.base[1] + a * kt.sa[1] + bh[ks] * kt.sb[1]] +
+                              kt.c[2] * lds[kt.base[2] + a * kt.sa[2] + bh[ks] * kt.sb[2]];
+                    av = (arow < NB && k < NB) ? av : 0.0;
+                    const double bv = (k < NB && bcol < na_t) ? Tt[k * na_t + bcol] : 0.0;
+                    c4 = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, c4, 0, 0, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int r = mt * 16 + kq + 4 * j;
+                    if (r < NB && bcol < na_t) W[r * na_t + bcol] = c4[j];
+                }
+            }
+            __syncthreads();
+            for (int tile = wave; tile < n_nt * n_nt; tile += 4) {
+                const int mt = tile / n_nt, nt = tile - n_nt * (tile / n_nt);
+                const int xrow = mt * 16 + col16, ycol = nt * 16 + col16;   // x; y
+                // scatter mode: the tile's CSR positions (and those of its mirror image in block
+                // (h, f)) are requested before its MFMA work, which hides their chain of dependent
+                // loads
+                [[maybe_unused]] int pos[4], pos2[4];
+                if constexpr (SCATTER) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int x = mt * 16 + kq + 4 * j;
+                        pos[j] = pos2[j] = -1;
+                        if (x < na_t && ycol < na_t) {
+                            const int32_t row = rows[f * na_t + x];
+                            const int32_t r0 = g.row_ptr[row], len = (g.row_ptr[row + 1] - r0) / NF;
+                            pos[j] = r0 + hb * len + rk[x * na_t + ycol];
+                            if (hb != f) {
+                                const int32_t row2 = rows[hb * na_t + ycol];
+                                const int32_t r2 = g.row_ptr[row2], len2 = (g.row_ptr[row2 + 1] - r2) / NF;
+                                pos2[j] = r2 + f * len2 + rk[ycol * na_t + x];
+                            }
+                        }
+                    }
+                }
+                doublex4_t c4 = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int ks = 0; ks < (NB + 3) / 4; ++ks) {
+                    const int k = 4 * ks + kq;   // a
+                    const double av = (k < NB && xrow < na_t) ? Tt[k * na_t + xrow] : 0.0;
+                    const double bv = (k < NB && ycol < na_t) ? W[k * na_t + ycol] : 0.0;
+                    c4 = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, c4, 0, 0, 0);
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int x = mt * 16 + kq + 4 * j;
+                    if constexpr (SCATTER) {
+                        if (pos[j] >= 0) unsafeAtomicAdd(vals + pos[j], c4[j]);
+                        if (pos2[j] >= 0) unsafeAtomicAdd(vals + pos2[j], c4[j]);
+                    } else if (x < na_t && ycol < na_t) {
+                        ke[(size_t)(f * na_t + x) * NA + hb * na_t + ycol] = c4[j];
+                        if (hb != f) ke[(size_t)(hb * na_t + ycol) * NA + f * na_t + x] = c4[j];
+                    }
+                }
+            }
+            __syncthreads();
+        }
+}
+
+template <int NF, bool SCATTER>
+void launch_elements_t(const GenView& g, int32_t n_tensor, int32_t n_general, const int32_t* els, const double* mom,
+                       double* vals, hipStream_t s) {
+    if (n_tensor > 0)
+        hipLaunchKernelGGL((k_hex27_tensor<NF, SCATTER>), dim3((unsigned)n_tensor), dim3(256), 0, s, g, els, mom, vals);
+    if (n_general > 0)
+        hipLaunchKernelGGL((k_hex27_general<NF, SCATTER>), dim3((unsigned)n_general), dim3(256), 0, s, g,
+                           els + n_tensor, mom, vals);
+}
+
+}  // namespace
+
+void launch_hex27_moments(const GenView& g, double* mom, hipStream_t s) {
+    hipLaunchKernelGGL(k_hex27_moments, dim3((unsigned)g.n_el), dim3(64), 0, s, g, mom);
+}
+
+void launch_hex27_elements(const GenView& g, int nf, bool scatter, int32_t n_tensor, int32_t n_general,
+                           const int32_t* els, const double* mom, double* vals, hipStream_t s) {
+    if (nf == 1) {
+        if (scatter) launch_elements_t<1, true>(g, n_tensor, n_general, els, mom, vals, s);
+        else launch_elements_t<1, false>(g, n_tensor, n_general, els, mom, vals, s);
+    } else {
+        if (scatter) launch_elements_t<3, true>(g, n_tensor, n_general, els, mom, vals, s);
+        else launch_elements_t<3, false>(g, n_tensor, n_general, els, mom, vals, s);
+    }
+}
+
+}  // namespace mgpu

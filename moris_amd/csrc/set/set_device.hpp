@@ -98,12 +98,14 @@ struct GenView {
     // scatter mode (HEX27 sets without a K_e pool)
     const int32_t* topo;         // rows of each element, nf * na_t from topo_ptr[e]
     const int64_t* topo_ptr;     // [n_el + 1]
-    const int32_t* colour_el;    // [n_el] elements by colour
     // gather mode: the processing order of the element workgroups (most sub-cells first), or
     // null for element order; the autotuner picks one
     const int32_t* order;
     const int64_t* rank_off;     // [n_el + 1]
     const uint16_t* rank;        // [na_t][na_t] per element: column of adof y among adof x's neighbours
+    // HEX27 sets: per element the tensor index of each adof where T is a tensor product (entry 27: 1
+    // nodal rows, 2 uniform quadratic B-splines, 0 any other T)
+    const uint8_t* t_perm;       // [n_el][kHex27PermStride]
 };
 
 // Storage of the cut-element matrices: FP64 on the plain path, FP32 with the FP32 integrands.

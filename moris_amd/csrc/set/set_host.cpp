@@ -37,6 +37,38 @@ void parallel_for(int64_t n, F f) {
 }
 }  // namespace
 
+// The tensor form of a HEX27 element's T (27 x 27, dense in D), if it has one: every column equal,
+// bit for bit, to a product T1[a_0][b_0] T1[a_1][b_1] T1[a_2][b_2], each (b_0, b_1, b_2) once.  The
+// entries of T1 are dyadic, so the products are exact in any order.
+static void hex27_tensor_form(const double* D, uint8_t* perm) {
+    static const double T1[2][3][3] = {{{1.0, 0.0, 0.0}, {0.0, 1.0, 0.0}, {0.0, 0.0, 1.0}},
+                                       {{0.5, 0.5, 0.0}, {0.125, 0.75, 0.125}, {0.0, 0.5, 0.5}}};
+    for (int kind = 0; kind < 2; ++kind) {
+        bool used[27] = {};
+        int y = 0;
+        for (; y < 27; ++y) {
+            int c = 0;
+            for (; c < 27; ++c) {
+                if (used[c]) continue;
+                int a = 0;
+                for (; a < 27; ++a) {
+                    const int* hf = kHex27Half[a];
+                    if (D[a * 27 + y] != T1[kind][hf[0]][c / 9] * T1[kind][hf[1]][(c / 3) % 3] * T1[kind][hf[2]][c % 3]) break;
+                }
+                if (a == 27) break;
+            }
+            if (c == 27) break;
+            used[c] = true;
+            perm[y] = (uint8_t)c;
+        }
+        if (y == 27) {
+            perm[27] = (uint8_t)(kind + 1);
+            return;
+        }
+    }
+    perm[27] = 0;
+}
+
 // Generic path: element topology of any T rows (sorted unique adofs per type), element-local T
 // columns, the CSR pattern as the union of the topologies (Sparse_Matrix_EpetraFECrs::build_graph,
 // cl_Sparse_Matrix_EpetraFECrs.cpp:195-240) and, per CSR value, the list of element-matrix
@@ -67,6 +99,17 @@ mgpu_status build_generic(const mgpu_set_desc& d, SetHost& h, std::string* err) 
     if (too_big.load()) {
         *err = "an element has more than " + std::to_string(kGenericMaxAdofsPerType) + " adofs per dof type";
         return MGPU_ERR_UNSUPPORTED;
+    }
+    if (nb == 27) {
+        h.t_perm.assign((size_t)h.n_el * kHex27PermStride, 0);
+        parallel_for(h.n_el, [&](int64_t e) {
+            if (h.na_t[(size_t)e] != 27) return;
+            double D[27 * 27] = {};
+            for (int b = 0; b < 27; ++b)
+                for (int32_t q = d.t_ptr[e * nb + b]; q < d.t_ptr[e * nb + b + 1]; ++q)
+                    D[b * 27 + h.t_col[(size_t)q]] += d.t_weight[q];
+            hex27_tensor_form(D, h.t_perm.data() + e * kHex27PermStride);
+        });
     }
     h.topo_ptr.assign((size_t)h.n_el + 1, 0);
     h.ke_off.assign((size_t)h.n_el + 1, 0);

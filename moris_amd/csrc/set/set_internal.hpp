@@ -17,6 +17,8 @@ constexpr int kGenericMaxAdofsPerType = 64;
 // The same for HEX27 IP cells (27 bases): level-0 quadratic B-splines or Lagrange nodes give 27,
 // truncated hierarchical rows up to about 40.
 constexpr int kHex27MaxAdofsPerType = 64;
+constexpr int kHex27Moments = 125;      // moments of degree <= 4 per axis of an element
+constexpr int kHex27PermStride = 28;    // SetHost::t_perm entries of an element
 // HEX27 sets whose element matrices hold more entries than this (a K_e pool of 2 GiB and gather
 // lists of as much again) take the scatter mode; MGPU_GENERIC_SCATTER=1 / =0 forces it on / off.
 constexpr int64_t kGatherMaxEntries = (int64_t)1 << 28;
@@ -61,6 +63,10 @@ struct SetHost {
     std::vector<int64_t> topo_ptr;       // [n_el + 1] into topo (nf * na_t per element; both paths)
     std::vector<int64_t> ke_off;         // [n_el + 1] K_e offsets, (nf * na_t)^2 per element
     std::vector<int32_t> t_col;          // [n T entries] element-local column of each T entry
+    // HEX27 sets, kHex27PermStride entries per element: where the element's T is the tensor product of
+    // one 1D matrix per axis, the tensor index (b_0 3 + b_1) 3 + b_2 of each of its 27 adofs and, last,
+    // that matrix: 1 the identity (nodal rows), 2 the uniform quadratic B-splines; last 0: any other T
+    std::vector<uint8_t> t_perm;
     std::vector<int64_t> gather_ptr;     // [nnz + 1]
     std::vector<int64_t> gather_src;     // [sum of K_e sizes] K_e entry summed into each value
     // scatter mode of the HEX27 kernel (no K_e pool, no gather lists): elements coloured so that

@@ -40,6 +40,11 @@ struct mgpu_set {
     int cut_order = 0;                      // 1: cut elements longest-first
     const int32_t* d_cut_order = nullptr;   // device permutation (built on first use)
     const int32_t* d_gen_order = nullptr;   // generic sets, gather mode: elements most sub-cells first
+    // HEX27 sets: the moments of every element, and the elements (of each colour in scatter mode, else
+    // of the set) with those of tensor T first; n_tensor: how many of them
+    double* d_mom = nullptr;
+    const int32_t* d_hex_els = nullptr;
+    std::vector<int32_t> n_tensor;
     // learned cut-cell quadrature
     std::vector<double> vphi_cut;      // host copy of the cut elements' nodal level sets
     mgpu::LqView lv{};
@@ -83,6 +88,11 @@ mgpu_status check_err_flag(mgpu_set* S);
 // launch_assemble; [1], [2] coincide with [0]).
 mgpu_status generic_upload(mgpu_set* S, const mgpu_set_desc& d);
 mgpu_status launch_generic(mgpu_set* S, const double* u, double* vals, double* rhs, hipEvent_t* ev);
+// HEX27 element kernels (hex27.hip): the moments of all elements, then K_e of n_tensor + n_general
+// elements (to the pool, or with scatter added into vals).
+void launch_hex27_moments(const GenView& g, double* mom, hipStream_t s);
+void launch_hex27_elements(const GenView& g, int nf, bool scatter, int32_t n_tensor, int32_t n_general,
+                           const int32_t* els, const double* mom, double* vals, hipStream_t s);
 // Rows per workgroup of stencil variant `variant` for nf fields; *n_variants: number of variants.
 int stencil_shape(int nf, int variant, int* n_variants);
 }  // namespace mgpu
