@@ -90,6 +90,10 @@ struct GenView {
     const int32_t* na_t;         // [n_el] adofs per dof type
     const int64_t* ke_off;       // [n_el + 1]
     double* ke;                  // element matrices, (nf na_t)^2 per element, row-major
+    // rows mode: elements of each adof (and its position among theirs), else gather lists
+    const int64_t* adof_ptr;     // [N + 1]
+    const int32_t* adof_el;
+    const int32_t* adof_x;
     const int64_t* gather_ptr;   // [nnz + 1]
     const int64_t* gather_src;   // K_e entries summed into each CSR value
     const int32_t* gather_src32; // the same in 32 bits when the pool has fewer than 2^31 entries

@@ -71,9 +71,10 @@ static void hex27_tensor_form(const double* D, uint8_t* perm) {
 
 // Generic path: element topology of any T rows (sorted unique adofs per type), element-local T
 // columns, the CSR pattern as the union of the topologies (Sparse_Matrix_EpetraFECrs::build_graph,
-// cl_Sparse_Matrix_EpetraFECrs.cpp:195-240) and, per CSR value, the list of element-matrix
-// entries summed into it in ascending element order (the deterministic replacement of
-// SumIntoGlobalValues, :103-133).  Large HEX27 sets take the scatter mode instead: elements in
+// cl_Sparse_Matrix_EpetraFECrs.cpp:195-240) and, per adof, the elements whose matrices are summed into
+// its rows in ascending order, with per-element tables of column positions (the deterministic
+// replacement of SumIntoGlobalValues, :103-133); sets with very long rows list the entries summed into
+// each CSR value instead.  Large HEX27 sets take the scatter mode instead: elements in
 // colour classes that share no adof, each adding its K_e into the values, one colour after the
 // other (a fixed order of summation again), with per-element tables of column positions.
 mgpu_status build_generic(const mgpu_set_desc& d, SetHost& h, std::string* err) {
@@ -195,12 +196,15 @@ mgpu_status build_generic(const mgpu_set_desc& d, SetHost& h, std::string* err) 
             h.cut_elems.push_back(e);
         }
     const int64_t n_src = h.ke_off[(size_t)h.n_el];
+    for (int32_t a = 0; a < N; ++a) h.max_nbr = std::max(h.max_nbr, (int32_t)nbr[(size_t)a].size());
     h.scatter = nb == 27 && n_src > kGatherMaxEntries;
+    h.rows = (int64_t)nf * h.max_nbr * (int64_t)sizeof(double) <= kRowsMaxLds;
     if (nb == 27)
         if (const char* env = std::getenv("MGPU_GENERIC_SCATTER")) {
             if (env[0] == '1') h.scatter = true;
-            if (env[0] == '0') h.scatter = false;
+            if (env[0] == '0') h.scatter = h.rows = false;
         }
+    if (h.scatter) h.rows = false;
     if (h.scatter) {
         // greedy colouring in element order: the smallest colour that no element sharing an
         // adof with e already holds
@@ -235,10 +239,11 @@ mgpu_status build_generic(const mgpu_set_desc& d, SetHost& h, std::string* err) 
                              [&](int32_t x, int32_t y) {
                                  return d.ig_ptr[x + 1] - d.ig_ptr[x] > d.ig_ptr[y + 1] - d.ig_ptr[y];
                              });
+    }
+    if (h.scatter || h.rows) {
         // rank tables: both the element's adofs and each adof's neighbours are ascending, so
         // one merge per row finds every column
-        for (int32_t a = 0; a < N; ++a)
-            if (nbr[(size_t)a].size() > 65535) { *err = "an adof has more than 65535 neighbours"; return MGPU_ERR_UNSUPPORTED; }
+        if (h.max_nbr > 65535) { *err = "an adof has more than 65535 neighbours"; return MGPU_ERR_UNSUPPORTED; }
         h.rank_off.assign((size_t)h.n_el + 1, 0);
         for (int32_t e = 0; e < h.n_el; ++e)
             h.rank_off[(size_t)e + 1] = h.rank_off[(size_t)e] + (int64_t)h.na_t[(size_t)e] * h.na_t[(size_t)e];
@@ -256,6 +261,17 @@ mgpu_status build_generic(const mgpu_set_desc& d, SetHost& h, std::string* err) 
                 }
             }
         });
+        if (h.rows) {
+            h.adof_ptr = std::move(a_ptr);
+            h.adof_el = std::move(a_el);
+            h.adof_x.resize(h.adof_el.size());
+            parallel_for(N, [&](int64_t a) {
+                for (int64_t q = h.adof_ptr[(size_t)a]; q < h.adof_ptr[(size_t)a + 1]; ++q) {
+                    const auto& u = loc[(size_t)h.adof_el[(size_t)q]];
+                    h.adof_x[(size_t)q] = (int32_t)(std::lower_bound(u.begin(), u.end(), (int32_t)a) - u.begin());
+                }
+            });
+        }
         return MGPU_OK;
     }
     // gather lists: K_e entry (x, y) of element e goes to CSR value (topo[x], topo[y]).  Built per

@@ -19,9 +19,12 @@ constexpr int kGenericMaxAdofsPerType = 64;
 constexpr int kHex27MaxAdofsPerType = 64;
 constexpr int kHex27Moments = 125;      // moments of degree <= 4 per axis of an element
 constexpr int kHex27PermStride = 28;    // SetHost::t_perm entries of an element
-// HEX27 sets whose element matrices hold more entries than this (a K_e pool of 2 GiB and gather
-// lists of as much again) take the scatter mode; MGPU_GENERIC_SCATTER=1 / =0 forces it on / off.
-constexpr int64_t kGatherMaxEntries = (int64_t)1 << 28;
+// HEX27 sets whose element matrices hold more entries than this (a K_e pool of 8 GiB) take the
+// scatter mode, which keeps no pool but is slower: 40^3 elements of 81 x 81 (3.4 GiB), elasticity:
+// 4.1 ms with the pool, 8.0 ms without.  MGPU_GENERIC_SCATTER=1 forces it on, =0 forces it off and the gather lists.
+constexpr int64_t kGatherMaxEntries = (int64_t)1 << 30;
+// LDS of one row's values in the row-wise sums (k_generic_rows); sets with a longer row keep gather lists
+constexpr int kRowsMaxLds = 32768;
 
 // Host-side products of set creation (pure C++, no HIP).
 struct SetHost {
@@ -55,8 +58,8 @@ struct SetHost {
     // cut elements
     std::vector<int32_t> cut_elems;  // element ids with sub-cells
     std::vector<int32_t> elem_cut;   // [n_el] cut index or -1
-    // generic path (T rows with several entries, or no lattice): element-local T and the gather
-    // lists of the CSR values
+    // generic path (T rows with several entries, or no lattice): element-local T, and either rows mode
+    // (the elements of every adof and the rank tables) or gather lists
     bool generic = false;
     int32_t na_t_max = 0;                // largest per-type element topology
     std::vector<int32_t> na_t;           // [n_el] adofs per dof type of each element
@@ -67,13 +70,19 @@ struct SetHost {
     // one 1D matrix per axis, the tensor index (b_0 3 + b_1) 3 + b_2 of each of its 27 adofs and, last,
     // that matrix: 1 the identity (nodal rows), 2 the uniform quadratic B-splines; last 0: any other T
     std::vector<uint8_t> t_perm;
+    bool rows = false;
+    int32_t max_nbr = 0;                 // most neighbours of an adof (per dof type)
+    std::vector<int64_t> adof_ptr;       // [n_adofs_type + 1] into adof_el / adof_x
+    std::vector<int32_t> adof_el;        // elements holding each adof, ascending
+    std::vector<int32_t> adof_x;         // and the adof's position among their adofs
     std::vector<int64_t> gather_ptr;     // [nnz + 1]
     std::vector<int64_t> gather_src;     // [sum of K_e sizes] K_e entry summed into each value
-    // scatter mode of the HEX27 kernel (no K_e pool, no gather lists): elements coloured so that
+    // scatter mode of the HEX27 kernels (no K_e pool): elements coloured so that
     // no two of one colour share an adof; each element adds its K_e into the CSR values
     bool scatter = false;
     std::vector<int32_t> colour_ptr;     // [n_colours + 1] into colour_el
     std::vector<int32_t> colour_el;      // [n_el] elements by colour, most sub-cells first within one
+    // rank tables (rows and scatter mode)
     std::vector<int64_t> rank_off;       // [n_el + 1] na_t^2 per element
     std::vector<uint16_t> rank;          // [x][y]: position of adof y in the sorted neighbours of adof x
 };

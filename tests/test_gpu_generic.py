@@ -318,13 +318,14 @@ def test_thb_scatter_mode_chosen_by_size_properties():
     assert rel(vm, vals) <= 1e-6 and rel(Rm, R) <= 1e-6
 
 
-@pytest.mark.parametrize("scatter", ["0", "1"])
+@pytest.mark.parametrize("scatter", ["", "0", "1"])
 @pytest.mark.parametrize("order", [1, 2])
 def test_hex27_tensor_and_general_rows(order, scatter, monkeypatch):
     """HEX27 elements whose T is a tensor product (nodal rows, p = 2 B-splines) take K_e straight from
     the element's moments, any other T takes K_e = T^T K_p T; both in one set, adofs numbered at random
     (every tensor order among the elements' sorted adofs), against the oracle: FP64 sums in another
-    order, K within 1e-13 (5e-16 measured; 27 x 27 products of unit-sized terms)."""
+    order, K within 1e-13 (5e-16 measured; 27 x 27 products of unit-sized terms).  Summed row by row (the default), by gather
+    lists or in scatter mode."""
     spec, keep = M.make_spec(3, (4, 3, 5), iwg=M.IWG_STRUC_LINEAR_BULK, spheres=[[0.45, 0.5, 0.55, 0.34]],
                              bspline_order=order, lagrange_order=2)
     P = M.Problem(spec, keep)
@@ -340,9 +341,10 @@ def test_hex27_tensor_and_general_rows(order, scatter, monkeypatch):
     ctypes.memmove(ctypes.byref(d), ctypes.byref(P.desc), ctypes.sizeof(M.SetDesc))
     d.t_adof = adof.ctypes.data_as(ctypes.POINTER(ctypes.c_int32))
     d.t_weight = weight.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
-    monkeypatch.setenv("MGPU_GENERIC_SCATTER", scatter)
+    if scatter:
+        monkeypatch.setenv("MGPU_GENERIC_SCATTER", scatter)
     S = M.Set(d, keepalive=(P, adof, weight))
-    monkeypatch.delenv("MGPU_GENERIC_SCATTER")
+    monkeypatch.delenv("MGPU_GENERIC_SCATTER", raising=False)
     rp, ci = S.pattern()
     u = rng.uniform(-1.0, 1.0, S.n_rows)
     vo, Ro, _ = O.assemble_desc(d, rp, ci, u)
@@ -351,3 +353,20 @@ def test_hex27_tensor_and_general_rows(order, scatter, monkeypatch):
             S.options(prec, quad)
             vals, R = S.compute_jacobian_and_residual(u)
             assert rel(vals, vo) <= 1e-13 and rel(R, Ro) <= 1e-13, (quad, prec, rel(vals, vo), rel(R, Ro))
+
+
+@pytest.mark.parametrize("case", ["p2_circle_16x12_plane_stress", "thb_sphere_4_hex27_diffusion", "thb_plane_5_hex27_elasticity",
+                                  "enriched_gyroid_6_p2_hex27_elasticity"])
+def test_rows_mode_sums_in_element_order(case, monkeypatch):
+    """Rows mode adds the element matrices into a row in ascending element order, as the gather lists
+    do: bit-identical K (HEX27 sets can be forced onto the lists), R the row times u to rounding."""
+    spec, keep = CASES[case]()
+    P = M.Problem(spec, keep)
+    S = M.Set(P.desc, keepalive=P)
+    monkeypatch.setenv("MGPU_GENERIC_SCATTER", "0")
+    S_lists = M.Set(P.desc, keepalive=P)
+    monkeypatch.delenv("MGPU_GENERIC_SCATTER")
+    u = np.random.default_rng(SEED + 52).uniform(-1.0, 1.0, S.n_rows)
+    v1, R1 = S.compute_jacobian_and_residual(u)
+    v2, R2 = S_lists.compute_jacobian_and_residual(u)
+    assert np.array_equal(v1.view(np.uint64), v2.view(np.uint64)) and rel(R1, R2) <= 1e-14
