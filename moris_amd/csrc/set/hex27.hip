@@ -9,10 +9,10 @@
 // in another order, and closer to that sum than a point-wise accumulation of M (K within 1.2e-16 ..
 // 2.9e-16 of sums in 80-bit long double, against 7.8e-16 .. 2.1e-15).  32^3 cut cells, elasticity, p = 2 (1.1M
 // sub-tets, 37.8M points): element kernels 11.8 ms with M accumulated point by point on 21 FP64 MFMA
-// tiles, 1.4 ms here.
+// tiles, 0.91 ms here.
 //
-//   k_hex27_moments    one wavefront per element: the 125 moments of a cut cell on FP64 MFMA, one
-//                      16 x 16 x 4 product per 4 points (whole cells: closed form).
+//   k_hex27_moments    two wavefronts per element: the 125 moments of a cut cell, a lane a point (whole
+//                      cells: closed form).
 //   k_hex27_tensor     elements whose T is a tensor product of one 1D matrix per axis (nodal rows,
 //                      untruncated p = 2 B-splines): T folded into the 1D factor tables, so that K_e
 //                      comes straight from the moments; one block of 4 wavefronts per element.
@@ -77,16 +77,16 @@ __constant__ const AxisTables kAxis{};
 __constant__ const double kBasisInt[5] = {1.0 / 3.0, 4.0 / 3.0, 1.0 / 3.0, 0.0, -4.0 / 15.0};
 
 // ------------------------------------------------------------------------------------------------
-// k_hex27_moments: mom[e][(i 5 + j) 5 + k] = sum_ip w* g_i(x) g_j(y) g_k(z), g the basis above.  64 points at
-// a time, a lane a point: mapped, its 15 row values w* g_i(x) l_n(y) and 10 column values g_k(z) {1, c(y)}
-// put in LDS 32 points at a time (stride 25 doubles: distinct banks; 6.4 KB, so that registers and not LDS
-// bound the wavefronts in flight), then 8 MFMA steps of 4 points with one 8-byte read per operand.
-// Splitting g_j over rows and columns lets one 16 x 16 tile hold all 125 moments (rows (i, j), columns k
-// would take two, 25 x 5 of 32 x 16 used): sum_n l_n = 1 and l_2 - l_0 = y give c and c y.  Bound by the FP64
-// units, MFMA and the per-point arithmetic together: 0.67 ms for 32^3 cut cells.
+// k_hex27_moments: mom[e][(i 5 + j) 5 + k] = sum_ip w* g_i(x) g_j(y) g_k(z), g the basis above.  Two wavefronts
+// per element, each with 13 or 12 of the 25 pairs (i, j) as 65 or 60 sums per lane in registers; 64 points
+// at a time, a lane a point.  A batch of 64 sub-tets is staged in LDS as vertex 2, the three edges and
+// the volume factor.  The lanes' sums are added pairwise by half and quarter wavefront (gfx950's lane
+// swaps reduce two registers at once), the last 16 in LDS.
+// Bound by FP64 arithmetic, 111 operations a point and wavefront: 32^3 cut cells (37.8M points) 0.47 ms; a
+// 16 x 16 x 4 FP64 MFMA tile per 4 points took 0.69 ms: its operands pass through LDS (25 doubles a point),
+// half the tile is padding, and FP64 MFMA runs at the rate of the vector unit.
 // ------------------------------------------------------------------------------------------------
-constexpr int kMomPt = 25;
-__device__ inline void hex27_basis(double x, double* v) {
+__device__ __forceinline__ void hex27_basis(double x, double* v) {
     const double x2 = x * x;
     v[0] = 0.5 * (x2 - x);
     v[1] = 1.0 - x2;
@@ -94,109 +94,142 @@ __device__ inline void hex27_basis(double x, double* v) {
     v[3] = -x * v[1];
     v[4] = x * v[3];
 }
-__global__ __launch_bounds__(64) void k_hex27_moments(GenView g, double* mom) {
-    __shared__ double rec[32 * kMomPt];
-    const int e = g.order ? g.order[blockIdx.x] : (int)blockIdx.x;
+
+// a + b over the two halves of the wavefront (SWAP 32) or of each half (16): lanes of the first get the
+// sum of a, lanes of the second that of b
+template <int SWAP>
+__device__ __forceinline__ double swap_add(double a, double b) {
+    const uint64_t ua = __double_as_longlong(a), ub = __double_as_longlong(b);
+    uint32_t r[4];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        const uint32_t x = (uint32_t)(ua >> (32 * w)), y = (uint32_t)(ub >> (32 * w));
+        const auto s = SWAP == 32 ? __builtin_amdgcn_permlane32_swap(x, y, false, false)
+                                  : __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        r[w] = s[0];
+        r[2 + w] = s[1];
+    }
+    return __longlong_as_double(((uint64_t)r[1] << 32) | r[0]) + __longlong_as_double(((uint64_t)r[3] << 32) | r[2]);
+}
+
+constexpr int kMomBatch = 64;                          // sub-tets staged at a time
+constexpr int kMomTet = 14;                            // x_2, edges, volume factor (even: 16-byte reads)
+constexpr int kMomRule = kMomBatch * kMomTet;          // LDS offset of TET_35 [q][xi_0, xi_1, xi_2, w]
+constexpr int kMomLds = 17 * 68;                       // the reduction's space
+static_assert(kMomRule + 4 * kTet35Points <= kMomLds, "staged sub-tets and the rule fit the reduction's space");
+
+template <int ROLE>
+__device__ __forceinline__ void hex27_cut_moments(const GenView& g, int ig0, int nsub, double vol6, double* lds, double* out) {
+    constexpr int P0 = ROLE == 0 ? 0 : 13, NP = ROLE == 0 ? 13 : 12, I0 = P0 / 5;
     const int lane = threadIdx.x;
+    double acc[NP][5];
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int k = 0; k < 5; ++k) acc[p][k] = 0.0;
+    for (int t = lane; t < 4 * kTet35Points; t += 64) {
+        const int q = t >> 2, c = t & 3;
+        lds[kMomRule + t] = c < 3 ? kTet35Xi[q][c] : kTet35W[q];
+    }
+    for (int t0 = 0; t0 < nsub; t0 += kMomBatch) {
+        const int nt = min(kMomBatch, nsub - t0), npts = nt * kTet35Points;
+        if (t0 > 0) __syncthreads();   // the previous batch is read
+        if (lane < nt) {
+            const double2* X2 = reinterpret_cast<const double2*>(g.ig_xi + (size_t)(ig0 + t0 + lane) * 12);
+            double X[12];
+#pragma unroll
+            for (int n = 0; n < 6; ++n) {
+                const double2 v = X2[n];
+                X[2 * n] = v.x;
+                X[2 * n + 1] = v.y;
+            }
+            double J[3][3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                J[0][d] = X[d] - X[6 + d];
+                J[1][d] = X[3 + d] - X[6 + d];
+                J[2][d] = X[9 + d] - X[6 + d];
+            }
+            const double detJ = (J[0][0] * (J[1][1] * J[2][2] - J[2][1] * J[1][2]) -
+                                 J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
+                                 J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0])) * vol6;
+            double* T = lds + lane * kMomTet;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                T[4 * d] = X[6 + d];
+#pragma unroll
+                for (int r = 0; r < 3; ++r) T[4 * d + 1 + r] = J[r][d];
+            }
+            T[12] = detJ < kDetJLowerLimit ? 0.0 : detJ;
+        }
+        __syncthreads();
+        for (int p0 = 0; p0 < npts; p0 += 64) {
+            // lanes past the end: point 0 with weight 0.  The point is vertex 2 plus the rule's
+            // coordinates along the edges (the same affine map as the vertex weights (xi0, xi1,
+            // 1 - xi0 - xi1 - xi2, xi2))
+            const int ip = p0 + lane, ipc = ip < npts ? ip : 0;
+            const int t = ipc / kTet35Points, q = ipc - kTet35Points * t;
+            const double* T = lds + t * kMomTet;
+            const double* b = lds + kMomRule + 4 * q;
+            double x[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) x[d] = T[4 * d] + b[0] * T[4 * d + 1] + b[1] * T[4 * d + 2] + b[2] * T[4 * d + 3];
+            const double w = ip < npts ? b[3] * T[12] : 0.0;
+            double gx[5], gy[5], gz[5];
+            hex27_basis(x[0], gx);
+            hex27_basis(x[1], gy);
+            hex27_basis(x[2], gz);
+#pragma unroll
+            for (int i = I0; i < 5; ++i) gx[i] *= w;
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                const double v = gx[(P0 + p) / 5] * gy[(P0 + p) % 5];
+#pragma unroll
+                for (int k = 0; k < 5; ++k) acc[p][k] += v * gz[k];
+            }
+        }
+    }
+    // values v and v + 33 by half wavefront, then r and r + 17 by quarter: register r of quarter c holds
+    // value r + 17 (c & 1) + 33 (c >> 1)
+    constexpr int NV = NP * 5;
+    double h[34];
+#pragma unroll
+    for (int v = 0; v < 34; ++v)
+        h[v] = v < 33 ? swap_add<32>(acc[v / 5][v % 5], v + 33 < NV ? acc[(v + 33 < NV ? v + 33 : 0) / 5][(v + 33) % 5] : 0.0) : 0.0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 17; ++r) lds[r * 68 + (lane >> 4) * 17 + (lane & 15)] = swap_add<16>(h[r], h[r + 17]);
+    __syncthreads();
+    for (int t = lane; t < 68; t += 64) {
+        const int r = t >> 2, c = t & 3;
+        const int v = r + ((c & 1) ? 17 : 0) + ((c & 2) ? 33 : 0);
+        double s = 0.0;
+#pragma unroll
+        for (int l = 0; l < 16; ++l) s += lds[r * 68 + c * 17 + l];
+        if (((c & 1) == 0 || r < 16) && v < NV) out[P0 * 5 + v] = s;
+    }
+}
+
+__global__ __launch_bounds__(64) void k_hex27_moments(GenView g, double* mom) {
+    __shared__ double lds[kMomLds];
+    // 16 blocks in a row hold 8 elements, the role changing after 8: the round robin over the 8 XCDs
+    // gives each both roles in turn
+    const int b = blockIdx.x, role = (b >> 3) & 1, be = (b >> 4) * 8 + (b & 7);
+    if (be >= g.n_el) return;
+    const int e = g.order ? g.order[be] : be;
     double hh[3];
     for (int d = 0; d < 3; ++d) hh[d] = g.ip_box[(size_t)e * 6 + 3 + d];
+    const double detJ = (0.5 * hh[0]) * (0.5 * hh[1]) * (0.5 * hh[2]);
     const int ig0 = g.ig_ptr[e], nsub = g.ig_ptr[e + 1] - ig0;
     double* out = mom + (size_t)e * kHex27Moments;
     if (nsub == 0) {
         // whole cell: products of 1D integrals (HEX_3x3x3 integrates the basis exactly)
-        const double detJ = (0.5 * hh[0]) * (0.5 * hh[1]) * (0.5 * hh[2]);
-        for (int t = lane; t < kHex27Moments; t += 64) {
+        for (int t = threadIdx.x; t < kHex27Moments && role == 0; t += 64)
             out[t] = detJ * (kBasisInt[t / 25] * kBasisInt[(t / 5) % 5] * kBasisInt[t % 5]);
-        }
-        return;
-    }
-    const int npts = nsub * kTet35Points;
-    const int r16 = lane & 15, kq = lane >> 4;
-    const int ao = kq * kMomPt + (r16 < 15 ? r16 : 0);
-    const int bo = kq * kMomPt + 15 + (r16 < 10 ? r16 : 0);
-    // summed per chunk (two chains), then over the chunks: shorter chains of rounded additions
-    doublex4_t tot = {0.0, 0.0, 0.0, 0.0}, acc0 = tot, acc1 = tot;
-    // the lane's point of the coming chunk: sub-tet vertices and rule (lanes past the end: point 0
-    // with weight 0), requested before the matrix work of the chunk before it
-    const double vol6 = (0.5 * hh[0]) * (0.5 * hh[1]) * (0.5 * hh[2]) / 6.0;
-    double X[12], bq[4];
-    auto request = [&](int p0) {
-        const int ip = p0 + lane, ipc = ip < npts ? ip : 0;
-        const int t = ipc / kTet35Points, q = ipc - kTet35Points * t;
-        const double2* X2 = reinterpret_cast<const double2*>(g.ig_xi + (size_t)(ig0 + t) * 12);
-#pragma unroll
-        for (int n = 0; n < 6; ++n) {
-            const double2 v = X2[n];
-            X[2 * n] = v.x;
-            X[2 * n + 1] = v.y;
-        }
-        bq[0] = kTet35Xi[q][0];
-        bq[1] = kTet35Xi[q][1];
-        bq[2] = kTet35Xi[q][2];
-        bq[3] = ip < npts ? kTet35W[q] : 0.0;
-    };
-    request(0);
-    for (int p0 = 0; p0 < npts; p0 += 64) {
-        // vertex 2 plus the rule's coordinates along the edges J to the others (the same affine map as
-        // the vertex weights (xi0, xi1, 1 - xi0 - xi1 - xi2, xi2))
-        double x[3], J[3][3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            J[0][d] = X[d] - X[6 + d];
-            J[1][d] = X[3 + d] - X[6 + d];
-            J[2][d] = X[9 + d] - X[6 + d];
-            x[d] = X[6 + d] + bq[0] * J[0][d] + bq[1] * J[1][d] + bq[2] * J[2][d];
-        }
-        const double detJ = (J[0][0] * (J[1][1] * J[2][2] - J[2][1] * J[1][2]) -
-                             J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
-                             J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0])) * vol6;
-        const double w = detJ < kDetJLowerLimit ? 0.0 : bq[3] * detJ;
-        double gx[5], gy[5], gz[5], av[15], cv[5];
-        hex27_basis(x[0], gx);
-        hex27_basis(x[1], gy);
-        hex27_basis(x[2], gz);
-#pragma unroll
-        for (int i = 0; i < 5; ++i) {
-            const double wg = w * gx[i];
-#pragma unroll
-            for (int n = 0; n < 3; ++n) av[3 * i + n] = wg * gy[n];
-            cv[i] = gz[i] * gy[3];
-        }
-        request(p0 + 64);   // (past the last chunk: point 0, unused)
-        tot += acc0 + acc1;
-        acc0 = acc1 = doublex4_t{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            __syncthreads();   // the previous records are read
-            if ((lane >> 5) == half) {
-                double* pp = rec + (lane & 31) * kMomPt;
-#pragma unroll
-                for (int n = 0; n < 15; ++n) pp[n] = av[n];
-#pragma unroll
-                for (int k = 0; k < 5; ++k) {
-                    pp[15 + 2 * k] = gz[k];
-                    pp[16 + 2 * k] = cv[k];
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int s = 0; s < 8; s += 2) {
-                const double* ps = rec + 4 * s * kMomPt;
-                acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(ps[ao], ps[bo], acc0, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(ps[4 * kMomPt + ao], ps[4 * kMomPt + bo], acc1, 0, 0, 0);
-            }
-        }
-    }
-    // the tile through LDS: register n of a lane holds row lane / 16 + 4 n = 3 i + l, column lane % 16 =
-    // 2 k + [times c]; the last row and columns 10 .. 15 repeat others
-    __syncthreads();
-#pragma unroll
-    for (int n = 0; n < 4; ++n) rec[(kq + 4 * n) * 17 + r16] = tot[n] + (acc0[n] + acc1[n]);
-    __syncthreads();
-    for (int t = lane; t < kHex27Moments; t += 64) {
-        const int i = t / 25, j = (t / 5) % 5, k = t % 5;
-        const double* D = rec + 3 * i * 17 + 2 * k + (j >= 3 ? 1 : 0);
-        out[t] = j < 3 ? D[17 * j] : (j == 3 ? (D[0] + D[17]) + D[34] : D[34] - D[0]);
+    } else if (role == 0) {
+        hex27_cut_moments<0>(g, ig0, nsub, detJ / 6.0, lds, out);
+    } else {
+        hex27_cut_moments<1>(g, ig0, nsub, detJ / 6.0, lds, out);
     }
 }
 
@@ -224,7 +257,7 @@ constexpr int sf_lds() {   // doubles
 static_assert(kSfY + 6 * 405 <= 6 * 729, "the contraction stages fit the space of G");
 
 template <int NF>
-__device__ inline void sf_moments(const GenView& g, const double* mom, int e, int kind, double* lds) {
+__device__ __forceinline__ void sf_moments(const GenView& g, const double* mom, int e, int kind, double* lds) {
     using B = Hex27Blocks<NF>;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -321,7 +354,7 @@ struct KTerms {
     int base[3], sa[3], sb[3];
 };
 template <int NF>
-__device__ inline KTerms k_terms(int f, int h, double c0, double c1, double cs) {
+__device__ __forceinline__ KTerms k_terms(int f, int h, double c0, double c1, double cs) {
     KTerms k;
     if (NF == 1) {
         k.c[0] = c0;
@@ -355,7 +388,7 @@ __device__ inline KTerms k_terms(int f, int h, double c0, double c1, double cs) 
 }
 
 template <int NF>
-__device__ inline void hex27_material(const GenView& g, int e, double& c0, double& c1, double& cs) {
+__device__ __forceinline__ void hex27_material(const GenView& g, int e, double& c0, double& c1, double& cs) {
     if (NF == 1) {
         c0 = g.material[e];
         c1 = cs = 0.0;
@@ -372,8 +405,8 @@ __device__ inline void hex27_material(const GenView& g, int e, double& c0, doubl
 // k_hex27_tensor: K_e of elements whose T is a tensor product (t_perm[e][27] = 1 nodal, 2 B-spline;
 // t_perm[e][y] the tensor index of the element's adof y).  Threads 0 .. 3 NA - 1 hold a column of K_e and
 // write NF rows' worth of consecutive values per step (stores of whole lines).  Without the products by T
-// and their LDS space four blocks instead of two fit a CU: 0.74 ms for 32^3 elements of 81 x 81 (1.7 GB
-// written), against 1.9 ms on the general path.
+// and their LDS space four blocks instead of two fit a CU: 0.44 ms for 32^3 elements of 81 x 81 (1.7 GB
+// written, 3.9 TB/s), against 1.7 ms on the general path.
 // ------------------------------------------------------------------------------------------------
 template <int NF, bool SCATTER>
 __global__ __launch_bounds__(256) void k_hex27_tensor(GenView g, const int32_t* els, const double* mom, double* vals) {
@@ -544,7 +577,7 @@ void launch_elements_t(const GenView& g, int32_t n_tensor, int32_t n_general, co
 }  // namespace
 
 void launch_hex27_moments(const GenView& g, double* mom, hipStream_t s) {
-    hipLaunchKernelGGL(k_hex27_moments, dim3((unsigned)g.n_el), dim3(64), 0, s, g, mom);
+    hipLaunchKernelGGL(k_hex27_moments, dim3((unsigned)((g.n_el + 7) / 8 * 16)), dim3(64), 0, s, g, mom);
 }
 
 void launch_hex27_elements(const GenView& g, int nf, bool scatter, int32_t n_tensor, int32_t n_general,
