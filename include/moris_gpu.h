@@ -55,23 +55,19 @@ typedef int32_t mgpu_status;
 
 /* Arithmetic of the element integrands. */
 #define MGPU_PREC_FP64   0   /* plain path: everything FP64                                        */
-#define MGPU_PREC_MIXED  1   /* FP32 integrands with FP32 accumulation; FP64 cut-cell Jacobians and
-                                FP64 global accumulation                                           */
+#define MGPU_PREC_MIXED  1   /* the 27-point rules of lattice sets (learned, moment fit) with FP32
+                                products and element matrices, FP64 sub-cell maps, moments and global
+                                accumulation; the subdivision and generic sets as MGPU_PREC_FP64     */
 
 /* Cut-cell quadrature. */
 #define MGPU_QUAD_SUBDIVISION  0   /* XTK regular subdivision + node hierarchy, TET_11 / TRI_7       */
 #define MGPU_QUAD_LEARNED      1   /* MLP weights on the HEX_3x3x3 Gauss points, moment-checked,
                                       falling back to subdivision per element                      */
-#define MGPU_QUAD_MOMENT_FIT   2   /* HEX27 cells (generic path): a cut cell's TET_35 points replaced
-                                      by the 5 x 5 x 5 Gauss-Legendre nodes, weighted by the cell's
-                                      degree-4 Lagrange moments over those points; the same sum as the
-                                      subdivision for integrands of degree <= 4 per axis (the box
-                                      HEX27 stiffness), i.e. the same K up to rounding, from 125
-                                      points per cut cell.  Generic HEX8 / QUAD4 cells: the 3^dim
-                                      tensor Gauss points, degree-2 Lagrange moments of the TET_11 /
-                                      TRI_7 points.  3D lattice (hex8) sets: the 27 HEX_3x3x3
-                                      points weighted by the degree-2 Lagrange moments over the
-                                      TET_11 points (exact for the trilinear stiffness), no model,
+#define MGPU_QUAD_MOMENT_FIT   2   /* generic sets: the same as the subdivision, which takes K from the
+                                      cell's moments over the sub-cells' points (degree 4 per axis on
+                                      HEX27, 2 on HEX8 / QUAD4 cells).  3D lattice (hex8) sets: the 27
+                                      HEX_3x3x3 points weighted by the degree-2 Lagrange moments over
+                                      the TET_11 points (exact for the trilinear stiffness), no model,
                                       no fallback; the 27-point product runs as in
                                       MGPU_QUAD_LEARNED (FP32 MFMA)                                  */
 

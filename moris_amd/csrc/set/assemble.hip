@@ -2,19 +2,18 @@
 // drive them.  Target: gfx950 (MI355X), 64-wide wavefronts.
 //
 // Path of one mgpu_set_assemble call on a lattice set:
-//   k_cut_diffusion / k_cut_elasticity
-//                   one wavefront per cut element.  For every IG sub-cell and every point of its
+//   k_cut           one wavefront per cut element.  For every IG sub-cell and every point of its
 //                   rule (TET_11 / TRI_7): map the point to the IP cell (Space_Interpolator::
 //                   map_integration_point, cl_MTK_Space_Interpolator.cpp:1381-1397), take detJ of
 //                   the sub-cell (:1180-1210 tet, :1120-1128 tri), skip if detJ < -1e-6
-//                   (cl_FEM_Element_Bulk.cpp:291), w* = w * detJ (:297), evaluate dN/dx of the IP
-//                   cell (Field_Interpolator::eval_d1Ndx1, cl_FEM_Field_Interpolator.cpp:464-496,
-//                   diagonal inverse Jacobian of a rectangular cell, cl_MTK_Space_Interpolator.cpp
-//                   :676-700) and accumulate the moment matrix M = sum_ip w* g g^T, g = dN/dx.
+//                   (cl_FEM_Element_Bulk.cpp:291), w* = w * detJ (:297).  The sums over the points of
+//                   w* times the quadratics of each axis determine M = sum_ip w* g g^T, g = dN/dx of
+//                   the IP cell (Field_Interpolator::eval_d1Ndx1, cl_FEM_Field_Interpolator.cpp
+//                   :464-496, diagonal inverse Jacobian of a rectangular cell,
+//                   cl_MTK_Space_Interpolator.cpp:676-700).
 //                   The element matrix K_p = B^T D B contracted with M (IWG compute_jacobian,
 //                   cl_FEM_IWG_Isotropic_Struc_Linear_Bulk.cpp:200, cl_FEM_IWG_Diffusion_Bulk.cpp
-//                   :280) is projected with the element's T rows into sorted adof order
-//                   (cl_MSI_Equation_Object.cpp:810-841) and stored.
+//                   :280) is stored in vertex order.
 //   k_prep          u gathered per lattice node, one material record per lattice cell.
 //   k_stencil       owner-computes scatter: one thread per CSR row.  The row sums the K_e rows of
 //                   the (up to 8 / 4) lattice cells around its node -- uncut cells from the
@@ -38,267 +37,53 @@
 #include "../setup/internal.hpp"
 #include "set_state.hpp"
 #include "../learned/quad.hpp"
+#include "cut_moments.hpp"
 
 namespace mgpu {
 
 // ------------------------------------------------------------------------------------------------
-// k_cut_diffusion: one wavefront per cut element.  Each lane integrates every 64th point and keeps
-// the symmetric moments S[a][b] = sum_ip w* g_a . g_b in registers; one LDS reduction per element.
+// k_cut: one wavefront per cut element: its moments (cut_moments.hpp), then lane (a, b) forms the element
+// matrix's entries of the vertex pair.  FP64 at either precision option; the element matrix is stored
+// in KT (FP32 beside the FP32 products of the 27-point rules on the mixed path).
+// Bound by FP64 arithmetic (61 operations a point) and the latency of its phases: 64^3 cells, sphere array
+// (33.6k cut elements), elasticity 0.117 ms, where accumulating M point by point on padded 32 x 32 FP64 MFMA
+// tiles took 0.65 ms; 128^3 cells, one sphere, diffusion 0.058 ms, 0.184 ms with the 36 products of the vertex
+// pairs summed per lane.
 // ------------------------------------------------------------------------------------------------
-template <int DIM, typename T>
-__global__ __launch_bounds__(64) void k_cut_diffusion(DevView s) {
+template <int DIM, int NF, typename KT>
+__global__ __launch_bounds__(64) void k_cut(DevView s) {
     constexpr int NB = DIM == 3 ? 8 : 4;
-    constexpr int NV = DIM + 1;
-    constexpr int NQ = DIM == 3 ? kTet11Points : kTri7Points;
-    constexpr int NSYM = NB * (NB + 1) / 2;
-    __shared__ double red[NSYM * 65];
-
+    constexpr int NA = NF * NB;
+    __shared__ __align__(16) double lds[LinearMoments<DIM>::LDS];
+    __shared__ double m[LinearMoments<DIM>::N];
     const int c = s.cut_order ? s.cut_order[blockIdx.x] : (int)blockIdx.x;
     if (s.skip && s.skip[c]) return;
-    const int lane = threadIdx.x;
     const int e = s.cut_elems[c];
     const int ig0 = s.ig_ptr[e];
-    const int nip = (s.ig_ptr[e + 1] - ig0) * NQ;
     double hh[DIM];
     for (int d = 0; d < DIM; ++d) hh[d] = s.h[d];
-    (void)NV;
-
-    // T = float: FP32 integrand with FP32 accumulation; the point map and the sub-cell Jacobian
-    // (cut_point) stay FP64
-    T acc[NSYM];
-#pragma unroll
-    for (int t = 0; t < NSYM; ++t) acc[t] = (T)0;
-    for (int ip = lane; ip < nip; ip += 64) {
-        double gd[DIM][NB];
-        const T w = (T)cut_point<DIM>(s, ig0, ip, hh, gd);
-        T g[DIM][NB];
-#pragma unroll
-        for (int i = 0; i < DIM; ++i)
-#pragma unroll
-            for (int a = 0; a < NB; ++a) g[i][a] = (T)gd[i][a];
-        int t = 0;
-#pragma unroll
-        for (int a = 0; a < NB; ++a)
-#pragma unroll
-            for (int b = a; b < NB; ++b) {
-                T v = (T)0;
-#pragma unroll
-                for (int i = 0; i < DIM; ++i) v += g[i][a] * g[i][b];
-                acc[t++] += w * v;
-            }
-    }
-#pragma unroll
-    for (int t = 0; t < NSYM; ++t) red[t * 65 + lane] = (double)acc[t];
-    __syncthreads();
-    T* ke = ke_store<T>(s) + (size_t)c * NB * NB;
-    const double k = s.material[e];
-    if (lane < NSYM) {
+    cut_moments<DIM>(s.ig_xi, ig0, s.ig_ptr[e + 1] - ig0, hh, lds, m);
+    const int lane = threadIdx.x;
+    if (lane >= NB * NB) return;
+    const int a = lane / NB, b = lane % NB;
+    double M[DIM][DIM];
+    moment_block<DIM>(m, a, b, hh, M);
+    KT* ke = ke_store<KT>(s) + (size_t)c * NA * NA;
+    if constexpr (NF == 1) {
         double v = 0.0;
-        for (int l = 0; l < 64; ++l) v += red[lane * 65 + l];
-        // (a, b) of the packed upper triangle
-        int a = 0, t = lane;
-        while (t >= NB - a) { t -= NB - a; ++a; }
-        const int b = a + t;
-        ke[a * NB + b] = (T)(k * v);
-        ke[b * NB + a] = (T)(k * v);
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) v += M[i][i];
+        ke[a * NB + b] = (KT)(s.material[e] * v);
+    } else {
+        constexpr int NS = DIM == 3 ? 6 : 3;
+        double D[NS][NS];
+        elastic_D<DIM>(s.material[2 * e], s.material[2 * e + 1], D);
+#pragma unroll
+        for (int al = 0; al < DIM; ++al)
+#pragma unroll
+            for (int be = 0; be < DIM; ++be)
+                ke[(a * DIM + al) * NA + (be * NB + b)] = (KT)elastic_entry<DIM>(D, M, al, be);
     }
-}
-
-// ------------------------------------------------------------------------------------------------
-// k_cut_elasticity: one wavefront per cut element.  Points are evaluated 64 at a time into LDS; lane
-// (a, b) accumulates the 3x3 (2x2) direction block M[(i,a),(j,b)] = sum w* g_ia g_jb over all points,
-// then contracts it with D (B^T D B) and projects to sorted adof order.
-// ------------------------------------------------------------------------------------------------
-template <int DIM, typename T>
-__global__ __launch_bounds__(64) void k_cut_elasticity(DevView s) {
-    constexpr int NB = DIM == 3 ? 8 : 4;
-    constexpr int NG = DIM * NB;
-    constexpr int NA = DIM * NB;
-    constexpr int NQ = DIM == 3 ? kTet11Points : kTri7Points;
-    constexpr int GPAD = NG + 1;
-    __shared__ T sgw[64 * GPAD];
-    __shared__ T sg[64 * GPAD];
-
-    const int c = s.cut_order ? s.cut_order[blockIdx.x] : (int)blockIdx.x;
-    if (s.skip && s.skip[c]) return;
-    const int lane = threadIdx.x;
-    const int e = s.cut_elems[c];
-    const int ig0 = s.ig_ptr[e];
-    const int nip = (s.ig_ptr[e + 1] - ig0) * NQ;
-    double hh[DIM];
-    for (int d = 0; d < DIM; ++d) hh[d] = s.h[d];
-    const int a = (lane / NB) % NB, b = lane % NB;
-    const bool active = lane < NB * NB;
-
-    T M[DIM][DIM];
-#pragma unroll
-    for (int i = 0; i < DIM; ++i)
-#pragma unroll
-        for (int j = 0; j < DIM; ++j) M[i][j] = (T)0;
-
-    for (int base = 0; base < nip; base += 64) {
-        const int ip = base + lane;
-        if (ip < nip) {
-            double g[DIM][NB];
-            const double w = cut_point<DIM>(s, ig0, ip, hh, g);
-            for (int i = 0; i < DIM; ++i)
-                for (int q = 0; q < NB; ++q) {
-                    sg[lane * GPAD + i * NB + q] = (T)g[i][q];
-                    sgw[lane * GPAD + i * NB + q] = (T)(w * g[i][q]);
-                }
-        } else {
-            for (int k = 0; k < NG; ++k) {
-                sg[lane * GPAD + k] = (T)0;
-                sgw[lane * GPAD + k] = (T)0;
-            }
-        }
-        __syncthreads();
-        const int cnt = min(64, nip - base);
-        if (active) {
-            for (int p = 0; p < cnt; ++p) {
-                T ga[DIM], gb[DIM];
-#pragma unroll
-                for (int i = 0; i < DIM; ++i) {
-                    ga[i] = sgw[p * GPAD + i * NB + a];
-                    gb[i] = sg[p * GPAD + i * NB + b];
-                }
-#pragma unroll
-                for (int i = 0; i < DIM; ++i)
-#pragma unroll
-                    for (int j = 0; j < DIM; ++j) M[i][j] += ga[i] * gb[j];
-            }
-        }
-        __syncthreads();
-    }
-    if (!active) return;
-    constexpr int NS = DIM == 3 ? 6 : 3;
-    double D[NS][NS];
-    elastic_D<DIM>(s.material[2 * e], s.material[2 * e + 1], D);
-    T* ke = ke_store<T>(s) + (size_t)c * NA * NA;
-#pragma unroll
-    for (int al = 0; al < DIM; ++al)
-#pragma unroll
-        for (int be = 0; be < DIM; ++be) {
-            double v = 0.0;
-#pragma unroll
-            for (int i = 0; i < DIM; ++i)
-#pragma unroll
-                for (int j = 0; j < DIM; ++j)
-                    if (d_nonzero<DIM>(voigt<DIM>(al, i), voigt<DIM>(be, j)))
-                        v += D[voigt<DIM>(al, i)][voigt<DIM>(be, j)] * (double)M[i][j];
-            ke[(a * DIM + al) * NA + (be * NB + b)] = (T)v;
-        }
-}
-
-// ------------------------------------------------------------------------------------------------
-// k_cut_elasticity_mfma: 3D elasticity, one wavefront per cut element, the moment matrix on MFMA.
-//   M (24 x 24, component c = 8 i + a, i the direction, a the vertex) = sum_p w*_p g_p g_p^T is
-//   symmetric; padded to 32 x 32 it is three 16 x 16 tiles (upper left, upper right, lower right).
-//   Points are mapped 64 at a time into FP64 records (xi, w*) in LDS (one lane per point: IG -> IP
-//   map and sub-cell detJ).  Each MFMA step takes 4 points: lane l handles point l / 16 of the step
-//   and component column l % 16 = col, and forms in registers, from the point's record, the two
-//   gradient entries it feeds -- g[col] (direction col / 8, vertex col % 8) and g[16 + col]
-//   (direction 2, vertex col; zero padding for col >= 8) -- and w* times them: those are its A
-//   (row col, k = point) and B (k = point, column col) operands of v_mfma_f64_16x16x4f64
-//   (v_mfma_f32_16x16x4f32 with FP32 operands and FP32 accumulation on the mixed path; the records
-//   are formed in FP64 there too).  The tiles go to LDS once, and the contraction with D and the
-//   store of K_e follow as in k_cut_elasticity.
-// ------------------------------------------------------------------------------------------------
-typedef double mgpu_doublex4_t __attribute__((ext_vector_type(4)));
-typedef float mgpu_floatx4_t __attribute__((ext_vector_type(4)));
-
-template <typename T>
-__device__ inline void mfma_16x16x4(T a, T b, typename std::conditional<sizeof(T) == 8, mgpu_doublex4_t,
-                                                                        mgpu_floatx4_t>::type& acc) {
-    if constexpr (sizeof(T) == 8) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
-    else acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
-}
-
-template <typename T>
-__global__ __launch_bounds__(64) void k_cut_elasticity_mfma(DevView s) {
-    constexpr int NB = 8, NG = 24, NA = 24;
-    constexpr int MP = NG + 1;
-    using acc_t = typename std::conditional<sizeof(T) == 8, mgpu_doublex4_t, mgpu_floatx4_t>::type;
-    __shared__ double4 rec[64];
-    __shared__ T Ms[NG * MP];
-
-    const int c = s.cut_order ? s.cut_order[blockIdx.x] : (int)blockIdx.x;
-    if (s.skip && s.skip[c]) return;
-    const int lane = threadIdx.x;
-    const int e = s.cut_elems[c];
-    const int ig0 = s.ig_ptr[e];
-    const int nip = (s.ig_ptr[e + 1] - ig0) * kTet11Points;
-    double hh[3];
-    for (int d = 0; d < 3; ++d) hh[d] = s.h[d];
-
-    // the lane's component column and the constant factors of its two gradient entries
-    const int col = lane & 15, grp = lane >> 4;
-    const int a = col & 7;
-    const double sx = kHex8XiHat[a][0], sy = kHex8XiHat[a][1], sz = kHex8XiHat[a][2];
-    const bool lo_x = col < 8;                 // g[col]: d/dx (col < 8) or d/dy (col >= 8)
-    const double c_lo = lo_x ? 0.25 * sx / hh[0] : 0.25 * sy / hh[1];
-    const double c_hi = lo_x ? 0.25 * sz / hh[2] : 0.0;   // g[16 + col]: d/dz, or padding
-
-    acc_t m00 = {0, 0, 0, 0}, m01 = {0, 0, 0, 0}, m11 = {0, 0, 0, 0};
-    for (int base = 0; base < nip; base += 64) {
-        {
-            const int ip = base + lane;
-            double4 r = make_double4(0.0, 0.0, 0.0, 0.0);
-            if (ip < nip) {
-                double xi[3];
-                r.w = cut_point_map<3>(s, ig0, ip, hh, xi);
-                r.x = xi[0];
-                r.y = xi[1];
-                r.z = xi[2];
-            }
-            rec[lane] = r;
-        }
-        __syncthreads();
-        const int steps = (min(64, nip - base) + 3) >> 2;
-        for (int st = 0; st < steps; ++st) {
-            const double4 r = rec[4 * st + grp];
-            const double fx = 1.0 + sx * r.x, fy = 1.0 + sy * r.y, fz = 1.0 + sz * r.z;
-            const double lo = c_lo * (lo_x ? fy : fx) * fz;
-            const double hi = c_hi * fx * fy;
-            const T blo = (T)lo, bhi = (T)hi;
-            const T alo = (T)(r.w * lo), ahi = (T)(r.w * hi);
-            mfma_16x16x4<T>(alo, blo, m00);
-            mfma_16x16x4<T>(alo, bhi, m01);
-            mfma_16x16x4<T>(ahi, bhi, m11);
-        }
-        __syncthreads();
-    }
-    // tiles -> M in LDS (result register j of a lane: row grp + 4 j for FP64, 4 grp + j for FP32;
-    // column col), the lower left tile mirrored from the upper right one
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int row = sizeof(T) == 8 ? grp + 4 * j : 4 * grp + j;
-        Ms[row * MP + col] = m00[j];
-        if (col < 8) {
-            Ms[row * MP + 16 + col] = m01[j];
-            Ms[(16 + col) * MP + row] = m01[j];
-            if (row < 8) Ms[(16 + row) * MP + 16 + col] = m11[j];
-        }
-    }
-    __syncthreads();
-    // B^T D B: lane (a, b) owns the 3 x 3 direction block of the vertex pair (a, b)
-    const int va = lane >> 3, vb = lane & 7;
-    double D[6][6];
-    elastic_D<3>(s.material[2 * e], s.material[2 * e + 1], D);
-    T* ke = ke_store<T>(s) + (size_t)c * NA * NA;
-#pragma unroll
-    for (int al = 0; al < 3; ++al)
-#pragma unroll
-        for (int be = 0; be < 3; ++be) {
-            double v = 0.0;
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-#pragma unroll
-                for (int j = 0; j < 3; ++j)
-                    if (d_nonzero<3>(voigt<3>(al, i), voigt<3>(be, j)))
-                        v += D[voigt<3>(al, i)][voigt<3>(be, j)] * (double)Ms[(i * NB + va) * MP + j * NB + vb];
-            ke[(va * 3 + al) * NA + (be * NB + vb)] = (T)v;
-        }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -721,20 +506,15 @@ void launch_subdivision(mgpu_set* S, const int32_t* skip) {
     DevView v = S->v;
     v.skip = skip;
     dim3 g((unsigned)v.n_cut), b(64);
-    const bool f32 = S->precision == MGPU_PREC_MIXED;
-    if (dim == 3 && nf == 1) {
-        if (f32) hipLaunchKernelGGL((k_cut_diffusion<3, float>), g, b, 0, S->stream, v);
-        else hipLaunchKernelGGL((k_cut_diffusion<3, double>), g, b, 0, S->stream, v);
-    } else if (dim == 3 && nf == 3) {
-        if (f32) hipLaunchKernelGGL((k_cut_elasticity_mfma<float>), g, b, 0, S->stream, v);
-        else hipLaunchKernelGGL((k_cut_elasticity_mfma<double>), g, b, 0, S->stream, v);
-    } else if (dim == 2 && nf == 1) {
-        if (f32) hipLaunchKernelGGL((k_cut_diffusion<2, float>), g, b, 0, S->stream, v);
-        else hipLaunchKernelGGL((k_cut_diffusion<2, double>), g, b, 0, S->stream, v);
-    } else {
-        if (f32) hipLaunchKernelGGL((k_cut_elasticity<2, float>), g, b, 0, S->stream, v);
-        else hipLaunchKernelGGL((k_cut_elasticity<2, double>), g, b, 0, S->stream, v);
-    }
+    const bool f32 = S->ke_f32();
+    auto go = [&](auto kernel64, auto kernel32) {
+        if (f32) hipLaunchKernelGGL(kernel32, g, b, 0, S->stream, v);
+        else hipLaunchKernelGGL(kernel64, g, b, 0, S->stream, v);
+    };
+    if (dim == 3 && nf == 1) go(k_cut<3, 1, double>, k_cut<3, 1, float>);
+    else if (dim == 3) go(k_cut<3, 3, double>, k_cut<3, 3, float>);
+    else if (nf == 1) go(k_cut<2, 1, double>, k_cut<2, 1, float>);
+    else go(k_cut<2, 2, double>, k_cut<2, 2, float>);
 }
 
 template <int DIM, int NF, int V>
@@ -742,7 +522,7 @@ void launch_stencil_variant(mgpu_set* S, const double* u, double* vals, double* 
     constexpr int ROWS = stencil_rows<NF>(V);
     const int n_rb = (S->v.N + ROWS - 1) / ROWS;
     const dim3 grid((unsigned)(((n_rb + 7) / 8) * 8 * NF));
-    if (S->precision == MGPU_PREC_MIXED)
+    if (S->ke_f32())
         hipLaunchKernelGGL((k_stencil<DIM, NF, ROWS, stencil_direct<NF>(V), float>), grid, dim3(ROWS * NF), 0, S->stream,
                            S->v, u, vals, rhs);
     else
@@ -790,11 +570,11 @@ mgpu_status launch_assemble(mgpu_set* S, const double* u, double* vals, double* 
     if (ev) HIP_TRY(hipEventRecord(ev[2], S->stream));
     if (S->v.n_cut > 0) {
         if (learned) {
-            lq_launch_element(S->v, S->lv, nf, S->precision == MGPU_PREC_MIXED, S->stream);
+            lq_launch_element(S->v, S->lv, nf, S->ke_f32(), S->stream);
             launch_subdivision(S, S->lv.flag);
         } else if (mfit) {
             // every element takes the fitted rule: no subdivision launch
-            lq_launch_element(S->v, S->lv, nf, S->precision == MGPU_PREC_MIXED, S->stream);
+            lq_launch_element(S->v, S->lv, nf, S->ke_f32(), S->stream);
         } else {
             launch_subdivision(S, nullptr);
         }

@@ -1,18 +1,21 @@
 // generic.hip -- the generic element path of an mgpu_set: any T rows (B-spline p = 2, THB-like
 // rows with several weighted entries) and sets without a lattice.
 //
-//   k_generic_element   one wavefront per element.  The moments
+//   k_generic_nodal, k_generic_element
+//                       HEX8 / QUAD4 IP cells, one wavefront per element.  The moments
 //                         M[(i,a),(j,b)] = sum_ip w* dN_a/dx_i dN_b/dx_j
 //                       over the element's integration points (HEX_2x2x2 / QUAD_2x2 on the IP box
 //                       when uncut, TET_11 / TRI_7 on the XTK sub-cells when cut; w* = w detJ,
-//                       points with detJ < -1e-6 skipped, cl_FEM_Element_Bulk.cpp:258-355) are
-//                       staged 64 points at a time in LDS; lane (a, b) owns the DIM x DIM block.
-//                       K_p = B^T D B from M (IWG compute_jacobian,
-//                       cl_FEM_IWG_Isotropic_Struc_Linear_Bulk.cpp:200, cl_FEM_IWG_Diffusion_Bulk.cpp
-//                       :280), then K_e = T^T K_p T with the element's dense T built from its rows
-//                       (Equation_Object::build_PADofMap / get_egn_obj_jacobian_and_residual,
-//                       cl_MSI_Equation_Object.cpp:426-493, :789-842), in FP64 through LDS, written
-//                       to the element's slot of the K_e pool.
+//                       points with detJ < -1e-6 skipped, cl_FEM_Element_Bulk.cpp:258-355) come
+//                       from the cell's 3^dim moments (cut_moments.hpp), in FP64 with either
+//                       quadrature and at either precision option.  K_p = B^T D B from M (IWG
+//                       compute_jacobian, cl_FEM_IWG_Isotropic_Struc_Linear_Bulk.cpp:200,
+//                       cl_FEM_IWG_Diffusion_Bulk.cpp:280), then K_e = T^T K_p T with the element's
+//                       dense T built from its rows (Equation_Object::build_PADofMap /
+//                       get_egn_obj_jacobian_and_residual, cl_MSI_Equation_Object.cpp:426-493,
+//                       :789-842), in FP64 through LDS, written to the element's slot of the K_e
+//                       pool; with nodal rows K_e is K_p in adof order.  HEX8 elements with uniform
+//                       p = 2 rows: k_hex8_moments, then k_hex27_tensor.
 //   hex27.hip           HEX27 IP cells (HEX_3x3x3 / TET_35): K_e from the element's moments.  In scatter
 //                       mode (sets too large for a K_e pool) colour by colour, each element adding its
 //                       K_e into the CSR values after k_generic_zero.
@@ -31,6 +34,7 @@
 #include <vector>
 
 #include "../common/fem_tables.hpp"
+#include "cut_moments.hpp"
 #include "set_state.hpp"
 
 namespace mgpu {
@@ -64,251 +68,128 @@ mgpu_status gupload(mgpu_set* S, const T* src, size_t n, T** dst) {
     return MGPU_OK;
 }
 
-// Integration point ip of element e: w* and the physical gradients g[i][a] of the IP cell.
+// The element's moments in m (LDS): of the cut cell's points, or of the whole cell.  scratch: LDS.
 template <int DIM>
-__device__ inline double generic_point(const GenView& g, int e, bool cut, int ip, const double* hh,
-                                       double (*grad)[DIM == 3 ? 8 : 4]) {
-    constexpr int NB = DIM == 3 ? 8 : 4;
-    double xi[DIM];
-    double w;
-    if (!cut) {
-        // IG cell = IP cell: HEX_2x2x2 / QUAD_2x2, detJ = prod(h / 2)
-        for (int d = 0; d < DIM; ++d) xi[d] = DIM == 3 ? kHex2Xi[ip][d] : kQuad2Xi[ip][d];
-        double detJ = 1.0;
-        for (int d = 0; d < DIM; ++d) detJ *= 0.5 * hh[d];
-        w = (DIM == 3 ? kHex2W[ip] : kQuad2W[ip]) * detJ;
-    } else {
-        constexpr int NV = DIM + 1;
-        constexpr int NQ = DIM == 3 ? kTet11Points : kTri7Points;
-        const int sc = g.ig_ptr[e] + ip / NQ;
-        const int q = ip % NQ;
-        const double* X = g.ig_xi + (size_t)sc * NV * DIM;
-        double N[NV];
-        if constexpr (DIM == 3) {
-            N[0] = kTet11Xi[q][0];
-            N[1] = kTet11Xi[q][1];
-            N[2] = 1.0 - kTet11Xi[q][0] - kTet11Xi[q][1] - kTet11Xi[q][2];
-            N[3] = kTet11Xi[q][2];
-        } else {
-            N[0] = kTri7Xi[q][0];
-            N[1] = kTri7Xi[q][1];
-            N[2] = 1.0 - kTri7Xi[q][0] - kTri7Xi[q][1];
-        }
-        for (int d = 0; d < DIM; ++d) {
-            double v = 0.0;
-            for (int k = 0; k < NV; ++k) v += N[k] * X[k * DIM + d];
-            xi[d] = v;
-        }
-        double detJ;
-        if constexpr (DIM == 3) {
-            double J[3][3];
-            const int rr[3] = {0, 1, 3};
-            for (int r = 0; r < 3; ++r)
-                for (int d = 0; d < 3; ++d) J[r][d] = (X[rr[r] * 3 + d] - X[2 * 3 + d]) * (0.5 * hh[d]);
-            detJ = (J[0][0] * (J[1][1] * J[2][2] - J[2][1] * J[1][2]) -
-                    J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
-                    J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0])) / 6.0;
-        } else {
-            double J[2][2];
-            for (int r = 0; r < 2; ++r)
-                for (int d = 0; d < 2; ++d) J[r][d] = (X[r * 2 + d] - X[2 * 2 + d]) * (0.5 * hh[d]);
-            detJ = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) / 2.0;
-        }
-        w = detJ < kDetJLowerLimit ? 0.0 : (DIM == 3 ? kTet11W[q] : kTri7W[q]) * detJ;
-    }
-    lagrange_dNdxi<DIM>(xi, grad);
-    for (int i = 0; i < DIM; ++i)
-        for (int a = 0; a < NB; ++a) grad[i][a] *= 2.0 / hh[i];
-    return w;
-}
-
-constexpr int kGenLds = 24 * 24 + 8 * kGenericMaxAdofsPerType + 24 * 3 * kGenericMaxAdofsPerType;
-
-// Moment-fitted rule of a cut HEX8 / QUAD4 cell (MGPU_QUAD_MOMENT_FIT on the generic path): the
-// 3^DIM tensor points of the 3-point Gauss rule with weights W_g = sum_q w*_q L_i(x_q) L_j(y_q)
-// (L_k(z_q)) over the cell's TET_11 / TRI_7 points, L the quadratics through the nodes -s, 0, s.
-// The (bi)trilinear moment integrand has degree <= 2 per axis, so the rule gives the subdivision's
-// sum.  One wavefront: lanes over the points, then a reduction in lane order into Wg.
-constexpr int kGenFitW = kGenLds - 32;   // LDS offset of the fitted weights (doubles)
-template <int DIM>
-__device__ inline void gen_mfit_weights(const GenView& g, int e, const double* hh, double* lds, int lane) {
-    constexpr int NV = DIM + 1;
-    constexpr int NQ = DIM == 3 ? kTet11Points : kTri7Points;
-    constexpr int NW = DIM == 3 ? 27 : 9;
-    static_assert(NW * 65 <= kGenFitW, "reduction rows and the fitted weights fit the LDS");
-    const double sg = kHex3Xi[1][0];   // the 3-point Gauss node (the rule's literal)
-    const int npts = (g.ig_ptr[e + 1] - g.ig_ptr[e]) * NQ;
-    double acc[NW];
-#pragma unroll
-    for (int k = 0; k < NW; ++k) acc[k] = 0.0;
-    for (int ip = lane; ip < npts; ip += 64) {
-        const int sc = g.ig_ptr[e] + ip / NQ, q = ip % NQ;
-        const double* X = g.ig_xi + (size_t)sc * NV * DIM;
-        double N[NV];
-        if constexpr (DIM == 3) {
-            N[0] = kTet11Xi[q][0];
-            N[1] = kTet11Xi[q][1];
-            N[2] = 1.0 - kTet11Xi[q][0] - kTet11Xi[q][1] - kTet11Xi[q][2];
-            N[3] = kTet11Xi[q][2];
-        } else {
-            N[0] = kTri7Xi[q][0];
-            N[1] = kTri7Xi[q][1];
-            N[2] = 1.0 - kTri7Xi[q][0] - kTri7Xi[q][1];
-        }
-        double L[DIM][3];
-        for (int d = 0; d < DIM; ++d) {
-            double x = 0.0;
-            for (int k = 0; k < NV; ++k) x += N[k] * X[k * DIM + d];
-            L[d][0] = x * (x - sg) / (2.0 * sg * sg);
-            L[d][1] = 1.0 - x * x / (sg * sg);
-            L[d][2] = x * (x + sg) / (2.0 * sg * sg);
-        }
-        double detJ;
-        if constexpr (DIM == 3) {
-            double J[3][3];
-            const int rr[3] = {0, 1, 3};
-            for (int r = 0; r < 3; ++r)
-                for (int d = 0; d < 3; ++d) J[r][d] = (X[rr[r] * 3 + d] - X[2 * 3 + d]) * (0.5 * hh[d]);
-            detJ = (J[0][0] * (J[1][1] * J[2][2] - J[2][1] * J[1][2]) -
-                    J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
-                    J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0])) / 6.0;
-        } else {
-            double J[2][2];
-            for (int r = 0; r < 2; ++r)
-                for (int d = 0; d < 2; ++d) J[r][d] = (X[r * 2 + d] - X[2 * 2 + d]) * (0.5 * hh[d]);
-            detJ = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) / 2.0;
-        }
-        const double w = detJ < kDetJLowerLimit ? 0.0 : (DIM == 3 ? kTet11W[q] : kTri7W[q]) * detJ;
-#pragma unroll
-        for (int k = 0; k < NW; ++k) {
-            const int ix = k % 3, iy = (k / 3) % 3, iz = k / 9;
-            double v = w * L[0][ix] * L[1][iy];
-            if constexpr (DIM == 3) v *= L[2][iz];
-            acc[k] += v;
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < NW; ++k) lds[k * 65 + lane] = acc[k];
-    __syncthreads();
-    if (lane < NW) {
-        double v = 0.0;
-        for (int l = 0; l < 64; ++l) v += lds[lane * 65 + l];
-        lds[kGenFitW + lane] = v;
-    }
-    __syncthreads();
-}
-
-template <int DIM, int NF, typename T, bool MFIT>
-__global__ __launch_bounds__(64) void k_generic_element(GenView g) {
-    constexpr int NB = DIM == 3 ? 8 : 4;
-    constexpr int NG = DIM * NB;
-    constexpr int NP = NF * NB;
-    constexpr int GP = NG + 1;
-    static_assert(2 * 64 * GP * sizeof(T) <= kGenLds * sizeof(double), "LDS phases");
-    __shared__ double lds[kGenLds];
-    const int e = g.order ? g.order[blockIdx.x] : (int)blockIdx.x;
-    const int lane = threadIdx.x;
-    double hh[DIM];
+__device__ __forceinline__ void generic_moments(const GenView& g, int e, double* scratch, double* m, double* hh) {
     for (int d = 0; d < DIM; ++d) hh[d] = g.ip_box[(size_t)e * 2 * DIM + DIM + d];
-    const bool cut = g.ig_ptr[e + 1] > g.ig_ptr[e];
-    const bool fit = MFIT && cut;
-    const int npts = fit ? (DIM == 3 ? 27 : 9)
-                         : (cut ? (g.ig_ptr[e + 1] - g.ig_ptr[e]) * (DIM == 3 ? kTet11Points : kTri7Points)
-                                : (DIM == 3 ? kHex2Points : kQuad2Points));
-    if constexpr (MFIT)
-        if (fit) gen_mfit_weights<DIM>(g, e, hh, lds, lane);
+    const int ig0 = g.ig_ptr[e], nsub = g.ig_ptr[e + 1] - ig0;
+    if (nsub > 0) cut_moments<DIM>(g.ig_xi, ig0, nsub, hh, scratch, m);
+    else whole_moments<DIM>(hh, m);
+}
 
-    // phase 1: moments, lane (a, b) owns M[(i,a),(j,b)], i, j < DIM
-    T* sgw = reinterpret_cast<T*>(lds);
-    T* sg = sgw + 64 * GP;
-    const int a = (lane / NB) % NB, b = lane % NB;
-    const bool owner = lane < NB * NB;
-    T M[DIM][DIM];
-    for (int i = 0; i < DIM; ++i)
-        for (int j = 0; j < DIM; ++j) M[i][j] = T(0);
-    for (int p0 = 0; p0 < npts; p0 += 64) {
-        const int ip = p0 + lane;
-        if (ip < npts) {
-            double grad[DIM][NB];
-            double w;
-            if (fit) {
-                // tensor point ip of the 3-point Gauss rule, x fastest, and its fitted weight
-                const double nd[3] = {-kHex3Xi[1][0], 0.0, kHex3Xi[1][0]};
-                double xi[DIM];
-                xi[0] = nd[ip % 3];
-                xi[1] = nd[(ip / 3) % 3];
-                if constexpr (DIM == 3) xi[2] = nd[ip / 9];
-                lagrange_dNdxi<DIM>(xi, grad);
-                for (int i = 0; i < DIM; ++i)
-                    for (int c = 0; c < NB; ++c) grad[i][c] *= 2.0 / hh[i];
-                w = lds[kGenFitW + ip];
-            } else {
-                w = generic_point<DIM>(g, e, cut, ip, hh, grad);
-            }
-            for (int i = 0; i < DIM; ++i)
-                for (int c = 0; c < NB; ++c) {
-                    sgw[lane * GP + i * NB + c] = (T)(w * grad[i][c]);
-                    sg[lane * GP + i * NB + c] = (T)grad[i][c];
-                }
-        }
-        __syncthreads();
-        const int np = min(64, npts - p0);
-        if (owner)
-            for (int p = 0; p < np; ++p)
-                for (int i = 0; i < DIM; ++i)
-                    for (int j = 0; j < DIM; ++j) M[i][j] += sgw[p * GP + i * NB + a] * sg[p * GP + j * NB + b];
-        __syncthreads();
+// K_p's entries of the vertex pair (a, b): kv[al DIM + be] (elasticity) or kv[0].
+template <int DIM, int NF>
+__device__ __forceinline__ void generic_kp(const GenView& g, int e, const double* m, const double* hh, int a, int b, double* kv) {
+    double M[DIM][DIM];
+    moment_block<DIM>(m, a, b, hh, M);
+    if constexpr (NF == 1) {
+        double v = 0.0;
+#pragma unroll
+        for (int i = 0; i < DIM; ++i) v += M[i][i];
+        kv[0] = g.material[e] * v;
+    } else {
+        constexpr int NS = DIM == 3 ? 6 : 3;
+        double D[NS][NS];
+        elastic_D<DIM>(g.material[2 * e], g.material[2 * e + 1], D);
+#pragma unroll
+        for (int al = 0; al < DIM; ++al)
+#pragma unroll
+            for (int be = 0; be < DIM; ++be) kv[al * DIM + be] = elastic_entry<DIM>(D, M, al, be);
     }
+}
 
-    // phase 2: K_p (NP x NP) from M and the material
+// Elements with nodal T rows (a permutation): K_e is K_p with rows and columns in adof order, each lane (a, b)
+// storing its entries; no T products and no LDS for them, so that six times as many wavefronts fit
+// a CU as with the general kernel below.  62120 elements, elasticity (40^3 cells): 0.09 ms, 0.81 ms
+// with the point-wise moments and the dense T products.
+template <int DIM, int NF>
+__global__ __launch_bounds__(64) void k_generic_nodal(GenView g, const int32_t* els) {
+    constexpr int NB = DIM == 3 ? 8 : 4, NA = NF * NB;
+    __shared__ __align__(16) double lds[LinearMoments<DIM>::LDS];
+    __shared__ double m[LinearMoments<DIM>::N];
+    const int e = els[blockIdx.x], lane = threadIdx.x;
+    double hh[DIM], kv[NF * NF];
+    generic_moments<DIM>(g, e, lds, m, hh);
+    if (lane >= NB * NB) return;
+    const int a = lane / NB, b = lane % NB;
+    generic_kp<DIM, NF>(g, e, m, hh, a, b, kv);
+    const int x = g.t_col[g.t_ptr[e * NB + a]], y = g.t_col[g.t_ptr[e * NB + b]];
+    double* ke = g.ke + g.ke_off[e];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+#pragma unroll
+        for (int h = 0; h < NF; ++h) ke[(f * NB + x) * NA + h * NB + y] = kv[f * NF + h];
+}
+
+// HEX8 elements with the 27 adofs of uniform quadratic B-splines: their moments in the layout that
+// k_hex27_tensor contracts (5 per axis, the last two zero), T folded into its tables.
+__global__ __launch_bounds__(64) void k_hex8_moments(GenView g, const int32_t* els, double* mom) {
+    __shared__ __align__(16) double lds[LinearMoments<3>::LDS];
+    __shared__ double m[LinearMoments<3>::N];
+    const int e = els[blockIdx.x];
+    double hh[3];
+    generic_moments<3>(g, e, lds, m, hh);
+    for (int t = threadIdx.x; t < kHex27Moments; t += 64) {
+        const int i = t / 25, j = (t / 5) % 5, k = t % 5;
+        mom[(size_t)e * kHex27Moments + t] = i < 3 && j < 3 && k < 3 ? m[(i * 3 + j) * 3 + k] : 0.0;
+    }
+}
+
+// Any other T rows: K_p in LDS, then K_e = T^T K_p T with dense T, one column block (dof type) at a time.
+template <int DIM, int NF>
+__global__ __launch_bounds__(64) void k_generic_element(GenView g, const int32_t* els) {
+    constexpr int NB = DIM == 3 ? 8 : 4;
+    constexpr int NP = NF * NB;
+    constexpr int MX = kGenericMaxAdofsPerType;
+    constexpr int kT = NP * NP, kW = kT + NB * MX;
+    // (the moments' scratch is dead once m is formed)
+    constexpr int kLds = kW + NP * MX > LinearMoments<DIM>::LDS ? kW + NP * MX : LinearMoments<DIM>::LDS;
+    __shared__ __align__(16) double lds[kLds];
+    __shared__ double m[LinearMoments<DIM>::N];
+    const int e = els[blockIdx.x], lane = threadIdx.x;
+    double hh[DIM];
+    generic_moments<DIM>(g, e, lds, m, hh);
     double* Kp = lds;
-    double* Tt = Kp + NP * NP;                        // [NB][na_t]
-    double* W = Tt + NB * kGenericMaxAdofsPerType;     // [NP][NF * na_t]
+    double* Tt = lds + kT;   // [NB][na_t]
+    double* W = lds + kW;    // [NP][na_t]
     const int na_t = g.na_t[e];
     const int NA = NF * na_t;
-    if (owner) {
-        if (NF == 1) {
-            double v = 0.0;
-            for (int i = 0; i < DIM; ++i) v += (double)M[i][i];
-            Kp[a * NP + b] = g.material[e] * v;
-        } else {
-            constexpr int NS = DIM == 3 ? 6 : 3;
-            double D[NS][NS];
-            elastic_D<DIM>(g.material[2 * e], g.material[2 * e + 1], D);
-            for (int al = 0; al < DIM; ++al)
-                for (int be = 0; be < DIM; ++be) {
-                    double v = 0.0;
-                    for (int i = 0; i < DIM; ++i)
-                        for (int j = 0; j < DIM; ++j)
-                            if (d_nonzero<DIM>(voigt<DIM>(al, i), voigt<DIM>(be, j)))
-                                v += D[voigt<DIM>(al, i)][voigt<DIM>(be, j)] * (double)M[i][j];
-                    Kp[(al * NB + a) * NP + be * NB + b] = v;
-                }
-        }
+    if (lane < NB * NB) {
+        const int a = lane / NB, b = lane % NB;
+        double kv[NF * NF];
+        generic_kp<DIM, NF>(g, e, m, hh, a, b, kv);
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int h = 0; h < NF; ++h) Kp[(f * NB + a) * NP + h * NB + b] = kv[f * NF + h];
     }
-    // phase 3: dense element-local T (per dof type; the same rows serve every type)
+    // dense element-local T (per dof type; the same rows serve every type)
     for (int idx = lane; idx < NB * na_t; idx += 64) Tt[idx] = 0.0;
     __syncthreads();
     if (lane < NB)
         for (int q = g.t_ptr[e * NB + lane]; q < g.t_ptr[e * NB + lane + 1]; ++q) Tt[lane * na_t + g.t_col[q]] += g.t_w[q];
     __syncthreads();
-    // phase 4: W = K_p T (block diagonal T over dof types)
-    for (int idx = lane; idx < NP * NA; idx += 64) {
-        const int r = idx / NA, cy = idx % NA;
-        const int gg = cy / na_t, y = cy % na_t;
-        double v = 0.0;
-        for (int b2 = 0; b2 < NB; ++b2) v += Kp[r * NP + gg * NB + b2] * Tt[b2 * na_t + y];
-        W[idx] = v;
-    }
-    __syncthreads();
-    // phase 5: K_e = T^T W
     double* ke = g.ke + g.ke_off[e];
-    for (int idx = lane; idx < NA * NA; idx += 64) {
-        const int X = idx / NA, Y = idx % NA;
-        const int f = X / na_t, x = X % na_t;
-        double v = 0.0;
-        for (int b1 = 0; b1 < NB; ++b1) v += Tt[b1 * na_t + x] * W[(f * NB + b1) * NA + Y];
-        ke[idx] = v;
+    for (int h = 0; h < NF; ++h) {
+        // W = K_p(:, h) T
+        for (int idx = lane; idx < NP * na_t; idx += 64) {
+            const int r = idx / na_t, y = idx - na_t * r;
+            double v = 0.0;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) v += Kp[r * NP + h * NB + b] * Tt[b * na_t + y];
+            W[idx] = v;
+        }
+        __syncthreads();
+        // K_e(:, h) = T^T W
+        for (int idx = lane; idx < NA * na_t; idx += 64) {
+            const int X = idx / na_t, y = idx - na_t * X;
+            const int f = X / na_t, x = X - na_t * f;
+            double v = 0.0;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) v += Tt[b * na_t + x] * W[(f * NB + b) * na_t + y];
+            ke[(size_t)X * NA + h * na_t + y] = v;
+        }
+        __syncthreads();
     }
 }
 
@@ -431,6 +312,16 @@ mgpu_status generic_upload(mgpu_set* S, const mgpu_set_desc& d) {
             (rc = upload_gather_src(S, h.gather_src, g)))
             return rc;
     }
+    auto tensor = [&](int32_t e) { return !h.t_perm.empty() && h.t_perm[(size_t)e * kHex27PermStride + 27] != 0; };
+    bool any_tensor = false;
+    for (int32_t e = 0; e < h.n_el && !any_tensor; ++e) any_tensor = tensor(e);
+    if (h.n_el > 0 && (h.nb == 27 || any_tensor)) {
+        void* p = nullptr;
+        HIP_TRY(hipMalloc(&p, (size_t)h.n_el * kHex27Moments * sizeof(double)));
+        S->allocs.push_back(p);
+        S->d_mom = static_cast<double*>(p);
+        if ((rc = gupload(S, h.t_perm.data(), h.t_perm.size(), const_cast<uint8_t**>(&g.t_perm)))) return rc;
+    }
     if (h.nb == 27 && h.n_el > 0) {
         // the elements with tensor T first, within each colour (scatter mode) or over the set
         std::vector<int32_t> els(h.colour_el), cp(h.colour_ptr);
@@ -441,18 +332,10 @@ mgpu_status generic_upload(mgpu_set* S, const mgpu_set_desc& d) {
         }
         S->n_tensor.clear();
         for (size_t c = 0; c + 1 < cp.size(); ++c) {
-            auto mid = std::stable_partition(els.begin() + cp[c], els.begin() + cp[c + 1], [&](int32_t e) {
-                return h.t_perm[(size_t)e * kHex27PermStride + 27] != 0;
-            });
+            auto mid = std::stable_partition(els.begin() + cp[c], els.begin() + cp[c + 1], tensor);
             S->n_tensor.push_back((int32_t)(mid - els.begin()) - cp[c]);
         }
-        void* p = nullptr;
-        HIP_TRY(hipMalloc(&p, (size_t)h.n_el * kHex27Moments * sizeof(double)));
-        S->allocs.push_back(p);
-        S->d_mom = static_cast<double*>(p);
-        if ((rc = gupload(S, els.data(), els.size(), const_cast<int32_t**>(&S->d_hex_els))) ||
-            (rc = gupload(S, h.t_perm.data(), h.t_perm.size(), const_cast<uint8_t**>(&g.t_perm))))
-            return rc;
+        if ((rc = gupload(S, els.data(), els.size(), const_cast<int32_t**>(&S->d_els)))) return rc;
     }
     if (h.scatter) {
         if ((rc = gupload(S, h.topo.data(), h.topo.size(), const_cast<int32_t**>(&g.topo))) ||
@@ -470,6 +353,26 @@ mgpu_status generic_upload(mgpu_set* S, const mgpu_set_desc& d) {
         });
         if (h.n_el > 0 && (rc = gupload(S, order.data(), order.size(), const_cast<int32_t**>(&S->d_gen_order))))
             return rc;
+        if (h.nb != 27 && h.n_el > 0) {
+            // HEX8 / QUAD4 elements by class (nodal rows, tensor rows, any other), in element order and
+            // most sub-cells first
+            std::vector<uint8_t> cls((size_t)h.n_el, 2);
+            for (int32_t e = 0; e < h.n_el; ++e) {
+                bool nodal = h.na_t[(size_t)e] == h.nb;
+                for (int64_t q = (int64_t)e * h.nb; q < (int64_t)(e + 1) * h.nb && nodal; ++q)
+                    nodal = d.t_ptr[q + 1] - d.t_ptr[q] == 1 && d.t_weight[d.t_ptr[q]] == 1.0;
+                cls[(size_t)e] = nodal ? 0 : (tensor(e) ? 1 : 2);
+            }
+            std::vector<int32_t> els((size_t)h.n_el);
+            std::iota(els.begin(), els.end(), 0);
+            for (int c = 0; c < 3; ++c) S->n_class[c] = (int32_t)std::count(cls.begin(), cls.end(), (uint8_t)c);
+            auto by_class = [&](int32_t x, int32_t y) { return cls[(size_t)x] < cls[(size_t)y]; };
+            std::stable_sort(els.begin(), els.end(), by_class);
+            std::stable_sort(order.begin(), order.end(), by_class);
+            if ((rc = gupload(S, els.data(), els.size(), const_cast<int32_t**>(&S->d_els))) ||
+                (rc = gupload(S, order.data(), order.size(), const_cast<int32_t**>(&S->d_els_order))))
+                return rc;
+        }
     }
     const size_t n_ke = h.ke_off.empty() ? 0 : (size_t)h.ke_off.back();
     if (n_ke > 0) {
@@ -482,24 +385,18 @@ mgpu_status generic_upload(mgpu_set* S, const mgpu_set_desc& d) {
 }
 
 namespace {
-template <bool MFIT>
-void launch_generic_element(mgpu_set* S, bool f32, dim3 gr, dim3 bl) {
-    const SetHost& h = S->h;
-    if (h.dim == 3 && h.nf == 1) {
-        if (f32) hipLaunchKernelGGL((k_generic_element<3, 1, float, MFIT>), gr, bl, 0, S->stream, S->g);
-        else hipLaunchKernelGGL((k_generic_element<3, 1, double, MFIT>), gr, bl, 0, S->stream, S->g);
-    } else if (h.dim == 3) {
-        if (f32) hipLaunchKernelGGL((k_generic_element<3, 3, float, MFIT>), gr, bl, 0, S->stream, S->g);
-        else hipLaunchKernelGGL((k_generic_element<3, 3, double, MFIT>), gr, bl, 0, S->stream, S->g);
-    } else if (h.nf == 1) {
-        if (f32) hipLaunchKernelGGL((k_generic_element<2, 1, float, MFIT>), gr, bl, 0, S->stream, S->g);
-        else hipLaunchKernelGGL((k_generic_element<2, 1, double, MFIT>), gr, bl, 0, S->stream, S->g);
-    } else {
-        if (f32) hipLaunchKernelGGL((k_generic_element<2, 2, float, MFIT>), gr, bl, 0, S->stream, S->g);
-        else hipLaunchKernelGGL((k_generic_element<2, 2, double, MFIT>), gr, bl, 0, S->stream, S->g);
+template <int DIM, int NF>
+void launch_linear_elements(mgpu_set* S, double* vals) {
+    const int32_t* els = S->g.order ? S->d_els_order : S->d_els;
+    const int32_t n0 = S->n_class[0], n1 = S->n_class[1], n2 = S->n_class[2];
+    if (n0 > 0) hipLaunchKernelGGL((k_generic_nodal<DIM, NF>), dim3((unsigned)n0), dim3(64), 0, S->stream, S->g, els);
+    if (n1 > 0) {
+        hipLaunchKernelGGL(k_hex8_moments, dim3((unsigned)n1), dim3(64), 0, S->stream, S->g, els + n0, S->d_mom);
+        launch_hex27_elements(S->g, NF, false, n1, 0, els + n0, S->d_mom, vals, S->stream);
     }
+    if (n2 > 0)
+        hipLaunchKernelGGL((k_generic_element<DIM, NF>), dim3((unsigned)n2), dim3(64), 0, S->stream, S->g, els + n0 + n1);
 }
-
 
 // Lanes per row: 16, 32 or 64, the least that holds the longest K_e row (64 at most) and lets a
 // wavefront's rows fit kRowsMaxLds; as many rows a block as that space and 256 threads allow.
@@ -533,8 +430,6 @@ mgpu_status launch_generic(mgpu_set* S, const double* u, double* vals, double* r
     if (ev)
         for (int k = 0; k < 3; ++k) HIP_TRY(hipEventRecord(ev[k], S->stream));
     if (h.n_el > 0) {
-        const bool f32 = S->precision == MGPU_PREC_MIXED;
-        const dim3 gr((unsigned)h.n_el), bl(64);
         if (h.nb == 27 && h.scatter) {
             // zero the values, then the elements colour by colour
             launch_hex27_moments(S->g, S->d_mom, S->stream);
@@ -544,17 +439,19 @@ mgpu_status launch_generic(mgpu_set* S, const double* u, double* vals, double* r
             for (size_t c = 0; c + 1 < h.colour_ptr.size(); ++c) {
                 const int32_t c0 = h.colour_ptr[c], cnt = h.colour_ptr[c + 1] - c0;
                 if (cnt > 0)
-                    launch_hex27_elements(S->g, h.nf, true, S->n_tensor[c], cnt - S->n_tensor[c], S->d_hex_els + c0,
+                    launch_hex27_elements(S->g, h.nf, true, S->n_tensor[c], cnt - S->n_tensor[c], S->d_els + c0,
                                           S->d_mom, vals, S->stream);
             }
         } else if (h.nb == 27) {
             launch_hex27_moments(S->g, S->d_mom, S->stream);
-            launch_hex27_elements(S->g, h.nf, false, S->n_tensor[0], h.n_el - S->n_tensor[0], S->d_hex_els, S->d_mom,
+            launch_hex27_elements(S->g, h.nf, false, S->n_tensor[0], h.n_el - S->n_tensor[0], S->d_els, S->d_mom,
                                   vals, S->stream);
-        } else if (S->quadrature == MGPU_QUAD_MOMENT_FIT) {
-            launch_generic_element<true>(S, f32, gr, bl);
+        } else if (h.dim == 3) {
+            if (h.nf == 1) launch_linear_elements<3, 1>(S, vals);
+            else launch_linear_elements<3, 3>(S, vals);
         } else {
-            launch_generic_element<false>(S, f32, gr, bl);
+            if (h.nf == 1) launch_linear_elements<2, 1>(S, vals);
+            else launch_linear_elements<2, 2>(S, vals);
         }
         HIP_TRY(hipGetLastError());
     }

@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../common/fem_tables.hpp"
+#include "cut_moments.hpp"
 #include "set_state.hpp"
 
 namespace mgpu {
@@ -46,9 +47,10 @@ constexpr double kQuad1D[2][3][3] = {
 };
 
 // v[kind][tau][3 alpha + beta][m]: coefficients of F_alpha F_beta in the basis; tau = 2 [alpha differentiated] +
-// [beta differentiated]; kind 0 Lagrange, 1 B-spline.
+// [beta differentiated]; kind 0 Lagrange, 1 B-spline; kind 2 the B-splines on a HEX8 cell (their linear
+// interpolant: l_0 / 2, 1 / 2, l_1 / 2 with l_0 = (1 - x) / 2, l_1 = (1 + x) / 2) in the basis {l_0^2, l_0 l_1, l_1^2, -, -}.
 struct AxisTables {
-    double v[2][4][9][5];
+    double v[3][4][9][5];
     constexpr AxisTables() : v{} {
         for (int kind = 0; kind < 2; ++kind)
             for (int tau = 0; tau < 4; ++tau)
@@ -70,6 +72,18 @@ struct AxisTables {
                         o[3] = r[3];
                         o[4] = r[4];
                     }
+        for (int tau = 0; tau < 4; ++tau)
+            for (int al = 0; al < 3; ++al)
+                for (int be = 0; be < 3; ++be) {
+                    // coefficients in {l_0, l_1}: of the value, or of the (constant) derivative
+                    const double lin[3][2] = {{0.5, 0.0}, {0.5, 0.5}, {0.0, 0.5}}, der[3] = {-0.25, 0.0, 0.25};
+                    const double p[2] = {tau & 2 ? der[al] : lin[al][0], tau & 2 ? der[al] : lin[al][1]};
+                    const double q[2] = {tau & 1 ? der[be] : lin[be][0], tau & 1 ? der[be] : lin[be][1]};
+                    double* o = v[2][tau][3 * al + be];
+                    o[0] = p[0] * q[0];
+                    o[1] = p[0] * q[1] + p[1] * q[0];
+                    o[2] = p[1] * q[1];
+                }
     }
 };
 __constant__ const AxisTables kAxis{};
@@ -93,23 +107,6 @@ __device__ __forceinline__ void hex27_basis(double x, double* v) {
     v[2] = 0.5 * (x2 + x);
     v[3] = -x * v[1];
     v[4] = x * v[3];
-}
-
-// a + b over the two halves of the wavefront (SWAP 32) or of each half (16): lanes of the first get the
-// sum of a, lanes of the second that of b
-template <int SWAP>
-__device__ __forceinline__ double swap_add(double a, double b) {
-    const uint64_t ua = __double_as_longlong(a), ub = __double_as_longlong(b);
-    uint32_t r[4];
-#pragma unroll
-    for (int w = 0; w < 2; ++w) {
-        const uint32_t x = (uint32_t)(ua >> (32 * w)), y = (uint32_t)(ub >> (32 * w));
-        const auto s = SWAP == 32 ? __builtin_amdgcn_permlane32_swap(x, y, false, false)
-                                  : __builtin_amdgcn_permlane16_swap(x, y, false, false);
-        r[w] = s[0];
-        r[2 + w] = s[1];
-    }
-    return __longlong_as_double(((uint64_t)r[1] << 32) | r[0]) + __longlong_as_double(((uint64_t)r[3] << 32) | r[2]);
 }
 
 constexpr int kMomBatch = 64;                          // sub-tets staged at a time
@@ -143,24 +140,7 @@ __device__ __forceinline__ void hex27_cut_moments(const GenView& g, int ig0, int
                 X[2 * n] = v.x;
                 X[2 * n + 1] = v.y;
             }
-            double J[3][3];
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                J[0][d] = X[d] - X[6 + d];
-                J[1][d] = X[3 + d] - X[6 + d];
-                J[2][d] = X[9 + d] - X[6 + d];
-            }
-            const double detJ = (J[0][0] * (J[1][1] * J[2][2] - J[2][1] * J[1][2]) -
-                                 J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
-                                 J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0])) * vol6;
-            double* T = lds + lane * kMomTet;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                T[4 * d] = X[6 + d];
-#pragma unroll
-                for (int r = 0; r < 3; ++r) T[4 * d + 1 + r] = J[r][d];
-            }
-            T[12] = detJ < kDetJLowerLimit ? 0.0 : detJ;
+            stage_simplex<3, false>(X, vol6, lds + lane * kMomTet);
         }
         __syncthreads();
         for (int p0 = 0; p0 < npts; p0 += 64) {
@@ -189,29 +169,19 @@ __device__ __forceinline__ void hex27_cut_moments(const GenView& g, int ig0, int
             }
         }
     }
-    // values v and v + 33 by half wavefront, then r and r + 17 by quarter: register r of quarter c holds
-    // value r + 17 (c & 1) + 33 (c >> 1)
-    constexpr int NV = NP * 5;
-    double h[34];
-#pragma unroll
-    for (int v = 0; v < 34; ++v)
-        h[v] = v < 33 ? swap_add<32>(acc[v / 5][v % 5], v + 33 < NV ? acc[(v + 33 < NV ? v + 33 : 0) / 5][(v + 33) % 5] : 0.0) : 0.0;
+    using WS = WaveSums<NP * 5>;
     __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 17; ++r) lds[r * 68 + (lane >> 4) * 17 + (lane & 15)] = swap_add<16>(h[r], h[r + 17]);
+    WS::store(&acc[0][0], lds, lane);
     __syncthreads();
-    for (int t = lane; t < 68; t += 64) {
-        const int r = t >> 2, c = t & 3;
-        const int v = r + ((c & 1) ? 17 : 0) + ((c & 2) ? 33 : 0);
-        double s = 0.0;
-#pragma unroll
-        for (int l = 0; l < 16; ++l) s += lds[r * 68 + c * 17 + l];
-        if (((c & 1) == 0 || r < 16) && v < NV) out[P0 * 5 + v] = s;
+    for (int t = lane; t < 4 * WS::NP; t += 64) {
+        const int v = WS::value(t);
+        const double s = WS::sum(lds, t);
+        if (v < NP * 5) out[P0 * 5 + v] = s;
     }
 }
 
 __global__ __launch_bounds__(64) void k_hex27_moments(GenView g, double* mom) {
-    __shared__ double lds[kMomLds];
+    __shared__ __align__(16) double lds[kMomLds];
     // 16 blocks in a row hold 8 elements, the role changing after 8: the round robin over the 8 XCDs
     // gives each both roles in turn
     const int b = blockIdx.x, role = (b >> 3) & 1, be = (b >> 4) * 8 + (b & 7);
@@ -402,8 +372,8 @@ __device__ __forceinline__ void hex27_material(const GenView& g, int e, double& 
 }
 
 // ------------------------------------------------------------------------------------------------
-// k_hex27_tensor: K_e of elements whose T is a tensor product (t_perm[e][27] = 1 nodal, 2 B-spline;
-// t_perm[e][y] the tensor index of the element's adof y).  Threads 0 .. 3 NA - 1 hold a column of K_e and
+// k_hex27_tensor: K_e of elements whose T is a tensor product (t_perm[e][27] = 1 nodal, 2 B-spline, 3 B-spline on
+// a HEX8 cell; t_perm[e][y] the tensor index of the element's adof y).  Threads 0 .. 3 NA - 1 hold a column of K_e and
 // write NF rows' worth of consecutive values per step (stores of whole lines).  Without the products by T
 // and their LDS space four blocks instead of two fit a CU: 0.44 ms for 32^3 elements of 81 x 81 (1.7 GB
 // written, 3.9 TB/s), against 1.7 ms on the general path.

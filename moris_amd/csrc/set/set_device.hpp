@@ -107,8 +107,8 @@ struct GenView {
     const int32_t* order;
     const int64_t* rank_off;     // [n_el + 1]
     const uint16_t* rank;        // [na_t][na_t] per element: column of adof y among adof x's neighbours
-    // HEX27 sets: per element the tensor index of each adof where T is a tensor product (entry 27: 1
-    // nodal rows, 2 uniform quadratic B-splines, 0 any other T)
+    // 3D sets: per element the tensor index of each adof where T is a tensor product with 27 adofs
+    // (entry 27: 1 nodal rows, 2 uniform quadratic B-splines, 3 those of HEX8 cells, 0 any other T)
     const uint8_t* t_perm;       // [n_el][kHex27PermStride]
 };
 
@@ -173,103 +173,6 @@ __device__ inline void lagrange_dNdxi(const double* xi, double (*out)[DIM == 3 ?
             out[1][a] = 0.25 * (1.0 + xi[0] * sx) * sy;
         }
     }
-}
-
-// ------------------------------------------------------------------------------------------------
-// Integration point ip of the cut element's IG sub-cells: its parametric position in the IP cell
-// (Space_Interpolator::map_integration_point, cl_MTK_Space_Interpolator.cpp:1381-1397) and its
-// weight w* = w detJ (0 where detJ < -1e-6, cl_FEM_Element_Bulk.cpp:291), all in FP64.
-// ------------------------------------------------------------------------------------------------
-template <int DIM>
-__device__ inline double cut_point_map(const DevView& s, int ig0, int ip, const double* hh, double* xip) {
-    constexpr int NV = DIM + 1;
-    constexpr int NQ = DIM == 3 ? kTet11Points : kTri7Points;
-    const int sc = ig0 + ip / NQ;
-    const int q = ip % NQ;
-    const double* X = s.ig_xi + (size_t)sc * NV * DIM;
-    double N[NV];
-    if constexpr (DIM == 3) {
-        N[0] = kTet11Xi[q][0];
-        N[1] = kTet11Xi[q][1];
-        N[2] = 1.0 - kTet11Xi[q][0] - kTet11Xi[q][1] - kTet11Xi[q][2];
-        N[3] = kTet11Xi[q][2];
-    } else {
-        N[0] = kTri7Xi[q][0];
-        N[1] = kTri7Xi[q][1];
-        N[2] = 1.0 - kTri7Xi[q][0] - kTri7Xi[q][1];
-    }
-    for (int d = 0; d < DIM; ++d) {
-        double v = 0.0;
-        for (int k = 0; k < NV; ++k) v += N[k] * X[k * DIM + d];
-        xip[d] = v;
-    }
-    double detJ;
-    if constexpr (DIM == 3) {
-        double J[3][3];
-        const int rr[3] = {0, 1, 3};
-        for (int r = 0; r < 3; ++r)
-            for (int d = 0; d < 3; ++d) J[r][d] = (X[rr[r] * 3 + d] - X[2 * 3 + d]) * (0.5 * hh[d]);
-        detJ = (J[0][0] * (J[1][1] * J[2][2] - J[2][1] * J[1][2]) -
-                J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
-                J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0])) / 6.0;
-    } else {
-        double J[2][2];
-        for (int r = 0; r < 2; ++r)
-            for (int d = 0; d < 2; ++d) J[r][d] = (X[r * 2 + d] - X[2 * 2 + d]) * (0.5 * hh[d]);
-        detJ = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) / 2.0;
-    }
-    return detJ < kDetJLowerLimit ? 0.0 : (DIM == 3 ? kTet11W[q] : kTri7W[q]) * detJ;
-}
-
-// ------------------------------------------------------------------------------------------------
-// Integration point ip of the cut element's IG sub-cells: weight w* and IP-cell gradients g[i][a].
-// ------------------------------------------------------------------------------------------------
-template <int DIM>
-__device__ inline double cut_point(const DevView& s, int ig0, int ip, const double* hh,
-                                   double (*g)[DIM == 3 ? 8 : 4]) {
-    constexpr int NV = DIM + 1;
-    constexpr int NQ = DIM == 3 ? kTet11Points : kTri7Points;
-    const int sc = ig0 + ip / NQ;
-    const int q = ip % NQ;
-    const double* X = s.ig_xi + (size_t)sc * NV * DIM;
-    double N[NV];
-    if constexpr (DIM == 3) {
-        N[0] = kTet11Xi[q][0];
-        N[1] = kTet11Xi[q][1];
-        N[2] = 1.0 - kTet11Xi[q][0] - kTet11Xi[q][1] - kTet11Xi[q][2];
-        N[3] = kTet11Xi[q][2];
-    } else {
-        N[0] = kTri7Xi[q][0];
-        N[1] = kTri7Xi[q][1];
-        N[2] = 1.0 - kTri7Xi[q][0] - kTri7Xi[q][1];
-    }
-    double xip[DIM];
-    for (int d = 0; d < DIM; ++d) {
-        double v = 0.0;
-        for (int k = 0; k < NV; ++k) v += N[k] * X[k * DIM + d];
-        xip[d] = v;
-    }
-    // detJ of the simplex in physical space: rows X_r - X_2 (r = 0, 1 [, 3]) scaled by h/2
-    double detJ;
-    if constexpr (DIM == 3) {
-        double J[3][3];
-        const int rr[3] = {0, 1, 3};
-        for (int r = 0; r < 3; ++r)
-            for (int d = 0; d < 3; ++d) J[r][d] = (X[rr[r] * 3 + d] - X[2 * 3 + d]) * (0.5 * hh[d]);
-        detJ = (J[0][0] * (J[1][1] * J[2][2] - J[2][1] * J[1][2]) -
-                J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) +
-                J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0])) / 6.0;
-    } else {
-        double J[2][2];
-        for (int r = 0; r < 2; ++r)
-            for (int d = 0; d < 2; ++d) J[r][d] = (X[r * 2 + d] - X[2 * 2 + d]) * (0.5 * hh[d]);
-        detJ = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) / 2.0;
-    }
-    const double w = detJ < kDetJLowerLimit ? 0.0 : (DIM == 3 ? kTet11W[q] : kTri7W[q]) * detJ;
-    lagrange_dNdxi<DIM>(xip, g);
-    for (int i = 0; i < DIM; ++i)
-        for (int a = 0; a < (DIM == 3 ? 8 : 4); ++a) g[i][a] *= 2.0 / hh[i];
-    return w;
 }
 
 }  // namespace mgpu

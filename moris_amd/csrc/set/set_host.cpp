@@ -37,13 +37,15 @@ void parallel_for(int64_t n, F f) {
 }
 }  // namespace
 
-// The tensor form of a HEX27 element's T (27 x 27, dense in D), if it has one: every column equal,
-// bit for bit, to a product T1[a_0][b_0] T1[a_1][b_1] T1[a_2][b_2], each (b_0, b_1, b_2) once.  The
-// entries of T1 are dyadic, so the products are exact in any order.
-static void hex27_tensor_form(const double* D, uint8_t* perm) {
-    static const double T1[2][3][3] = {{{1.0, 0.0, 0.0}, {0.0, 1.0, 0.0}, {0.0, 0.0, 1.0}},
-                                       {{0.5, 0.5, 0.0}, {0.125, 0.75, 0.125}, {0.0, 0.5, 0.5}}};
-    for (int kind = 0; kind < 2; ++kind) {
+// The tensor form of a 3D element's T (nb x 27, dense in D), if it has one: every column equal, bit for
+// bit, to a product T1[a_0][b_0] T1[a_1][b_1] T1[a_2][b_2], each (b_0, b_1, b_2) once.  The entries of T1
+// are dyadic, so the products are exact in any order.  HEX27: nodal rows (1) and uniform quadratic
+// B-splines (2); HEX8: the latter (3).
+static void tensor_form(const double* D, int nb, uint8_t* perm) {
+    static const double T1[3][3][3] = {{{1.0, 0.0, 0.0}, {0.0, 1.0, 0.0}, {0.0, 0.0, 1.0}},
+                                       {{0.5, 0.5, 0.0}, {0.125, 0.75, 0.125}, {0.0, 0.5, 0.5}},
+                                       {{0.5, 0.5, 0.0}, {0.0, 0.5, 0.5}, {0.0, 0.0, 0.0}}};
+    for (int kind = nb == 27 ? 0 : 2; kind < (nb == 27 ? 2 : 3); ++kind) {
         bool used[27] = {};
         int y = 0;
         for (; y < 27; ++y) {
@@ -51,11 +53,11 @@ static void hex27_tensor_form(const double* D, uint8_t* perm) {
             for (; c < 27; ++c) {
                 if (used[c]) continue;
                 int a = 0;
-                for (; a < 27; ++a) {
-                    const int* hf = kHex27Half[a];
+                for (; a < nb; ++a) {
+                    const int* hf = nb == 27 ? kHex27Half[a] : kHex8Off[a];
                     if (D[a * 27 + y] != T1[kind][hf[0]][c / 9] * T1[kind][hf[1]][(c / 3) % 3] * T1[kind][hf[2]][c % 3]) break;
                 }
-                if (a == 27) break;
+                if (a == nb) break;
             }
             if (c == 27) break;
             used[c] = true;
@@ -101,15 +103,16 @@ mgpu_status build_generic(const mgpu_set_desc& d, SetHost& h, std::string* err) 
         *err = "an element has more than " + std::to_string(kGenericMaxAdofsPerType) + " adofs per dof type";
         return MGPU_ERR_UNSUPPORTED;
     }
-    if (nb == 27) {
+    for (int32_t n : h.na_t) h.na_t_max = std::max(h.na_t_max, n);
+    if (h.dim == 3 && (nb == 27 || h.na_t_max >= 27)) {
         h.t_perm.assign((size_t)h.n_el * kHex27PermStride, 0);
         parallel_for(h.n_el, [&](int64_t e) {
             if (h.na_t[(size_t)e] != 27) return;
             double D[27 * 27] = {};
-            for (int b = 0; b < 27; ++b)
+            for (int b = 0; b < nb; ++b)
                 for (int32_t q = d.t_ptr[e * nb + b]; q < d.t_ptr[e * nb + b + 1]; ++q)
                     D[b * 27 + h.t_col[(size_t)q]] += d.t_weight[q];
-            hex27_tensor_form(D, h.t_perm.data() + e * kHex27PermStride);
+            tensor_form(D, nb, h.t_perm.data() + e * kHex27PermStride);
         });
     }
     h.topo_ptr.assign((size_t)h.n_el + 1, 0);
@@ -118,7 +121,6 @@ mgpu_status build_generic(const mgpu_set_desc& d, SetHost& h, std::string* err) 
         const int64_t na = (int64_t)nf * h.na_t[(size_t)e];
         h.topo_ptr[(size_t)e + 1] = h.topo_ptr[(size_t)e] + na;
         h.ke_off[(size_t)e + 1] = h.ke_off[(size_t)e] + na * na;
-        h.na_t_max = std::max(h.na_t_max, h.na_t[(size_t)e]);
     }
     h.topo.resize((size_t)h.topo_ptr[(size_t)h.n_el]);
     parallel_for(h.n_el, [&](int64_t e) {

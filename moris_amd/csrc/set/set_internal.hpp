@@ -66,9 +66,10 @@ struct SetHost {
     std::vector<int64_t> topo_ptr;       // [n_el + 1] into topo (nf * na_t per element; both paths)
     std::vector<int64_t> ke_off;         // [n_el + 1] K_e offsets, (nf * na_t)^2 per element
     std::vector<int32_t> t_col;          // [n T entries] element-local column of each T entry
-    // HEX27 sets, kHex27PermStride entries per element: where the element's T is the tensor product of
-    // one 1D matrix per axis, the tensor index (b_0 3 + b_1) 3 + b_2 of each of its 27 adofs and, last,
-    // that matrix: 1 the identity (nodal rows), 2 the uniform quadratic B-splines; last 0: any other T
+    // 3D sets with elements of 27 adofs, kHex27PermStride entries per element: where the element's T is the
+    // tensor product of one 1D matrix per axis, the tensor index (b_0 3 + b_1) 3 + b_2 of each of its 27
+    // adofs and, last, that matrix: 1 the identity (nodal rows of HEX27 cells), 2 the uniform quadratic
+    // B-splines on HEX27 cells, 3 on HEX8 cells; last 0: any other T
     std::vector<uint8_t> t_perm;
     bool rows = false;
     int32_t max_nbr = 0;                 // most neighbours of an adof (per dof type)

@@ -229,3 +229,33 @@ def test_lattice_moment_fit_refused_in_2d():
     S = M.Set(P.desc, keepalive=P)
     with pytest.raises(M.MgpuError, match="3D"):
         S.options(M.PREC_MIXED, M.QUAD_MOMENT_FIT)
+
+
+@pytest.mark.parametrize("iwg", [M.IWG_SPATIALDIFF_BULK, M.IWG_STRUC_LINEAR_BULK])
+@pytest.mark.parametrize("order,m", [(1, 1), (1, 2), (1, 3), (2, 3)])
+def test_linear_cells_with_few_and_many_sub_tets(iwg, order, m):
+    """HEX8 cells take K from 27 moments, 64 sub-tets staged at a time, 64 points at a time: elements given
+    as 6, 48 and 162 sub-tets (less than one batch, one, three; a remainder of points in each) on the
+    lattice and the generic path against the oracle.  FP64 sums of 66 .. 1782 positive terms in another
+    order, up to 1e-14; TET_11 integrates the trilinear stiffness (degree 4), so K equals the uncut
+    cell's up to its literals' 1e-13."""
+    print("case", iwg, order, m, flush=True)
+    spec, keep = M.make_spec(3, (3, 2, 2), iwg=iwg, bspline_order=order)
+    P = M.Problem(spec, keep)
+    d = M.SetDesc()
+    M.ctypes.memmove(M.ctypes.byref(d), M.ctypes.byref(P.desc), M.ctypes.sizeof(M.SetDesc))
+    tets = _box_tets(m)
+    ig_ptr = np.zeros(P.n_elements + 1, np.int32)
+    ig_ptr[2:] = len(tets)                        # element 1, and the last element
+    ig_ptr[-1] = 2 * len(tets)
+    ig_xi = np.ascontiguousarray(np.concatenate([tets, tets]).reshape(-1))
+    d.ig_ptr = ig_ptr.ctypes.data_as(M.ctypes.POINTER(M.ctypes.c_int32))
+    d.ig_xi = ig_xi.ctypes.data_as(M.ctypes.POINTER(M.ctypes.c_double))
+    S = M.Set(d, keepalive=(P, ig_ptr, ig_xi))
+    rp, ci = S.pattern()
+    u = np.random.default_rng(SEED + 25).uniform(-1.0, 1.0, S.n_rows)
+    vo, Ro, _ = O.assemble_desc(d, rp, ci, u)
+    vals, R = S.compute_jacobian_and_residual(u)
+    assert rel(vals, vo) <= 1e-14 and rel(R, Ro) <= 1e-14, (rel(vals, vo), rel(R, Ro))
+    v_box, _ = M.Set(P.desc, keepalive=P).compute_jacobian_and_residual(u)
+    assert rel(vals, v_box) <= 1e-12
