@@ -295,12 +295,6 @@ __global__ __launch_bounds__(kThreads) void k_gm_add(int32_t n, const double* u,
     for (int64_t r = (int64_t)blockIdx.x * kThreads + threadIdx.x; r < n; r += (int64_t)gridDim.x * kThreads) x[r] += u[r];
 }
 
-// ILU path: z = v_j before M^-1 is applied to it in place (nothing once the cycle has ended).
-__global__ __launch_bounds__(kThreads) void k_gm_copy(int32_t n, const double* v, double* z, const State* st) {
-    if (st->cycle_end) return;
-    for (int64_t r = (int64_t)blockIdx.x * kThreads + threadIdx.x; r < n; r += (int64_t)gridDim.x * kThreads) z[r] = v[r];
-}
-
 __global__ __launch_bounds__(kThreads) void k_gm_final(const double* partial, State* st) {
     __shared__ double sh[kThreads];
     double a = 0.0;
@@ -411,8 +405,7 @@ mgpu_status gmres_run(int32_t n, const int32_t* rp, const int32_t* ci, const dou
                 gm::launch_spmv<false>(L, n, rp, ci, vals, dinv, vj, nullptr, w, partial, st, s);
             } else {
                 // w = K M^-1 v_j
-                hipLaunchKernelGGL(gm::k_gm_copy, gv, t, 0, s, n, vj, zb, st);
-                ilu_apply_launch(pc, zb, &st->cycle_end, s);
+                ilu_apply_launch(pc, vj, zb, &st->cycle_end, s);
                 gm::launch_spmv<false>(L, n, rp, ci, vals, dinv, zb, nullptr, w, partial, st, s, false);
             }
             hipLaunchKernelGGL(gm::k_gm_zero_col, dim3(1), dim3(gm::kMaxRestart + 1), 0, s, st);
@@ -431,7 +424,7 @@ mgpu_status gmres_run(int32_t n, const int32_t* rp, const int32_t* ci, const dou
         } else {
             // x += M^-1 V y
             hipLaunchKernelGGL(gm::k_gm_vy, gv, t, 0, s, n, V, ldv, zb, st);
-            ilu_apply_launch(pc, zb, nullptr, s);
+            ilu_apply_launch(pc, zb, zb, nullptr, s);
             hipLaunchKernelGGL(gm::k_gm_add, gv, t, 0, s, n, zb, x);
         }
         GM_TRY(hipGetLastError());

@@ -434,3 +434,43 @@ def test_full_size_displacement_error_with_ghost(case):
     assert out["fp64"]["K"] <= 1e-12 and out["fp64"]["euclid"] <= 1e-8
     assert out["mixed+learned"]["K"] <= 1e-6
     assert out["mixed+learned"]["L2"] <= 1e-5 and out["mixed+learned"]["euclid"] <= 1e-5
+
+
+@pytest.mark.parametrize("kind,n", [("diagonal", 1), ("diagonal", 700), ("band", 3), ("band", 65), ("band", 513),
+                                    ("random", 97), ("random", 2000), ("arrow", 700), ("grid", 16383), ("grid", 16384)])
+def test_ilu_apply_solves_with_its_factors(kind, n):
+    """z = U^-1 L^-1 v against sparse triangular solves on the host with the handle's own factors: one row per
+    level (band), one level (diagonal), a row of n entries (arrow: many steps a row), rows of differing
+    length, and the longest vector of the one-workgroup solve (16383) beside the first that takes a
+    launch per level.  Substitution in another order of summation: 1e-12 (diagonally dominant, condition
+    below 10, at most 700 terms a row)."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as spla
+    rng = np.random.default_rng(n)
+    if kind == "diagonal":
+        K = sp.eye(n)
+    elif kind == "band":
+        K = sp.diags([np.ones(n - 1), np.ones(n - 1), np.ones(max(n - 2, 0))], [-1, 1, -2])
+    elif kind == "random":
+        K = sp.random(n, n, density=min(1.0, 12.0 / n), random_state=7)
+    elif kind == "arrow":
+        K = sp.lil_matrix((n, n))
+        K[n - 1, :] = 1.0
+        K[:, n - 1] = 1.0
+    else:
+        w = 128
+        K = sp.diags([np.ones(n - w), np.ones(n - 1), np.ones(n - 1), np.ones(n - w)], [-w, -1, 1, w])
+    K = sp.csr_matrix(K)
+    K.data = rng.uniform(-1.0, 1.0, K.nnz)
+    K = sp.csr_matrix(K + sp.diags(np.abs(K).sum(axis=1).A1 + 1.0))
+    K.sort_indices()
+    A = SV.DeviceCSR(K.indptr, K.indices, K.data)
+    F = SV.ILU(A, fill_level=0)
+    _, rp, ci, lu, _ = F.factors()
+    LU = sp.csr_matrix((lu, ci, rp), shape=(n, n))
+    v = rng.uniform(-1.0, 1.0, n)
+    L = sp.tril(LU, -1) + sp.eye(n)
+    z = spla.spsolve_triangular(sp.csr_matrix(sp.triu(LU)), spla.spsolve_triangular(sp.csr_matrix(L), v, lower=True), lower=False)
+    got = F.apply(v)
+    assert np.linalg.norm(got - z) <= 1e-12 * np.linalg.norm(z)
+    assert np.array_equal(F.apply(v).view(np.uint64), got.view(np.uint64))
