@@ -474,3 +474,29 @@ def test_ilu_apply_solves_with_its_factors(kind, n):
     got = F.apply(v)
     assert np.linalg.norm(got - z) <= 1e-12 * np.linalg.norm(z)
     assert np.array_equal(F.apply(v).view(np.uint64), got.view(np.uint64))
+
+
+@pytest.mark.parametrize("n,dense", [(1, 0), (7, 0), (256, 0), (257, 0), (16385, 0), (70001, 0), (300, 1), (1, 1)])
+def test_cg_sizes_and_row_lengths(n, dense):
+    """CG at grid edges (one row, a block, one row more, more rows than lanes of the largest grid) and with
+    rows longer than the entries in flight (dense), against a host solve: rtol 1e-12 on condition
+    numbers below 10, so the solutions agree to 1e-10; a repeated call gives the same bits, also after one
+    that stopped at an odd iteration limit."""
+    import scipy.sparse as sp
+    import scipy.sparse.linalg as spla
+    rng = np.random.default_rng(n)
+    if dense:
+        B = rng.uniform(-1.0, 1.0, (n, n))
+        K = sp.csr_matrix(np.eye(n) * n + B @ B.T)
+    else:
+        K = sp.csr_matrix(sp.diags([-np.ones(n - 1), rng.uniform(3.0, 4.0, n), -np.ones(n - 1)], [-1, 0, 1]))
+    K.sort_indices()
+    b = rng.uniform(-1.0, 1.0, n)
+    A = SV.DeviceCSR(K.indptr, K.indices, K.data)
+    x, info = SV.cg(A, b, rtol=1e-12)
+    want = spla.spsolve(K.tocsc(), b)
+    assert info.converged == 1 and np.linalg.norm(x - want) <= 1e-10 * np.linalg.norm(want)
+    _, short = SV.cg(A, b, rtol=1e-30, max_iter=3)
+    assert short.iterations <= 3 and short.converged in (0, 1)
+    x2, info2 = SV.cg(A, b, rtol=1e-12)
+    assert np.array_equal(x2.view(np.uint64), x.view(np.uint64)) and info2.iterations == info.iterations
