@@ -52,10 +52,11 @@ def log(*a):
 # with two rocprofv3 --pmc runs (FETCH_SIZE scaled x2.0, WRITE_SIZE x1.0 by the copy-kernel
 # calibration): 97,555 KiB x 2 + 445,915 KiB.
 STENCIL_TRAFFIC_BYTES = (97555 * 2 + 445915) * 1024
-# The same for k_generic_hex27<3,double,false> on the 32^3 HEX27 gyroid set (gather mode):
-# 109,644 KiB fetched, 1,470,336 KiB written (the K_e pool).
+# The same for an earlier HEX27 element kernel, k_generic_hex27<3,double,false>, on the 32^3 gyroid set:
+# 109,644 KiB fetched, 1,470,336 KiB written (the K_e pool, which k_hex27_tensor writes now; its counters
+# have not been taken, so no line reports these bytes).
 HEX27_32_TRAFFIC_BYTES = (109644 * 2 + 1470336) * 1024
-# The same for k_generic_hex27<3,double,true,false> on the 48^3-base THB gyroid set (scatter mode,
+# The same for the earlier k_generic_hex27<3,double,true,false> on the 48^3-base THB gyroid set (scatter mode,
 # FP64 atomic adds), summed over the 42 colour launches of one call: 4,423,474 KiB fetched,
 # 70,966,197 KiB written (the atomics count as write requests only).
 THB48_SCATTER_TRAFFIC_BYTES = (4423474 * 2 + 70966197) * 1024
@@ -161,8 +162,9 @@ def cpu_baseline(P, S, u, budget_s=20.0, probe_n=4000, rule="TET_11", budget_1co
 def run_hex27(args):
     """HEX27 IP cells with p = 2 B-splines (the quadratic configuration): 3D elasticity on an n^3
     lattice of the unit cube cut by a gyroid of period 4 cells, HEX_3x3x3 on whole cells and TET_35
-    on the XTK sub-tets, generic element path.  One JSON line: FP64 and mixed-precision assembly
-    rates, the moment kernel's MFMA rate, mixed-vs-FP64 error, and the oracle on a sample."""
+    on the XTK sub-tets, generic element path.  One JSON line: assembly rates with either precision and
+    quadrature option (one FP64 path on this set), the element kernels' FP64 rate, and the oracle on a
+    sample."""
     n = args.n if args.n_given else (16 if args.refine else 32)
     spec, keep = M.make_spec(3, (n, n, n), iwg=M.IWG_STRUC_LINEAR_BULK, ls_kind=M.LS_GYROID,
                              gyroid_scale=2 * np.pi * n / 4.0, bspline_order=2, lagrange_order=2,
@@ -173,27 +175,22 @@ def run_hex27(args):
                                                                          P.n_ig))
     S = M.Set(P.desc, keepalive=P)
     t_host = time.time() - t0
-    # sets whose element matrices exceed 2^28 entries assemble in scatter mode (no K_e pool);
+    # sets whose element matrices exceed 2^30 entries assemble in scatter mode (no K_e pool);
     # MGPU_GENERIC_SCATTER=1 / =0 forces it on / off
     ke_entries = int(np.sum(np.diff(S.topology_offsets()).astype(np.int64) ** 2))
     force = os.environ.get("MGPU_GENERIC_SCATTER", "")[:1]
-    mode = "scatter" if force == "1" or (ke_entries > 2 ** 28 and force != "0") else "gather"
+    mode = "scatter" if force == "1" or (ke_entries > 2 ** 30 and force != "0") else "gather"
     log("hex27 setup %.1fs: %d^3, elements %d, cut %d, sub-tets %d, rows %d, nnz %d, %s mode" % (
         time.time() - t0, n, P.n_elements, P.n_cut, P.n_ig, S.n_rows, S.nnz, mode))
     u = np.random.default_rng(SEED + 27).uniform(-1.0, 1.0, S.n_rows)
     ub, vb, rb = M.DeviceBuffer.from_array(u), M.DeviceBuffer(8 * S.nnz), M.DeviceBuffer(8 * S.n_rows)
     ig = np.diff(P.arrays()["ig_ptr"])
     npts = np.where(ig > 0, ig * 35, 27)
-    # executed MFMA work: per 64-point chunk the 21 upper 16 x 16 tiles of M x 16 k-steps of 4 points;
-    # per element and dof-type block h >= f (6 blocks, the other 3 mirrored) the 2 n_t + n_t^2 tiles
-    # of K_p T and T^T (K_p T) x 7 k-steps (n_t = ceil(adofs per type / 16))
-    n_t = (np.diff(S.topology_offsets()) // 3 + 15) // 16
-    proj_flops = float(np.sum(6 * (2 * n_t + n_t * n_t)) * 7 * 2 * 16 * 16 * 4)
-    mfma_flops = float(np.sum(np.ceil(npts / 64.0)) * 21 * 16 * 2 * 16 * 16 * 4) + proj_flops
-    # the moment-fitted rule (cut elements): only the weights on MFMA, 2 tiles x 16 k-steps per
-    # 64-point chunk of the TET_35 points (M by sum factorisation on the VALU)
-    mfma_flops_fit = float(np.sum(np.where(ig > 0, np.ceil(npts / 64.0) * 2 * 16,
-                                           np.ceil(npts / 64.0) * 21 * 16)) * 2 * 16 * 16 * 4) + proj_flops
+    # executed FP64 work of the element kernels: per cut point (lanes past an element's points included) and
+    # wavefront of k_hex27_moments 111 vector operations, 74 of them multiply-adds, two wavefronts; per element
+    # the axis-by-axis contraction of the 125 moments (9 x (3 x 25 + 6 x 45 + 6 x 81) x 5 multiply-adds)
+    flops = float(np.sum(np.where(ig > 0, 64 * np.ceil(npts / 64.0), 0.0))) * 2 * (111 + 74)
+    flops += 2.0 * P.n_elements * 9 * 5 * (3 * 25 + 6 * 45 + 6 * 81)
     native, _, _ = elasticity_flops(int(npts.sum()), P.n_elements, nb=27)
     out = {"metric": "elements/s for K+R assembly, HEX27 p=2 elasticity (gyroid cut), generic path",
            "unit": "elements/s", "n_gpus": 1, "steps": args.steps, "higher_is_better": True,
@@ -211,11 +208,10 @@ def run_hex27(args):
         S.autotune(ub, vb, rb, iters=2)   # element order of the gather mode
         per, st = S.time_assemble(ub, vb, rb, max(3, args.steps))
         res[name] = (vb.to_array(np.float64, S.nnz), rb.to_array(np.float64, S.n_rows))
-        flops = mfma_flops_fit if quad == M.QUAD_MOMENT_FIT else mfma_flops
         out[name] = {"value": P.n_elements / (per * 1e-3), "ms_per_call": per,
-                     "ms_element_kernel": st[2], "ms_gather": st[3], "ms_rhs": st[4],
-                     "element_kernel_mfma_TFLOP/s": flops / (st[2] * 1e-3) / 1e12,
-                     "element_kernel_native_TFLOP/s": native / (st[2] * 1e-3) / 1e12}
+                     "ms_element_kernels": st[2], "ms_rows": st[3] + st[4],
+                     "element_kernels_TFLOP/s": flops / (st[2] * 1e-3) / 1e12,
+                     "element_kernels_reference_shape_TFLOP/s": native / (st[2] * 1e-3) / 1e12}
         log("hex27 %s: %.3f ms per call, stages %s" % (name, per, ["%.4f" % x for x in st]))
     for name in ("mixed", "fp64_moment_fit", "mixed_moment_fit"):
         out[name]["rel_err_K_vs_fp64"] = float(np.linalg.norm(res[name][0] - res["fp64"][0]) /
@@ -224,21 +220,12 @@ def run_hex27(args):
     out["value_path"] = "mixed_moment_fit"
     out["dtype"] = "f32+f64"
     out["max_rel_err_K_mixed_vs_fp64"] = out["mixed"]["rel_err_K_vs_fp64"]
-    out["mfma_flops_per_call"] = mfma_flops
-    out["mfma_flops_per_call_moment_fit"] = mfma_flops_fit
-    out["native_flops_per_call"] = native
-    out["roofline"] = {"bound": "mfma", "kernel": "k_generic_hex27<3,double>",
-                       "achieved": out["fp64"]["element_kernel_mfma_TFLOP/s"], "peak": FP64_PEAK_TFLOPS,
-                       "unit": "TFLOP/s", "frac": out["fp64"]["element_kernel_mfma_TFLOP/s"] / FP64_PEAK_TFLOPS,
+    out["executed_flops_per_call"] = flops
+    out["reference_shape_flops_per_call"] = native
+    out["roofline"] = {"bound": "fp64", "kernel": "k_hex27_moments + k_hex27_tensor / k_hex27_general",
+                       "achieved": out["fp64"]["element_kernels_TFLOP/s"], "peak": FP64_PEAK_TFLOPS,
+                       "unit": "TFLOP/s", "frac": out["fp64"]["element_kernels_TFLOP/s"] / FP64_PEAK_TFLOPS,
                        "traffic": None}
-    if n == 32 and not args.refine and mode == "gather":
-        out["roofline"]["traffic"] = HEX27_32_TRAFFIC_BYTES
-        out["roofline"]["traffic_source"] = "rocprofv3 --pmc FETCH_SIZE (x2.0) + WRITE_SIZE (x1.0) per launch"
-    elif n == 48 and args.refine == 1 and mode == "scatter":
-        out["roofline"]["traffic"] = THB48_SCATTER_TRAFFIC_BYTES
-        out["roofline"]["traffic_source"] = ("rocprofv3 --pmc FETCH_SIZE (x2.0) + WRITE_SIZE (x1.0), summed over "
-                                             "the colour launches of one call; the atomic adds count as write "
-                                             "requests only, so this is a lower bound")
     if not args.refine:
         # the set-up of the same set on the GPU (cut, numbering, T rows at the 27 nodes, pattern)
         from moris_amd import gpu_setup as G
@@ -247,8 +234,8 @@ def run_hex27(args):
         t1 = time.time()
         Gs = G.GpuSetup(spec, keep)
         wall = time.time() - t1
-        # the generic set is made on the host from the set-up's descriptor (its gather lists are
-        # built there): the rest of a re-meshing loop's cost
+        # the generic set is made on the host from the set-up's descriptor (its pattern and rank tables
+        # are built there): the rest of a re-meshing loop's cost
         t1 = time.time()
         S_g = M.Set(Gs.desc, keepalive=Gs)
         t_set = time.time() - t1
