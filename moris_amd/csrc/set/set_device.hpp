@@ -155,24 +155,4 @@ __device__ inline void elastic_D(double E, double nu, double (*D)[DIM == 3 ? 6 :
     }
 }
 
-// dN/dxi of the linear Lagrange IP cell at xi: out[i][a].
-template <int DIM>
-__device__ inline void lagrange_dNdxi(const double* xi, double (*out)[DIM == 3 ? 8 : 4]) {
-    if constexpr (DIM == 3) {
-        for (int a = 0; a < 8; ++a) {
-            const double sx = kHex8XiHat[a][0], sy = kHex8XiHat[a][1], sz = kHex8XiHat[a][2];
-            const double fx = 1.0 + xi[0] * sx, fy = 1.0 + xi[1] * sy, fz = 1.0 + xi[2] * sz;
-            out[0][a] = 0.125 * sx * fy * fz;
-            out[1][a] = 0.125 * fx * sy * fz;
-            out[2][a] = 0.125 * fx * fy * sz;
-        }
-    } else {
-        for (int a = 0; a < 4; ++a) {
-            const double sx = kQuad4XiHat[a][0], sy = kQuad4XiHat[a][1];
-            out[0][a] = 0.25 * sx * (1.0 + xi[1] * sy);
-            out[1][a] = 0.25 * (1.0 + xi[0] * sx) * sy;
-        }
-    }
-}
-
 }  // namespace mgpu
