@@ -168,6 +168,15 @@ __global__ __launch_bounds__(kThreads) void k_spmv(int32_t n, const int32_t* rp,
     if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
+// Whether the solve has ended, the same in every thread of the block.  Block 0 of k_update and k_pupdate
+// sets the flag while other blocks of the launch may still read it: one thread reads it, so that no
+// wavefront leaves a block whose others go on to its barriers and sums.
+__device__ inline bool ended(const State* st, int32_t* sh_done) {
+    if (threadIdx.x == 0) *sh_done = st->done;
+    __syncthreads();
+    return *sh_done != 0;
+}
+
 enum { kInit = 0, kFinal = 1 };
 
 // The sum of n partials in a fixed order, the same in every thread of every block.
@@ -213,12 +222,14 @@ __global__ __launch_bounds__(kThreads) void k_init_z(int32_t n, const double* r,
 }
 
 // alpha = rho / p.q, x += alpha p, r -= alpha q, z = D^-1 r; partial streams [1] r.z, [2] r.r.  Every block finds
-// the same p.q; block 0 notes a breakdown, which stops the kernels that follow.
+// the same p.q, and at a breakdown none updates its part of x and r, whether it sees block 0's note of
+// it already or finds p.q itself: x stays the last iterate.
 __global__ __launch_bounds__(kThreads) void k_update(int32_t n, double* x, double* r, double* z, const double* p,
                                                      const double* q, const double* dinv, double* partial, int n_spmv,
                                                      int odd, State* st) {
     __shared__ double sh[kThreads];
-    if (st->done) return;
+    __shared__ int32_t sh_done;
+    if (ended(st, &sh_done)) return;
     const double pq = partial_sum(partial, n_spmv, sh);
     if (!(pq > 0.0)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) st->done = 3;
@@ -246,11 +257,12 @@ __global__ __launch_bounds__(kThreads) void k_update(int32_t n, double* x, doubl
 
 // rho' = r.z, the stopping tests, p = z + (rho' / rho) p.  Every block finds the same sums; block 0 writes the
 // state: rho' beside the rho that the others still read, and done, whether another block sees it already
-// or not (p is not needed any more).
+// (and leaves) or not (and updates its part of p, which is not needed any more).
 __global__ __launch_bounds__(kThreads) void k_pupdate(int32_t n, double* p, const double* z, const double* partial,
                                                       int n_vec, int odd, State* st) {
     __shared__ double sh[kThreads];
-    if (st->done) return;
+    __shared__ int32_t sh_done;
+    if (ended(st, &sh_done)) return;
     const double rz = partial_sum(partial + kBlocks, n_vec, sh), rr = partial_sum(partial + 2 * kBlocks, n_vec, sh);
     const bool converged = rr <= st->rtol2 * st->rr0;
     if (blockIdx.x == 0 && threadIdx.x == 0) {

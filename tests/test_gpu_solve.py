@@ -19,6 +19,8 @@
   3.5e-7 and Euclidean 3.9e-7 (both under the 1e-5 target); C5 L2 1.4e-7 but Euclidean 2.9e-5,
   above the target, held here to 5e-5.  The FP64 GPU path is within 2e-11 (Euclidean) on both.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -113,6 +115,48 @@ def test_cg_reports_breakdown_on_indefinite_matrix():
     SV.apply_dirichlet(A, rb, fixed)
     with pytest.raises(M.MgpuError):
         SV.cg(A, rb, rtol=1e-10)
+
+
+@pytest.mark.parametrize("kind", ["first", "later"])
+@pytest.mark.parametrize("n", [5, 257, 300001])
+def test_cg_breakdown_returns_the_last_iterate(kind, n):
+    """At p.Kp <= 0 x is the iterate before it, bit for bit, on one block, two blocks and more blocks than
+    run at a time: the initial guess where the first direction breaks down, else what the same number
+    of iterations gives as their limit; and the same on every call, with its true residual."""
+    print("case", kind, n, flush=True)
+    rng = np.random.default_rng(n)
+    b = rng.uniform(-1.0, 1.0, n)
+    if kind == "first":
+        d = np.ones(n)
+        d[n // 2] = -1e9
+        b[n // 2] = 1.0
+        K = sp.csr_matrix(sp.diags(d))
+    else:   # a Laplacian with its low modes shifted below zero
+        K = sp.csr_matrix(sp.diags([-np.ones(n - 1), np.full(n, 1.6), -np.ones(n - 1)], [-1, 0, 1]))
+    K.sort_indices()
+    x0 = rng.uniform(-1.0, 1.0, n) if kind == "later" else np.zeros(n)
+    A = SV.DeviceCSR(K.indptr, K.indices, K.data)
+    bb = M.DeviceBuffer.from_array(b)
+
+    def solve(max_iter):
+        xb, info = M.DeviceBuffer.from_array(x0), SV.CgInfo()
+        rc = SV._lib().mgpu_cg_solve(n, A.row_ptr.ptr, A.col_idx.ptr, A.vals.ptr, bb.ptr, xb.ptr, 1e-14, max_iter, None,
+                                     ctypes.byref(info))
+        return rc, xb.to_array(np.float64, n), info
+
+    runs = [solve(20000) for _ in range(5)]
+    its = runs[0][2].iterations
+    assert (its == 0) == (kind == "first")
+    rc_it, x_it, info_it = solve(its)
+    assert rc_it == 0 and info_it.iterations == its
+    if kind == "first":
+        assert np.array_equal(x_it.view(np.uint64), x0.view(np.uint64))
+    want = np.linalg.norm(b - K @ x_it) / np.linalg.norm(b - K @ x0)
+    for rc, x, info in runs:
+        assert rc != 0 and info.iterations == its and info.converged == 0
+        assert np.array_equal(x.view(np.uint64), x_it.view(np.uint64))
+        assert info.true_rel_residual == info_it.true_rel_residual
+        assert abs(info.true_rel_residual - want) <= 1e-10 * want
 
 
 def _unsymmetric_nitsche_system(n=10):
