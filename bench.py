@@ -187,10 +187,11 @@ def run_hex27(args):
     ig = np.diff(P.arrays()["ig_ptr"])
     npts = np.where(ig > 0, ig * 35, 27)
     # executed FP64 work of the element kernels: per cut point (lanes past an element's points included) and
-    # wavefront of k_hex27_moments 111 vector operations, 74 of them multiply-adds, two wavefronts; per element
-    # the axis-by-axis contraction of the 125 moments (9 x (3 x 25 + 6 x 45 + 6 x 81) x 5 multiply-adds)
-    flops = float(np.sum(np.where(ig > 0, 64 * np.ceil(npts / 64.0), 0.0))) * 2 * (111 + 74)
-    flops += 2.0 * P.n_elements * 9 * 5 * (3 * 25 + 6 * 45 + 6 * 81)
+    # wavefront of k_hex27_moments 112 vector operations, 71.5 of them multiply-adds (means of its two
+    # wavefronts); per element the axis-by-axis contraction of the 125 moments, 45 multiply-adds per
+    # moment vector and pair of equal factors, 54 of differing ones: 25 x 144 + 45 x 288 + 81 x 288
+    flops = float(np.sum(np.where(ig > 0, 64 * np.ceil(npts / 64.0), 0.0))) * 2 * (112 + 71.5)
+    flops += 2.0 * P.n_elements * (25 * 144 + 45 * 288 + 81 * 288)
     native, _, _ = elasticity_flops(int(npts.sum()), P.n_elements, nb=27)
     out = {"metric": "elements/s for K+R assembly, HEX27 p=2 elasticity (gyroid cut), generic path",
            "unit": "elements/s", "n_gpus": 1, "steps": args.steps, "higher_is_better": True,

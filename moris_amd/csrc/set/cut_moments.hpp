@@ -57,10 +57,10 @@ struct WaveSums {
 };
 
 // A sub-cell (simplex, vertices X) as the affine map of its rule: per axis vertex 2 and the edges to the
-// others, the coordinates scaled to [0, 1] where UNIT; then the factor of the rule's weights (0 where
-// the sub-cell's detJ < -1e-6).  vol: product of the half extents of the cell over DIM!.
-template <int DIM, bool UNIT>
-__device__ __forceinline__ void stage_simplex(const double* X, double vol, double* T) {
+// others, in the coordinate (x - lo) sc; then the factor of the rule's weights (0 where the sub-cell's
+// detJ < -1e-6).  vol: product of the half extents of the cell over DIM!.
+template <int DIM>
+__device__ __forceinline__ void stage_simplex(const double* X, const double* lo, const double* sc, double vol, double* T) {
     double J[DIM][DIM];
 #pragma unroll
     for (int d = 0; d < DIM; ++d)
@@ -74,9 +74,9 @@ __device__ __forceinline__ void stage_simplex(const double* X, double vol, doubl
         detJ = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * vol;
 #pragma unroll
     for (int d = 0; d < DIM; ++d) {
-        T[(DIM + 1) * d] = UNIT ? 0.5 * (1.0 + X[2 * DIM + d]) : X[2 * DIM + d];
+        T[(DIM + 1) * d] = (X[2 * DIM + d] - lo[d]) * sc[d];
 #pragma unroll
-        for (int r = 0; r < DIM; ++r) T[(DIM + 1) * d + 1 + r] = UNIT ? 0.5 * J[r][d] : J[r][d];
+        for (int r = 0; r < DIM; ++r) T[(DIM + 1) * d + 1 + r] = J[r][d] * sc[d];
     }
     T[(DIM + 1) * DIM] = detJ < kDetJLowerLimit ? 0.0 : detJ;
 }
@@ -120,7 +120,8 @@ __device__ __forceinline__ void cut_moments(const double* ig_xi, int ig0, int ns
                 X[2 * n] = v.x;
                 X[2 * n + 1] = v.y;
             }
-            stage_simplex<DIM, true>(X, vol, lds + lane * LM::TET);
+            const double lo[3] = {-1.0, -1.0, -1.0}, sc[3] = {0.5, 0.5, 0.5};   // [-1, 1] to [0, 1]
+            stage_simplex<DIM>(X, lo, sc, vol, lds + lane * LM::TET);
         }
         __syncthreads();
         for (int p0 = 0; p0 < npts; p0 += 64) {

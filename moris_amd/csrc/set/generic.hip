@@ -122,16 +122,23 @@ __global__ __launch_bounds__(64) void k_generic_nodal(GenView g, const int32_t* 
 }
 
 // HEX8 elements with the 27 adofs of uniform quadratic B-splines: their moments in the layout that
-// k_hex27_tensor contracts (5 per axis, the last two zero), T folded into its tables.
+// k_hex27_tensor contracts (5 per axis, the last two zero), T folded into its tables: on the cell the B-splines
+// are their linear interpolants l_0 / 2, 1 / 2, l_1 / 2 = f_0 l_0 + f_1 l_1, the derivatives constant.
 __global__ __launch_bounds__(64) void k_hex8_moments(GenView g, const int32_t* els, double* mom) {
     __shared__ __align__(16) double lds[LinearMoments<3>::LDS];
     __shared__ double m[LinearMoments<3>::N];
     const int e = els[blockIdx.x];
     double hh[3];
     generic_moments<3>(g, e, lds, m, hh);
+    double* out = mom + (size_t)e * kHex27MomStride;
     for (int t = threadIdx.x; t < kHex27Moments; t += 64) {
         const int i = t / 25, j = (t / 5) % 5, k = t % 5;
-        mom[(size_t)e * kHex27Moments + t] = i < 3 && j < 3 && k < 3 ? m[(i * 3 + j) * 3 + k] : 0.0;
+        out[t] = i < 3 && j < 3 && k < 3 ? m[(i * 3 + j) * 3 + k] : 0.0;
+    }
+    if (threadIdx.x < 54) {
+        const int r = threadIdx.x % 18, al = (r % 9) / 3, k = r % 3;
+        out[kHex27MomTab + threadIdx.x] =
+            k == 2 ? 0.0 : (r >= 9 ? 0.25 * (al - 1) : (al == 1 || al == 2 * k ? 0.5 : 0.0));
     }
 }
 
@@ -317,7 +324,7 @@ mgpu_status generic_upload(mgpu_set* S, const mgpu_set_desc& d) {
     for (int32_t e = 0; e < h.n_el && !any_tensor; ++e) any_tensor = tensor(e);
     if (h.n_el > 0 && (h.nb == 27 || any_tensor)) {
         void* p = nullptr;
-        HIP_TRY(hipMalloc(&p, (size_t)h.n_el * kHex27Moments * sizeof(double)));
+        HIP_TRY(hipMalloc(&p, (size_t)h.n_el * kHex27MomStride * sizeof(double)));
         S->allocs.push_back(p);
         S->d_mom = static_cast<double*>(p);
         if ((rc = gupload(S, h.t_perm.data(), h.t_perm.size(), const_cast<uint8_t**>(&g.t_perm)))) return rc;

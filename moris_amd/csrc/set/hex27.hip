@@ -5,11 +5,11 @@
 // integration points (TET_35 on the XTK sub-tets, w* = w detJ, points with detJ < -1e-6 skipped,
 // cl_FEM_Element_Bulk.cpp:258-355; HEX_3x3x3 on whole cells) is therefore a fixed linear function of
 // the cell's 125 moments of degree <= 4 per axis, and factorises over the axes.
-// Both quadrature options take this route, in FP64 at either precision option: it is the point sum
-// in another order, and closer to that sum than a point-wise accumulation of M (K within 1.2e-16 ..
-// 2.9e-16 of sums in 80-bit long double, against 7.8e-16 .. 2.1e-15).  32^3 cut cells, elasticity, p = 2 (1.1M
-// sub-tets, 37.8M points): element kernels 11.8 ms with M accumulated point by point on 21 FP64 MFMA
-// tiles, 0.91 ms here.
+// Both quadrature options take this route, in FP64 at either precision option: it is the point sum in
+// another order, K (as a whole) within 1.2e-16 .. 2.8e-16 of sums in 80-bit long double, against 7.8e-16 ..
+// 2.1e-15 with M accumulated point by point; for its small entries see the basis below.  32^3 cut cells,
+// elasticity, p = 2 (1.1M sub-tets, 37.8M points): element kernels 11.8 ms with M accumulated point by point
+// on 21 FP64 MFMA tiles, 0.98 ms here.
 //
 //   k_hex27_moments    two wavefronts per element: the 125 moments of a cut cell, a lane a point (whole
 //                      cells: closed form).
@@ -20,6 +20,8 @@
 //                      Lagrange tables, K_e = T^T K_p T on FP64 MFMA.
 // K_e goes to the element's slot of the pool, or (scatter mode) is added into the CSR values.
 #include <hip/hip_runtime.h>
+
+#include <cmath>
 
 #include "../common/fem_tables.hpp"
 #include "cut_moments.hpp"
@@ -32,81 +34,70 @@ namespace {
 typedef double doublex4_t __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------------------------------------
-// 1D tables.  The moments are taken in the basis {l_0, l_1, l_2, c, c x} of each axis: the quadratic
-// Lagrange functions of the nodes -1, 0, 1 and c = x^3 - x, which vanishes there.  A polynomial of degree
-// <= 4 is sum_n p(n - 1) l_n + p_3 c + p_4 c x, so the tables of the (dyadic) 1D functions below are
-// exact, and the basis is well conditioned.  Monomials cost 4e-15 on K of nodal rows; the degree-4
-// Lagrange basis through the Gauss-Legendre nodes, with rounded tables, is as accurate as this one but
-// takes three times the arithmetic per point.
-// kQuad1D: polynomial coefficients [function][power] of l_0 .. l_2 and of the uniform quadratic B-splines
-// of a cell (those of the T rows: vertex rows 1/2 1/2, mid rows 1/8 3/4 1/8, times l_0 .. l_2).
+// The moments are taken in the Bernstein basis of the box that holds the cell's material: on each axis
+// the sub-cells' vertices span [lo, hi], t = (x - lo) / (hi - lo), s = 1 - t, and the basis is
+// g_m = t^m s^(4 - m), m <= 4, so that every moment is a sum of terms of one sign.  The 1D functions (and
+// their derivatives) are f_0 s^2 + f_1 t s + f_2 t^2 with coefficients of the box (axis_coefficient), a
+// product F_a F_b is sum_kl f_ak f_bl g_(k+l).  Because t spans [0, 1] over the material itself, the terms of a
+// product are of the size of the product: small entries (a basis function that a sliver in a corner,
+// along an edge or around the cell's centre barely touches) keep their digits as in the sum over the
+// points.  Relative error of the worst diagonal entry, slivers of edge 0.1 .. 1e-5 at a corner: 4e-16 ..
+// 6e-15, summed point by point 3e-15 .. 2e-11; a fixed basis on [-1, 1] fails either at the corners (Lagrange
+// functions and multiples of x^3 - x: 2e-12 .. 1e-4) or at the centre (Bernstein: 1e-10 .. all digits).
+//
+// A record of kHex27MomStride doubles per element: the moments, then from kHex27MomTab the coefficients
+// [axis][function, derivative][alpha][k].
 // ------------------------------------------------------------------------------------------------
-constexpr double kQuad1D[2][3][3] = {
-    {{0.0, -0.5, 0.5}, {1.0, 0.0, -1.0}, {0.0, 0.5, 0.5}},
-    {{0.125, -0.25, 0.125}, {0.75, 0.0, -0.25}, {0.125, 0.25, 0.125}},
-};
+static_assert(kHex27MomTab + 54 <= kHex27MomStride && kHex27MomTab >= kHex27Moments, "the tables follow the moments");
 
-// v[kind][tau][3 alpha + beta][m]: coefficients of F_alpha F_beta in the basis; tau = 2 [alpha differentiated] +
-// [beta differentiated]; kind 0 Lagrange, 1 B-spline; kind 2 the B-splines on a HEX8 cell (their linear
-// interpolant: l_0 / 2, 1 / 2, l_1 / 2 with l_0 = (1 - x) / 2, l_1 = (1 + x) / 2) in the basis {l_0^2, l_0 l_1, l_1^2, -, -}.
-struct AxisTables {
-    double v[3][4][9][5];
-    constexpr AxisTables() : v{} {
-        for (int kind = 0; kind < 2; ++kind)
-            for (int tau = 0; tau < 4; ++tau)
-                for (int al = 0; al < 3; ++al)
-                    for (int be = 0; be < 3; ++be) {
-                        double p[3] = {}, q[3] = {}, r[5] = {};
-                        for (int n = 0; n < 3; ++n) {
-                            if (tau & 2) { if (n > 0) p[n - 1] = n * kQuad1D[kind][al][n]; }
-                            else p[n] = kQuad1D[kind][al][n];
-                            if (tau & 1) { if (n > 0) q[n - 1] = n * kQuad1D[kind][be][n]; }
-                            else q[n] = kQuad1D[kind][be][n];
-                        }
-                        for (int a = 0; a < 3; ++a)
-                            for (int b = 0; b < 3; ++b) r[a + b] += p[a] * q[b];
-                        double* o = v[kind][tau][3 * al + be];
-                        o[0] = r[0] - r[1] + r[2] - r[3] + r[4];
-                        o[1] = r[0];
-                        o[2] = r[0] + r[1] + r[2] + r[3] + r[4];
-                        o[3] = r[3];
-                        o[4] = r[4];
-                    }
-        for (int tau = 0; tau < 4; ++tau)
-            for (int al = 0; al < 3; ++al)
-                for (int be = 0; be < 3; ++be) {
-                    // coefficients in {l_0, l_1}: of the value, or of the (constant) derivative
-                    const double lin[3][2] = {{0.5, 0.0}, {0.5, 0.5}, {0.0, 0.5}}, der[3] = {-0.25, 0.0, 0.25};
-                    const double p[2] = {tau & 2 ? der[al] : lin[al][0], tau & 2 ? der[al] : lin[al][1]};
-                    const double q[2] = {tau & 1 ? der[be] : lin[be][0], tau & 1 ? der[be] : lin[be][1]};
-                    double* o = v[2][tau][3 * al + be];
-                    o[0] = p[0] * q[0];
-                    o[1] = p[0] * q[1] + p[1] * q[0];
-                    o[2] = p[1] * q[1];
-                }
+// Coefficient k of 1D function alpha (0 .. 2) or its derivative on [lo, hi].  Every function is p q + c with
+// linear p, q, its coefficients p q, p q' + p' q, p' q' of their values at the ends; with u = (1 + x) / 2,
+// v = (1 - x) / 2: Lagrange -v x, 4 u v, u x; uniform quadratic B-splines (the T rows, vertex rows 1/2 1/2, mid
+// rows 1/8 3/4 1/8, times those) v v / 2, 1/2 + u v, u u / 2.
+__device__ __forceinline__ double axis_coefficient(bool spline, bool deriv, int alpha, int k, double lo, double hi) {
+    double p[2], q[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+        const double x = n ? hi : lo, u = 0.5 * (1.0 + x), v = 0.5 * (1.0 - x);
+        if (deriv) {
+            p[n] = spline ? (alpha == 0 ? -0.5 * v : (alpha == 1 ? -0.5 * x : 0.5 * u))
+                          : (alpha == 0 ? x - 0.5 : (alpha == 1 ? -2.0 * x : x + 0.5));
+            q[n] = 1.0;
+        } else {
+            p[n] = spline ? (alpha == 0 ? 0.5 * v : (alpha == 1 ? u : 0.5 * u))
+                          : (alpha == 0 ? -v : (alpha == 1 ? 4.0 * u : u));
+            q[n] = spline ? (alpha == 2 ? u : v) : (alpha == 1 ? v : x);
+        }
     }
-};
-__constant__ const AxisTables kAxis{};
-// integrals of the basis over [-1, 1]
-__constant__ const double kBasisInt[5] = {1.0 / 3.0, 4.0 / 3.0, 1.0 / 3.0, 0.0, -4.0 / 15.0};
+    const double c = spline && !deriv && alpha == 1 ? 0.5 : 0.0;
+    return k == 0 ? p[0] * q[0] + c : (k == 2 ? p[1] * q[1] + c : p[0] * q[1] + p[1] * q[0] + 2.0 * c);
+}
+__device__ __forceinline__ void write_tables(bool spline, const double* lo, const double* hi, double* tab) {
+    const int t = threadIdx.x;
+    if (t >= 54) return;
+    const int d = t / 18, r = t - 18 * d;
+    tab[t] = axis_coefficient(spline, r >= 9, (r % 9) / 3, r % 3, d == 0 ? lo[0] : (d == 1 ? lo[1] : lo[2]),
+                              d == 0 ? hi[0] : (d == 1 ? hi[1] : hi[2]));
+}
 
 // ------------------------------------------------------------------------------------------------
-// k_hex27_moments: mom[e][(i 5 + j) 5 + k] = sum_ip w* g_i(x) g_j(y) g_k(z), g the basis above.  Two wavefronts
-// per element, each with 13 or 12 of the 25 pairs (i, j) as 65 or 60 sums per lane in registers; 64 points
-// at a time, a lane a point.  A batch of 64 sub-tets is staged in LDS as vertex 2, the three edges and
-// the volume factor.  The lanes' sums are added pairwise by half and quarter wavefront (gfx950's lane
-// swaps reduce two registers at once), the last 16 in LDS.
-// Bound by FP64 arithmetic, 111 operations a point and wavefront: 32^3 cut cells (37.8M points) 0.47 ms; a
+// k_hex27_moments: mom[e][(i 5 + j) 5 + k] = sum_ip w* g_i(x) g_j(y) g_k(z), and the element's tables.  Two
+// wavefronts per element, each with 13 or 12 of the 25 pairs (i, j) as 65 or 60 sums per lane in registers;
+// 64 points at a time, a lane a point.  A batch of 64 sub-tets is staged in LDS as vertex 2, the three
+// edges and the volume factor.  The lanes' sums are added pairwise by half and quarter wavefront
+// (gfx950's lane swaps reduce two registers at once), the last 16 in LDS.
+// Bound by FP64 arithmetic, 112 operations a point and wavefront: 32^3 cut cells (37.8M points) 0.50 ms
+// (0.56 with two wavefronts a SIMD instead of three, the weight read under a branch); a
 // 16 x 16 x 4 FP64 MFMA tile per 4 points took 0.69 ms: its operands pass through LDS (25 doubles a point),
 // half the tile is padding, and FP64 MFMA runs at the rate of the vector unit.
 // ------------------------------------------------------------------------------------------------
-__device__ __forceinline__ void hex27_basis(double x, double* v) {
-    const double x2 = x * x;
-    v[0] = 0.5 * (x2 - x);
-    v[1] = 1.0 - x2;
-    v[2] = 0.5 * (x2 + x);
-    v[3] = -x * v[1];
-    v[4] = x * v[3];
+__device__ __forceinline__ void hex27_basis(double t, double* v) {
+    const double s = 1.0 - t, t2 = t * t, ts = t * s, s2 = s * s;
+    v[0] = s2 * s2;
+    v[1] = ts * s2;
+    v[2] = ts * ts;
+    v[3] = ts * t2;
+    v[4] = t2 * t2;
 }
 
 constexpr int kMomBatch = 64;                          // sub-tets staged at a time
@@ -115,8 +106,89 @@ constexpr int kMomRule = kMomBatch * kMomTet;          // LDS offset of TET_35 [
 constexpr int kMomLds = 17 * 68;                       // the reduction's space
 static_assert(kMomRule + 4 * kTet35Points <= kMomLds, "staged sub-tets and the rule fit the reduction's space");
 
+// min over the lanes of equal lane % 8
+__device__ __forceinline__ double min_mod8(double v) {
+    auto both = [](double x, auto f) {
+        const uint64_t u = __double_as_longlong(x);
+        uint32_t r[4];
+        f((uint32_t)u, r[0], r[2]);
+        f((uint32_t)(u >> 32), r[1], r[3]);
+        return fmin(__longlong_as_double(((uint64_t)r[1] << 32) | r[0]), __longlong_as_double(((uint64_t)r[3] << 32) | r[2]));
+    };
+    v = both(v, [](uint32_t w, uint32_t& x, uint32_t& y) {
+        x = w;
+        y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x128, 0xf, 0xf, true);   // lane + 8 within 16
+    });
+    v = both(v, [](uint32_t w, uint32_t& x, uint32_t& y) {
+        const auto s = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+        x = s[0];
+        y = s[1];
+    });
+    return both(v, [](uint32_t w, uint32_t& x, uint32_t& y) {
+        const auto s = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+        x = s[0];
+        y = s[1];
+    });
+}
+__device__ __forceinline__ double read_lane(double v, int lane) {
+    const uint64_t u = __double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)u, lane), hi = __builtin_amdgcn_readlane((uint32_t)(u >> 32), lane);
+    return __longlong_as_double(((uint64_t)hi << 32) | lo);
+}
+
+__device__ __forceinline__ void load_tet(const GenView& g, int tet, double* X) {
+    const double2* X2 = reinterpret_cast<const double2*>(g.ig_xi + (size_t)tet * 12);
+#pragma unroll
+    for (int n = 0; n < 6; ++n) {
+        const double2 v = X2[n];
+        X[2 * n] = v.x;
+        X[2 * n + 1] = v.y;
+    }
+}
+
+// The box of the sub-tets' vertices and the factors to [0, 1] (0 for an axis without extent: t = 0, the
+// functions' values at lo), the same in every lane.  X: the lane's sub-tet of the first batch.
+__device__ __forceinline__ void hex27_box(const GenView& g, int ig0, int nsub, const double* X, double* lds, double* lo,
+                                          double* hi, double* sc) {
+    const int lane = threadIdx.x;
+    double b[6];   // the least of x, y, z and of -x, -y, -z
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        b[d] = fmin(fmin(X[d], X[3 + d]), fmin(X[6 + d], X[9 + d]));
+        b[3 + d] = fmin(fmin(-X[d], -X[3 + d]), fmin(-X[6 + d], -X[9 + d]));
+    }
+    for (int t = kMomBatch + lane; t < nsub; t += 64) {
+        double Y[12];
+        load_tet(g, ig0 + t, Y);
+#pragma unroll
+        for (int n = 0; n < 12; ++n) {
+            b[n % 3] = fmin(b[n % 3], Y[n]);
+            b[3 + n % 3] = fmin(b[3 + n % 3], -Y[n]);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < 6; ++d) lds[d * 65 + lane] = b[d];
+    __syncthreads();
+    const double* col = lds + min(lane & 7, 5) * 65 + (lane >> 3) * 8;
+    double v = col[0];
+#pragma unroll
+    for (int n = 1; n < 8; ++n) v = fmin(v, col[n]);
+    v = min_mod8(v);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        lo[d] = read_lane(v, d);
+        hi[d] = -read_lane(v, 3 + d);
+    }
+    const double ext = lane == 0 ? hi[0] - lo[0] : (lane == 1 ? hi[1] - lo[1] : hi[2] - lo[2]);
+    const double inv = ext > 1e-290 ? 1.0 / ext : 0.0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) sc[d] = read_lane(inv, d);
+    __syncthreads();   // the space is free again
+}
+
 template <int ROLE>
-__device__ __forceinline__ void hex27_cut_moments(const GenView& g, int ig0, int nsub, double vol6, double* lds, double* out) {
+__device__ __forceinline__ void hex27_cut_moments(const GenView& g, int ig0, int nsub, double vol6, const double* lo,
+                                                  const double* sc, double* lds, double* out) {
     constexpr int P0 = ROLE == 0 ? 0 : 13, NP = ROLE == 0 ? 13 : 12, I0 = P0 / 5;
     const int lane = threadIdx.x;
     double acc[NP][5];
@@ -130,17 +202,13 @@ __device__ __forceinline__ void hex27_cut_moments(const GenView& g, int ig0, int
     }
     for (int t0 = 0; t0 < nsub; t0 += kMomBatch) {
         const int nt = min(kMomBatch, nsub - t0), npts = nt * kTet35Points;
-        if (t0 > 0) __syncthreads();   // the previous batch is read
-        if (lane < nt) {
-            const double2* X2 = reinterpret_cast<const double2*>(g.ig_xi + (size_t)(ig0 + t0 + lane) * 12);
-            double X[12];
-#pragma unroll
-            for (int n = 0; n < 6; ++n) {
-                const double2 v = X2[n];
-                X[2 * n] = v.x;
-                X[2 * n + 1] = v.y;
+        if (t0 > 0) {   // (the first batch is staged)
+            __syncthreads();   // the previous batch is read
+            if (lane < nt) {
+                double X[12];
+                load_tet(g, ig0 + t0 + lane, X);
+                stage_simplex<3>(X, lo, sc, vol6, lds + lane * kMomTet);
             }
-            stage_simplex<3, false>(X, vol6, lds + lane * kMomTet);
         }
         __syncthreads();
         for (int p0 = 0; p0 < npts; p0 += 64) {
@@ -154,7 +222,7 @@ __device__ __forceinline__ void hex27_cut_moments(const GenView& g, int ig0, int
             double x[3];
 #pragma unroll
             for (int d = 0; d < 3; ++d) x[d] = T[4 * d] + b[0] * T[4 * d + 1] + b[1] * T[4 * d + 2] + b[2] * T[4 * d + 3];
-            const double w = ip < npts ? b[3] * T[12] : 0.0;
+            const double wt = b[3] * T[12], w = ip < npts ? wt : 0.0;
             double gx[5], gy[5], gz[5];
             hex27_basis(x[0], gx);
             hex27_basis(x[1], gy);
@@ -180,36 +248,73 @@ __device__ __forceinline__ void hex27_cut_moments(const GenView& g, int ig0, int
     }
 }
 
-__global__ __launch_bounds__(64) void k_hex27_moments(GenView g, double* mom) {
+__global__ __launch_bounds__(64, 3) void k_hex27_moments(GenView g, double* mom) {
     __shared__ __align__(16) double lds[kMomLds];
     // 16 blocks in a row hold 8 elements, the role changing after 8: the round robin over the 8 XCDs
     // gives each both roles in turn
     const int b = blockIdx.x, role = (b >> 3) & 1, be = (b >> 4) * 8 + (b & 7);
     if (be >= g.n_el) return;
-    const int e = g.order ? g.order[be] : be;
+    const int e = __builtin_amdgcn_readfirstlane(g.order ? g.order[be] : be);
     double hh[3];
     for (int d = 0; d < 3; ++d) hh[d] = g.ip_box[(size_t)e * 6 + 3 + d];
     const double detJ = (0.5 * hh[0]) * (0.5 * hh[1]) * (0.5 * hh[2]);
-    const int ig0 = g.ig_ptr[e], nsub = g.ig_ptr[e + 1] - ig0;
-    double* out = mom + (size_t)e * kHex27Moments;
+    const double vol6 = read_lane(detJ / 6.0, 0);   // (in scalar registers)
+    const int ig0 = __builtin_amdgcn_readfirstlane(g.ig_ptr[e]), nsub = __builtin_amdgcn_readfirstlane(g.ig_ptr[e + 1]) - ig0;
+    double* out = mom + (size_t)e * kHex27MomStride;
+    double lo[3] = {-1.0, -1.0, -1.0}, hi[3] = {1.0, 1.0, 1.0}, sc[3];
+    if (nsub > 0) {
+        double X[12];
+        load_tet(g, ig0 + min((int)threadIdx.x, nsub - 1), X);   // (lanes past the end: the last one again)
+        hex27_box(g, ig0, nsub, X, lds, lo, hi, sc);
+        if ((int)threadIdx.x < nsub) stage_simplex<3>(X, lo, sc, vol6, lds + threadIdx.x * kMomTet);
+    }
+    if (role == 0) write_tables(g.t_perm[(size_t)e * kHex27PermStride + 27] == 2, lo, hi, out + kHex27MomTab);
     if (nsub == 0) {
-        // whole cell: products of 1D integrals (HEX_3x3x3 integrates the basis exactly)
+        // whole cell: products of the 1D integrals 2/5, 1/10, 1/15, 1/10, 2/5 (HEX_3x3x3 is exact for them)
+        auto n30 = [](int m) { return m == 2 ? 2 : (m == 0 || m == 4 ? 12 : 3); };
         for (int t = threadIdx.x; t < kHex27Moments && role == 0; t += 64)
-            out[t] = detJ * (kBasisInt[t / 25] * kBasisInt[(t / 5) % 5] * kBasisInt[t % 5]);
+            out[t] = detJ * ((double)(n30(t / 25) * n30((t / 5) % 5) * n30(t % 5)) / 27000.0);
     } else if (role == 0) {
-        hex27_cut_moments<0>(g, ig0, nsub, detJ / 6.0, lds, out);
+        hex27_cut_moments<0>(g, ig0, nsub, vol6, lo, sc, lds, out);
     } else {
-        hex27_cut_moments<1>(g, ig0, nsub, detJ / 6.0, lds, out);
+        hex27_cut_moments<1>(g, ig0, nsub, vol6, lo, sc, lds, out);
     }
 }
 
 // ------------------------------------------------------------------------------------------------
 // M from the moments, by sum factorisation over the axes: block p = (i, j), i <= j, of
 //   M[(i,a),(j,b)] = s_i s_j sum_{x,y,z <= 4} mom_xyz P_0(a_0,b_0; x) P_1(a_1,b_1; y) P_2(a_2,b_2; z),
-// s_i = 2 / h_i, contracted over z, y, x.  Wavefronts take whole tasks, so that the 1D tables are
-// scalar loads.  Result G[p][a][b] in LDS, a = (a_0 3 + a_1) 3 + a_2; NF == 1: the sum of the three
-// diagonal blocks only.  LDS: mom, Z[zt][x 5 + y][ab_2], Y[block][x][ab_1][ab_2], then G over Z and Y.
+// s_i = 2 / h_i, P_d(alpha,beta; m) = sum_(k + l = m) f_alpha,k f_beta,l of the element's tables, contracted over z,
+// y, x.  Wavefronts take whole tasks, so that the tables are scalar loads.  Result G[p][a][b] in LDS,
+// a = (a_0 3 + a_1) 3 + a_2; NF == 1: the sum of the three diagonal blocks only.  The diagonal blocks are
+// symmetric bit for bit.  LDS: mom, Z[zt][x 5 + y][ab_2], Y[block][x][ab_1][ab_2], then G over Z and Y.
 // ------------------------------------------------------------------------------------------------
+typedef const __attribute__((address_space(4))) double* scalar_table;   // memory that this kernel only reads
+
+// o[3 alpha + beta] = sum_kl A[alpha][k] B[beta][l] T[k + l], A == B where SYM
+template <bool SYM>
+__device__ __forceinline__ void axis_contract(const double* T, scalar_table A, scalar_table B, double* o) {
+#pragma unroll
+    for (int al = 0; al < 3; ++al) {
+        double v[3];
+#pragma unroll
+        for (int l = 0; l < 3; ++l) v[l] = A[3 * al] * T[l] + A[3 * al + 1] * T[l + 1] + A[3 * al + 2] * T[l + 2];
+#pragma unroll
+        for (int be = 0; be < 3; ++be) {
+            if (SYM && be < al) continue;
+            const double w = v[0] * B[3 * be] + v[1] * B[3 * be + 1] + v[2] * B[3 * be + 2];
+            o[3 * al + be] = w;
+            if (SYM) o[3 * be + al] = w;
+        }
+    }
+}
+// tau = 2 [alpha differentiated] + [beta differentiated] (the same for the wavefront); tab: the axis' tables
+__device__ __forceinline__ void axis_contract(const double* T, scalar_table tab, int tau, double* o) {
+    scalar_table A = tab + (tau & 2 ? 9 : 0), B = tab + (tau & 1 ? 9 : 0);
+    if (tau == 0 || tau == 3) axis_contract<true>(T, A, A, o);
+    else axis_contract<false>(T, A, B, o);
+}
+
 template <int NF> struct Hex27Blocks;
 template <> struct Hex27Blocks<1> {
     static constexpr int n = 3;
@@ -227,49 +332,47 @@ constexpr int sf_lds() {   // doubles
 static_assert(kSfY + 6 * 405 <= 6 * 729, "the contraction stages fit the space of G");
 
 template <int NF>
-__device__ __forceinline__ void sf_moments(const GenView& g, const double* mom, int e, int kind, double* lds) {
+__device__ __forceinline__ void sf_moments(const GenView& g, const double* mom, int e, double* lds) {
     using B = Hex27Blocks<NF>;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     double* Z = lds + kSfZ;
     double* Y = lds + kSfY;
-    if (tid < kHex27Moments) lds[tid] = mom[(size_t)e * kHex27Moments + tid];
+    const double* rec = mom + (size_t)__builtin_amdgcn_readfirstlane(e) * kHex27MomStride;
+    const scalar_table tab = (scalar_table)(rec + kHex27MomTab);
+    if (tid < kHex27Moments) lds[tid] = rec[tid];
+    // the tables' lines are requested here: a stage that asked for its own would wait for memory each time
+    double line[7];
+#pragma unroll
+    for (int n = 0; n < 7; ++n) line[n] = tab[8 * n < 54 ? 8 * n : 53];
     double sc[3];
     for (int d = 0; d < 3; ++d) sc[d] = 2.0 / g.ip_box[(size_t)e * 6 + 3 + d];
     __syncthreads();
+#pragma unroll
+    for (int n = 0; n < 7; ++n) asm volatile("" ::"s"(line[n]));   // (used here: not dropped, not moved down)
     // z: task zt = wave, tau_2 = 0, 1, 3 (alpha alone is differentiated on axis 2 in no block i <= j)
     if (wave < 3 && lane < 25) {
-        const double(*P)[5] = kAxis.v[kind][wave == 2 ? 3 : wave];
-        double m[5];
+        double m[5], o[9];
 #pragma unroll
         for (int k = 0; k < 5; ++k) m[k] = lds[lane * 5 + k];
+        axis_contract(m, tab + 36, wave == 2 ? 3 : wave, o);
 #pragma unroll
-        for (int ab = 0; ab < 9; ++ab) {
-            double v = 0.0;
-#pragma unroll
-            for (int k = 0; k < 5; ++k) v += m[k] * P[ab][k];
-            Z[wave * 225 + lane * 9 + ab] = v;
-        }
+        for (int ab = 0; ab < 9; ++ab) Z[wave * 225 + lane * 9 + ab] = o[ab];
     }
     __syncthreads();
     // y: task block p, lane (x, ab_2)
     for (int p = wave; p < B::n; p += 4) {
         const int i = NF == 1 ? p : (p >= 3) + (p >= 5), j = NF == 1 ? p : (p < 3 ? p : (p < 5 ? p - 2 : 2));
         const int tau1 = 2 * (i == 1) + (j == 1), tau2 = 2 * (i == 2) + (j == 2);
-        const double(*P)[5] = kAxis.v[kind][tau1];
         if (lane < 45) {
             const int x = lane / 9, ab2 = lane - 9 * x;
             const double* Zp = Z + (tau2 == 3 ? 2 : tau2) * 225 + x * 45 + ab2;
-            double z[5];
+            double z[5], o[9];
 #pragma unroll
             for (int y = 0; y < 5; ++y) z[y] = Zp[9 * y];
+            axis_contract(z, tab + 18, tau1, o);
 #pragma unroll
-            for (int ab1 = 0; ab1 < 9; ++ab1) {
-                double v = 0.0;
-#pragma unroll
-                for (int y = 0; y < 5; ++y) v += z[y] * P[ab1][y];
-                Y[p * 405 + x * 81 + ab1 * 9 + ab2] = v;
-            }
+            for (int ab1 = 0; ab1 < 9; ++ab1) Y[p * 405 + x * 81 + ab1 * 9 + ab2] = o[ab1];
         }
     }
     __syncthreads();
@@ -288,16 +391,13 @@ __device__ __forceinline__ void sf_moments(const GenView& g, const double* mom, 
         for (int pp = 0; pp < (NF == 3 ? 1 : 3); ++pp) {
             const int p = NF == 3 ? task >> 1 : pp;
             const int i = NF == 1 ? p : (p >= 3) + (p >= 5), j = NF == 1 ? p : (p < 3 ? p : (p < 5 ? p - 2 : 2));
-            const int tau0 = 2 * (i == 0) + (j == 0);
-            const double(*P)[5] = kAxis.v[kind][tau0];
             const double s2 = (i == 0 ? sc[0] : (i == 1 ? sc[1] : sc[2])) * (j == 0 ? sc[0] : (j == 1 ? sc[1] : sc[2]));
-            double y[5];
+            double y[5], o[9];
 #pragma unroll
             for (int x = 0; x < 5; ++x) y[x] = s2 * Y[p * 405 + x * 81 + ab12];
+            axis_contract(y, tab, 2 * (i == 0) + (j == 0), o);
 #pragma unroll
-            for (int ab0 = 0; ab0 < 9; ++ab0)
-#pragma unroll
-                for (int x = 0; x < 5; ++x) r[n][ab0] += y[x] * P[ab0][x];
+            for (int ab0 = 0; ab0 < 9; ++ab0) r[n][ab0] += o[ab0];
         }
     }
     __syncthreads();
@@ -375,8 +475,8 @@ __device__ __forceinline__ void hex27_material(const GenView& g, int e, double& 
 // k_hex27_tensor: K_e of elements whose T is a tensor product (t_perm[e][27] = 1 nodal, 2 B-spline, 3 B-spline on
 // a HEX8 cell; t_perm[e][y] the tensor index of the element's adof y).  Threads 0 .. 3 NA - 1 hold a column of K_e and
 // write NF rows' worth of consecutive values per step (stores of whole lines).  Without the products by T
-// and their LDS space four blocks instead of two fit a CU: 0.44 ms for 32^3 elements of 81 x 81 (1.7 GB
-// written, 3.9 TB/s), against 1.7 ms on the general path.
+// and their LDS space four blocks instead of two fit a CU: 0.48 ms for 32^3 elements of 81 x 81 (1.7 GB
+// written, 3.5 TB/s), against 1.7 ms on the general path.
 // ------------------------------------------------------------------------------------------------
 template <int NF, bool SCATTER>
 __global__ __launch_bounds__(256) void k_hex27_tensor(GenView g, const int32_t* els, const double* mom, double* vals) {
@@ -389,7 +489,7 @@ __global__ __launch_bounds__(256) void k_hex27_tensor(GenView g, const int32_t* 
     const int tid = threadIdx.x;
     const uint8_t* pm = g.t_perm + (size_t)e * kHex27PermStride;
     if (tid < 27) perm[tid] = pm[tid];
-    sf_moments<NF>(g, mom, e, __builtin_amdgcn_readfirstlane((int)pm[27]) - 1, lds);
+    sf_moments<NF>(g, mom, e, lds);
     double c0, c1, cs;
     hex27_material<NF>(g, e, c0, c1, cs);
     if (tid >= RPS * NA) return;
@@ -446,7 +546,7 @@ __global__ __launch_bounds__(256) void k_hex27_general(GenView g, const int32_t*
     __syncthreads();
     if (tid < NB)
         for (int q = g.t_ptr[e * NB + tid]; q < g.t_ptr[e * NB + tid + 1]; ++q) Tt[tid * na_t + g.t_col[q]] += g.t_w[q];
-    sf_moments<NF>(g, mom, e, 0, lds);
+    sf_moments<NF>(g, mom, e, lds);
     double c0, c1, cs;
     hex27_material<NF>(g, e, c0, c1, cs);
     // HEX27 basis of row / column operand n of a tile -> its tensor index in G

@@ -18,6 +18,8 @@ constexpr int kGenericMaxAdofsPerType = 64;
 // truncated hierarchical rows up to about 40.
 constexpr int kHex27MaxAdofsPerType = 64;
 constexpr int kHex27Moments = 125;      // moments of degree <= 4 per axis of an element
+constexpr int kHex27MomTab = 126;       // and from here the coefficients of its 1D functions (hex27.hip)
+constexpr int kHex27MomStride = 180;    // doubles of an element's record
 constexpr int kHex27PermStride = 28;    // SetHost::t_perm entries of an element
 // HEX27 sets whose element matrices hold more entries than this (a K_e pool of 8 GiB) take the
 // scatter mode, which keeps no pool but is slower: 40^3 elements of 81 x 81 (3.4 GiB), elasticity:

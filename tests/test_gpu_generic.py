@@ -370,3 +370,116 @@ def test_rows_mode_sums_in_element_order(case, monkeypatch):
     v1, R1 = S.compute_jacobian_and_residual(u)
     v2, R2 = S_lists.compute_jacobian_and_residual(u)
     assert np.array_equal(v1.view(np.uint64), v2.view(np.uint64)) and rel(R1, R2) <= 1e-14
+
+
+# HEX27 node order: half steps along each axis (corners, edges, centre, faces)
+HEX27_HALF = ("000 200 220 020 002 202 222 022 100 210 120 010 001 201 221 021 102 212 122 012 "
+              "111 110 112 011 211 101 121")
+
+
+def _slivers():
+    """Sub-tets of [-1, 1]^3 that leave a basis function almost untouched: at corners, along edges and
+    faces, around the cell's centre, and inside, of extent d."""
+    def tet(p, e):
+        X = np.array([p, p, p, p], float)
+        X[0, 0] += e[0]
+        X[1, 1] += e[1]
+        X[3, 2] += e[2]
+        return X if e[0] * e[1] * e[2] > 0 else X[[1, 0, 2, 3]]
+    out = []
+    for d in (1e-1, 1e-3, 1e-5):
+        out += [("corner", d, [tet((-1, -1, -1), (d, d, d))]), ("corner", d, [tet((1, 1, -1), (-d, -d, d))]),
+                ("edge", d, [tet((-1, 1, -1), (d, -d, 2))]), ("face", d, [tet((-1, -1, 1), (2, 2, -d))]),
+                ("centre", d, [tet((0, 0, 0), (a * d, b * d, c * d)) for a in (1, -1) for b in (1, -1) for c in (1, -1)]),
+                ("axis", d, [tet((0, 0, -1), (d, d, 2))]), ("mid slab", d, [tet((0, -1, -1), (d, 2, 2))]),
+                ("inside", d, [tet((0.5, 0.5, 0.5), (d, d, d))])]
+    return out
+
+
+@pytest.mark.parametrize("iwg", [M.IWG_SPATIALDIFF_BULK, M.IWG_STRUC_LINEAR_BULK])
+@pytest.mark.parametrize("order", [1, 2])
+def test_hex27_small_diagonal_entries_on_slivers(order, iwg):
+    """Every diagonal entry of a HEX27 element matrix to its own relative error, however small the
+    entry: a diagonal is a sum of w |grad N|^2 over the TET_35 points, all terms of one sign, so the
+    error of a correct sum is that of grad N.  The coordinates' rounding, 1e-16 of the cell, is 1e-16 / d of a
+    distance d to a corner where grad N vanishes with d^2 (nodal rows) or N and grad N with d^6 (B-spline
+    rows, squared): 12 x 1e-16 / d; 200 points' roundings add 1e-14.  Each sliver is an element of its
+    own, without shared adofs, against sums in extended precision."""
+    spec, keep = M.make_spec(3, (3, 3, 3), iwg=iwg, bspline_order=order, lagrange_order=2)
+    P = M.Problem(spec, keep)
+    a = P.arrays()
+    nf = 3 if iwg == M.IWG_STRUC_LINEAR_BULK else 1
+    cases = _slivers()
+    # the T rows and box of the middle element, adofs of its own for every sliver, in a random order
+    e0 = 13
+    tp = a["t_ptr"].astype(np.int64)
+    r0, r1 = tp[27 * e0], tp[27 * e0 + 27]
+    ids = np.unique(a["t_adof"][r0:r1])
+    rng = np.random.default_rng(SEED + 53)
+    n = len(cases)
+    order_of = [rng.permutation(27) for _ in range(n)]
+    col = np.searchsorted(ids, a["t_adof"][r0:r1])
+    ig = [np.array(c[2]).reshape(-1) for c in cases]
+    nm = 2 if nf == 3 else 1
+    box = a["ip_box"].reshape(-1, 6)[e0]
+    arrays = {"t_ptr": np.concatenate([[0]] + [tp[27 * e0 + 1:27 * e0 + 28] - r0 + i * (r1 - r0) for i in range(n)]),
+              "t_adof": np.concatenate([27 * i + order_of[i][col] for i in range(n)]),
+              "t_weight": np.tile(a["t_weight"][r0:r1], n),
+              "ig_ptr": np.concatenate([[0], np.cumsum([len(c[2]) for c in cases])]), "ig_xi": np.concatenate(ig),
+              "material": np.tile(a["material"].reshape(-1, nm)[e0], n), "ip_box": np.tile(box, n),
+              "elem_cell": np.zeros(n, np.int32), "vertex_phi": np.zeros(0)}
+    d, keep_arrays = M.desc_from_arrays(P.desc, arrays)
+    d.n_elements = n
+    d.n_adofs_per_type = 27 * n
+    d.elem_cell = None
+    d.lattice = M.Lattice()
+    S = M.Set(d, keepalive=(P, keep_arrays))
+    rp, ci = S.pattern()
+    vals, _ = S.compute_jacobian_and_residual(np.zeros(S.n_rows))
+    import scipy.sparse as sp
+    diag = sp.csr_matrix((vals, ci, rp), shape=(S.n_rows, S.n_rows)).diagonal()
+    # reference: the rows' functions at the points, in extended precision
+    ld = np.longdouble
+    xi, w = (v.astype(ld) for v in O.rule("TET_35"))
+    bary = np.stack([xi[:, 0], xi[:, 1], 1 - xi[:, 0] - xi[:, 1] - xi[:, 2], xi[:, 2]], 1)
+    h = box[3:].astype(ld)
+    # 1D functions of an adof per axis: Lagrange, or uniform quadratic B-splines; which, from T
+    T = np.zeros((27, 27))
+    for b in range(27):
+        for q in range(tp[27 * e0 + b], tp[27 * e0 + b + 1]):
+            T[b, col[q - r0]] += a["t_weight"][q]
+    half = np.array([[int(c) for c in t] for t in HEX27_HALF.split()])
+    T1 = np.array([[0.5, 0.5, 0], [0.125, 0.75, 0.125], [0, 0.5, 0.5]]) if order == 2 else np.eye(3)
+    tensor = {tuple(T1[half[:, 0], i] * T1[half[:, 1], j] * T1[half[:, 2], k]): (i, j, k)
+              for i in range(3) for j in range(3) for k in range(3)}
+    worst = {}
+    for i, (kind, size, tets) in enumerate(cases):
+        X = np.array(tets).astype(ld)
+        x = np.einsum("qv,tvd->tqd", bary, X).reshape(-1, 3)
+        J = np.stack([(X[:, r] - X[:, 2]) * (h / 2) for r in (0, 1, 3)], 1)
+        det = (J[:, 0, 0] * (J[:, 1, 1] * J[:, 2, 2] - J[:, 2, 1] * J[:, 1, 2]) -
+               J[:, 0, 1] * (J[:, 1, 0] * J[:, 2, 2] - J[:, 1, 2] * J[:, 2, 0]) +
+               J[:, 0, 2] * (J[:, 1, 0] * J[:, 2, 1] - J[:, 1, 1] * J[:, 2, 0])) / 6
+        ws = (det[:, None] * w[None]).reshape(-1)
+        u, v = (1 + x) / 2, (1 - x) / 2
+        if order == 2:
+            f, df = [v * v / 2, (1 + 2 * u * v) / 2, u * u / 2], [-v / 2, -x / 2, u / 2]
+        else:
+            f, df = [-x * v, 4 * u * v, x * u], [x - ld(0.5), -2 * x, x + ld(0.5)]
+        for c in range(27):
+            t = tensor[tuple(T[:, c])]
+            g2 = [ws @ (np.prod([(df if k == ax else f)[t[k]][:, k] for k in range(3)], axis=0) * 2 / h[ax]) ** 2
+                  for ax in range(3)]
+            for fld in range(nf):
+                if nf == 1:
+                    want = ld(arrays["material"][0]) * sum(g2)
+                else:
+                    E, nu = (ld(m) for m in arrays["material"][:2])
+                    lam, mu = E * nu / ((1 + nu) * (1 - 2 * nu)), E / (2 * (1 + nu))
+                    want = lam * g2[fld] + mu * (sum(g2) + g2[fld])
+                got = diag[fld * 27 * n + 27 * i + order_of[i][c]]
+                err = float(abs(got - want) / want)
+                worst[kind, size] = max(worst.get((kind, size), 0.0), err)
+    for k, e in sorted(worst.items()):
+        print(k, "%.1e" % e, flush=True)
+    assert all(e <= 1e-14 + 12e-16 / k[1] for k, e in worst.items()), worst
