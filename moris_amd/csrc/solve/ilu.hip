@@ -52,8 +52,13 @@ namespace ilu {
 
 constexpr int kMaxRow = 5000;   // longest factor row the numeric kernel keeps in LDS (60 KB)
 constexpr size_t kMaxUpdates = (size_t)1 << 25;   // elimination lists up to 256 MiB; beyond, the rows are searched
-// A step of k_ilu_tri and a level launched on its own, in microseconds: 8825 rows, 1264 steps for 400
-// levels 0.217 ms, 400 launches 1.4 ms.
+// Stream of k_ilu_tri (24 bytes a slot) up to 512 MiB; beyond, a launch per level.  A level takes a step's 512
+// slots however few rows it has: 16383 rows of one level each 0.40 GB (5.6 ms a solve against 80 launched),
+// rows of 1000 entries each side would take 6.4 GB beside 0.4 GB of factor.
+constexpr size_t kMaxTriBytes = (size_t)1 << 29;
+// A step of k_ilu_tri and a level launched on its own, in microseconds: 0.17 .. 0.21 (8825, 8000 and 15625 rows,
+// 1264, 672 and 1184 steps: 0.22, 0.15 and 0.26 ms a call) and 3.2 .. 3.5 (8825 rows, 400 levels: 1.4 ms; 216k
+// and 729k rows, 828 and 1248 levels: 2.6 and 4.1 ms).
 constexpr double kTriStepUs = 0.17, kLevelUs = 3.5;
 
 __global__ void k_ilu_clear(int32_t* err) {
@@ -183,6 +188,8 @@ struct __align__(16) TriSlot {
     uint32_t dword;  // backward, last step of a row: lanes 0 and 1 of the row hold its diagonal's words
 };
 
+constexpr size_t kTriSlotBytes = sizeof(TriSlot) + 2 * sizeof(int32_t);   // with its factor and diagonal entry
+
 template <int L>
 __global__ __launch_bounds__(kTriThreads) void k_ilu_tri(int32_t n, int32_t n_fwd, int32_t n_bwd, const TriSlot* slots,
                                                          const double* src, double* dst, const int32_t* skip) {
@@ -293,45 +300,76 @@ mgpu_status dev_upload(mgpu_ilu* f, const std::vector<T>& h, T** d) {
     return MGPU_OK;
 }
 
-// The stream of one triangular solve with L lanes per row: the rows of each level (order: most entries
-// first), kTriThreads / L at a time; range: the entries of a row that the solve uses; diag: the rows' diagonals
-// (backward) or null.
+// The same for an array that the solve can do without: false, and no allocation kept, where it does not fit.
+template <class T>
+bool dev_upload_optional(mgpu_ilu* f, const std::vector<T>& h, T** d) {
+    *d = nullptr;
+    void* p = nullptr;
+    if (hipMalloc(&p, h.size() * sizeof(T)) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (hipMemcpy(p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(p);
+        return false;
+    }
+    f->allocs.push_back(p);
+    *d = static_cast<T*>(p);
+    return true;
+}
+template <class T>
+void dev_drop(mgpu_ilu* f, T** d) {
+    if (!*d) return;
+    f->allocs.erase(std::find(f->allocs.begin(), f->allocs.end(), static_cast<void*>(*d)));
+    (void)hipFree(*d);
+    *d = nullptr;
+}
+
+// One triangular solve as a stream with L lanes per row: the rows of each level (order: most entries first),
+// kTriThreads / L at a time; range: the entries of a row that the solve uses.
+template <class Range>
+int tri_chunks(int L, int32_t row, Range range) {
+    return std::max(1, (int)((range(row).second - range(row).first + L - 1) / L));
+}
+// its steps (whole multiples of kTriAhead, the last ones doing nothing)
+template <class Range>
+int64_t tri_steps(int L, const std::vector<int32_t>& order, const std::vector<int32_t>& off, Range range) {
+    int64_t steps = 0;
+    for (size_t l = 0; l + 1 < off.size(); ++l)
+        for (int32_t g = off[l]; g < off[l + 1]; g += kTriThreads / L) steps += tri_chunks(L, order[(size_t)g], range);
+    return (steps + kTriAhead - 1) / kTriAhead * kTriAhead;
+}
 struct TriStream {
     std::vector<TriSlot> slots;
     std::vector<int32_t> pos, dpos;
-    int64_t steps = 0;
 };
+// and its slots, from slot `at` of the stream on (all empty before); diag: the rows' diagonals (backward) or null
 template <class Range>
-void tri_stream(int L, int32_t n, const std::vector<int32_t>& order, const std::vector<int32_t>& off, Range range,
-                const std::vector<int32_t>& fci, const std::vector<int32_t>* diag, bool build, TriStream& out) {
+void tri_fill(int L, int32_t n, const std::vector<int32_t>& order, const std::vector<int32_t>& off, Range range,
+              const std::vector<int32_t>& fci, const std::vector<int32_t>* diag, size_t at, TriStream& out) {
     const int RPS = kTriThreads / L;
-    auto length = [&](int32_t i) { return range(i).second - range(i).first; };
-    auto slot = [&](int32_t p, int32_t dp, uint32_t meta) {
-        out.pos.push_back(p);
-        out.dpos.push_back(dp);
-        out.slots.push_back(TriSlot{0.0, meta, 0u});
-    };
     for (size_t l = 0; l + 1 < off.size(); ++l) {
         for (int32_t g = off[l]; g < off[l + 1]; g += RPS) {
             const int32_t g1 = std::min(g + RPS, off[l + 1]);
-            const int chunks = std::max(1, (int)((length(order[(size_t)g]) + L - 1) / L));
-            out.steps += chunks;
-            for (int c = 0; c < chunks && build; ++c) {
+            const int chunks = tri_chunks(L, order[(size_t)g], range);
+            for (int c = 0; c < chunks; ++c) {
                 const uint32_t flags = (c + 1 == chunks ? kTriRowEnd : 0u) |
                                        (c + 1 == chunks && g1 == off[l + 1] ? kTriLevelEnd : 0u);
                 for (int k = 0; k < RPS; ++k) {
                     const int32_t i = g + k < g1 ? order[(size_t)(g + k)] : n;
-                    for (int lane = 0; lane < L; ++lane) {
-                        const int32_t p = i < n && c * L + lane < length(i) ? range(i).first + c * L + lane : -1;
-                        const int32_t dp = diag && c + 1 == chunks && lane == 0 ? (i < n ? (*diag)[(size_t)i] : -2) : -1;
-                        slot(p, dp, (uint32_t)(p >= 0 ? fci[(size_t)p] : n) | ((uint32_t)i << 14) | flags);
+                    const auto r = i < n ? range(i) : std::make_pair(0, 0);
+                    if (diag && c + 1 == chunks) out.dpos[at] = i < n ? (*diag)[(size_t)i] : -2;
+                    for (int lane = 0; lane < L; ++lane, ++at) {
+                        const int32_t p = r.first + c * L + lane;
+                        const bool some = p < r.second;
+                        if (some) out.pos[at] = p;
+                        out.slots[at].meta = (uint32_t)(some ? fci[(size_t)p] : n) | ((uint32_t)i << 14) | flags;
                     }
                 }
             }
         }
     }
-    for (; out.steps % kTriAhead; ++out.steps)   // whole multiples of kTriAhead: steps that do nothing
-        for (int k = 0; k < kTriThreads && build; ++k) slot(-1, -1, (uint32_t)n | ((uint32_t)n << 14));
 }
 
 // Rows ordered by level (counting sort, ascending row within a level); offsets per level.
@@ -533,38 +571,40 @@ extern "C" mgpu_status mgpu_ilu_create(int32_t n, const int32_t* row_ptr, const 
         // more lanes per row only where they save a quarter of the steps: fewer lanes, fewer
         // additions across them (8825 rows of 30: 8 lanes 0.19 ms, 16 lanes 0.22 ms, 4 lanes 0.31 ms)
         int best = 0;
-        int64_t best_steps = INT64_MAX;
+        int64_t steps[2] = {0, 0};
         for (int L = 4; L <= 64; L *= 2) {
-            ilu::TriStream a, b;
-            ilu::tri_stream(L, n, ord_f, F->lev_f, low, fci, nullptr, false, a);
-            ilu::tri_stream(L, n, ord_b, F->lev_b, upp, fci, &diag, false, b);
-            if (best == 0 || 4 * (a.steps + b.steps) < 3 * best_steps) {
+            const int64_t sf = ilu::tri_steps(L, ord_f, F->lev_f, low), sb = ilu::tri_steps(L, ord_b, F->lev_b, upp);
+            if (best == 0 || 4 * (sf + sb) < 3 * (steps[0] + steps[1])) {
                 best = L;
-                best_steps = a.steps + b.steps;
+                steps[0] = sf;
+                steps[1] = sb;
             }
         }
+        const int64_t all = steps[0] + steps[1];
+        const size_t slots = (size_t)all * ilu::kTriThreads;
         const double launches = (double)(F->lev_f.size() + F->lev_b.size() - 2);
-        if (best_steps * ilu::kTriStepUs < launches * ilu::kLevelUs) {
-            ilu::TriStream a, b;
-            for (ilu::TriStream* x : {&a, &b}) {
-                const size_t k = (size_t)best_steps * ilu::kTriThreads;
-                x->slots.reserve(k);
-                x->pos.reserve(k);
-                x->dpos.reserve(k);
+        if (all * ilu::kTriStepUs < launches * ilu::kLevelUs && slots * ilu::kTriSlotBytes <= ilu::kMaxTriBytes) {
+            try {
+                ilu::TriStream st;
+                st.slots.assign(slots, ilu::TriSlot{0.0, (uint32_t)n | ((uint32_t)n << 14), 0u});
+                st.pos.assign(slots, -1);
+                st.dpos.assign(slots, -1);
+                ilu::tri_fill(best, n, ord_f, F->lev_f, low, fci, nullptr, 0, st);
+                ilu::tri_fill(best, n, ord_b, F->lev_b, upp, fci, &diag, (size_t)steps[0] * ilu::kTriThreads, st);
+                ilu::TriSlot* sl = nullptr;
+                if (ilu::dev_upload_optional(F.get(), st.slots, &sl) &&
+                    ilu::dev_upload_optional(F.get(), st.pos, &F->tri_pos) &&
+                    ilu::dev_upload_optional(F.get(), st.dpos, &F->tri_dpos)) {
+                    F->tri_slots = sl;
+                    F->tri_lanes = best;
+                    F->n_steps[0] = (int32_t)steps[0];
+                    F->n_steps[1] = (int32_t)steps[1];
+                } else {
+                    ilu::dev_drop(F.get(), &sl);
+                    ilu::dev_drop(F.get(), &F->tri_pos);
+                }
+            } catch (const std::bad_alloc&) {   // (a launch per level)
             }
-            ilu::tri_stream(best, n, ord_f, F->lev_f, low, fci, nullptr, true, a);
-            ilu::tri_stream(best, n, ord_b, F->lev_b, upp, fci, &diag, true, b);
-            F->tri_lanes = best;
-            F->n_steps[0] = (int32_t)a.steps;
-            F->n_steps[1] = (int32_t)b.steps;
-            a.slots.insert(a.slots.end(), b.slots.begin(), b.slots.end());
-            a.pos.insert(a.pos.end(), b.pos.begin(), b.pos.end());
-            a.dpos.insert(a.dpos.end(), b.dpos.begin(), b.dpos.end());
-            ilu::TriSlot* sl = nullptr;
-            if ((rc = ilu::dev_upload(F.get(), a.slots, &sl)) || (rc = ilu::dev_upload(F.get(), a.pos, &F->tri_pos)) ||
-                (rc = ilu::dev_upload(F.get(), a.dpos, &F->tri_dpos)))
-                return rc;
-            F->tri_slots = sl;
         }
     }
     void* p = nullptr;

@@ -520,6 +520,43 @@ def test_ilu_apply_solves_with_its_factors(kind, n):
     assert np.array_equal(F.apply(v).view(np.uint64), got.view(np.uint64))
 
 
+@pytest.mark.parametrize("half,device_mib", [(1, 448), (100, 128)])
+def test_ilu_one_row_per_level(half, device_mib):
+    """A band of 16383 rows, one row per level each way (the longest schedule of the one-workgroup solve): its
+    stream takes 0.40 GB at half bandwidth 1; at 100 it would take 0.8 GB beside 40 MB of factor, and the
+    levels are launched instead.  Either way the solve agrees with one on the host (1e-12: diagonally dominant,
+    condition below 10, 200 terms a row), and the factors with K's product (rows of 200 terms, 1e-13)."""
+    print("case", half, flush=True)
+
+    def device_free():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert M.load_library().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0   # (of its HIP runtime)
+        return free.value
+
+    n = 16383
+    SV.ILU(SV.DeviceCSR([0, 1], [0], [1.0]))   # (the kernels' code is on the device)
+    rng = np.random.default_rng(half)
+    offs = [o for o in range(-half, half + 1) if o != 0]
+    K = sp.csr_matrix(sp.diags([rng.uniform(-1.0, 1.0, n - abs(o)) for o in offs], offs))
+    K = sp.csr_matrix(K + sp.diags(abs(K).sum(axis=1).A1 + 1.0))
+    K.sort_indices()
+    A = SV.DeviceCSR(K.indptr, K.indices, K.data)
+    free = device_free()
+    F = SV.ILU(A, fill_level=0)
+    used = (free - device_free()) / 2**20
+    print("device memory of the factors %.0f MiB" % used, flush=True)
+    assert used <= device_mib
+    _, rp, ci, lu, levels = F.factors()
+    assert levels == (n, n)
+    LU = sp.csr_matrix((lu, ci, rp), shape=(n, n))
+    L, U = sp.csr_matrix(sp.tril(LU, -1) + sp.eye(n)), sp.csr_matrix(sp.triu(LU))
+    assert abs(L @ U - K).max() <= 1e-13 * abs(K).max()   # (a band has no fill)
+    v = rng.uniform(-1.0, 1.0, n)
+    z = spla.spsolve_triangular(U, spla.spsolve_triangular(L, v, lower=True), lower=False)
+    got = F.apply(v)
+    assert np.linalg.norm(got - z) <= 1e-12 * np.linalg.norm(z)
+
+
 @pytest.mark.parametrize("n,dense", [(1, 0), (7, 0), (256, 0), (257, 0), (16385, 0), (70001, 0), (300, 1), (1, 1)])
 def test_cg_sizes_and_row_lengths(n, dense):
     """CG at grid edges (one row, a block, one row more, more rows than lanes of the largest grid) and with
