@@ -530,28 +530,41 @@ extern "C" mgpu_status mgpu_ilu_create(int32_t n, const int32_t* row_ptr, const 
         (rc = ilu::dev_upload(F.get(), diag, &F->diag)) || (rc = ilu::dev_upload(F.get(), pos, &F->pos)) ||
         (rc = ilu::dev_upload(F.get(), rows_f, &F->rows_f)) || (rc = ilu::dev_upload(F.get(), rows_b, &F->rows_b)))
         return rc;
-    // elimination lists: row k's upper part merged into row i for every lower entry (i, k)
-    {
-        std::vector<int64_t> up((size_t)F->nnz + 1, 0);
-        std::vector<int2> upd;
-        bool fits = true;
-        for (int32_t i = 0; i < n && fits; ++i) {
-            for (int32_t q = frp[(size_t)i]; q < frp[(size_t)i + 1]; ++q) {
+    // elimination lists: the entries of row i that row k's upper part updates, for every lower entry (i, k).
+    // Their number is estimated first, from every 64th row: patterns far beyond the limit pay for no list.
+    try {
+        std::vector<int32_t> at((size_t)n, -1);   // position of each column in the current row
+        auto row_updates = [&](int32_t i, auto hit, auto entry) {
+            const int32_t r0 = frp[(size_t)i], r1 = frp[(size_t)i + 1];
+            for (int32_t t = r0; t < r1; ++t) at[(size_t)fci[(size_t)t]] = t - r0;
+            for (int32_t q = r0; q < r1; ++q) {
                 if (q < diag[(size_t)i]) {
                     const int32_t k = fci[(size_t)q];
-                    int32_t t = q + 1;
-                    for (int32_t u = diag[(size_t)k] + 1; u < frp[(size_t)k + 1]; ++u) {
-                        while (t < frp[(size_t)i + 1] && fci[(size_t)t] < fci[(size_t)u]) ++t;
-                        if (t == frp[(size_t)i + 1]) break;
-                        if (fci[(size_t)t] == fci[(size_t)u]) upd.push_back(make_int2(t - frp[(size_t)i], u));
-                    }
+                    for (int32_t u = diag[(size_t)k] + 1; u < frp[(size_t)k + 1]; ++u)
+                        if (at[(size_t)fci[(size_t)u]] >= 0) hit(at[(size_t)fci[(size_t)u]], u);
                 }
-                up[(size_t)q + 1] = (int64_t)upd.size();
+                entry(q);
             }
+            for (int32_t t = r0; t < r1; ++t) at[(size_t)fci[(size_t)t]] = -1;
+        };
+        size_t expected = 0;
+        for (int32_t i = 0; i < n; i += 64) row_updates(i, [&](int32_t, int32_t) { expected += 64; }, [](int32_t) {});
+        bool fits = expected <= ilu::kMaxUpdates;
+        std::vector<int64_t> up;
+        std::vector<int2> upd;
+        if (fits) {
+            up.assign((size_t)F->nnz + 1, 0);
+            upd.reserve(expected + expected / 8);
+        }
+        for (int32_t i = 0; i < n && fits; ++i) {
+            row_updates(i, [&](int32_t x, int32_t u) { upd.push_back(make_int2(x, u)); },
+                        [&](int32_t q) { up[(size_t)q + 1] = (int64_t)upd.size(); });
             fits = upd.size() <= ilu::kMaxUpdates;
         }
-        if (fits && !upd.empty())
-            if ((rc = ilu::dev_upload(F.get(), up, &F->upd_ptr)) || (rc = ilu::dev_upload(F.get(), upd, &F->upd))) return rc;
+        if (fits && !upd.empty() && ilu::dev_upload_optional(F.get(), up, &F->upd_ptr) &&
+            !ilu::dev_upload_optional(F.get(), upd, &F->upd))
+            ilu::dev_drop(F.get(), &F->upd_ptr);
+    } catch (const std::bad_alloc&) {   // (the rows are searched)
     }
     // one workgroup for the triangular solves where its steps take less time than the levels' launches
     if (n > 0 && n <= ilu::kTriMaxRows) {

@@ -557,6 +557,29 @@ def test_ilu_one_row_per_level(half, device_mib):
     assert np.linalg.norm(got - z) <= 1e-12 * np.linalg.norm(z)
 
 
+@pytest.mark.parametrize("n,half,long_every_64th", [(130, 20, False), (130, 20, True), (12000, 60, False)])
+def test_ilu_rows_of_differing_length(n, half, long_every_64th):
+    """ILU(0) reproduces K on K's pattern (rows of at most 121 terms: 1e-13), whatever the rows that the number
+    of its updates is estimated from: every 64th row is a diagonal entry only, the others are a band (more
+    updates than expected, at n = 12000 more than the lists take), or the other way round."""
+    print("case", n, half, long_every_64th, flush=True)
+    rng = np.random.default_rng(n)
+    offs = [o for o in range(-half, half + 1) if o != 0]
+    keep = sp.diags(((np.arange(n) % 64 == 0) == long_every_64th).astype(float))
+    K = sp.csr_matrix(keep @ sp.diags([rng.uniform(-1.0, 1.0, n - abs(o)) for o in offs], offs))
+    K.eliminate_zeros()
+    K = sp.csr_matrix(K + sp.diags(abs(K).sum(axis=1).A1 + 1.0))
+    K.sort_indices()
+    A = SV.DeviceCSR(K.indptr, K.indices, K.data)
+    F = SV.ILU(A, fill_level=0)
+    _, rp, ci, lu, _ = F.factors()
+    assert np.array_equal(rp, K.indptr) and np.array_equal(ci, K.indices)
+    LU = sp.csr_matrix((lu, ci, rp), shape=(n, n))
+    D = (sp.tril(LU, -1) + sp.eye(n)) @ sp.triu(LU) - K
+    pattern = sp.csr_matrix((np.ones(len(ci)), ci, rp), shape=(n, n))
+    assert abs(D.multiply(pattern)).max() <= 1e-13 * abs(K).max()
+
+
 @pytest.mark.parametrize("n,dense", [(1, 0), (7, 0), (256, 0), (257, 0), (16385, 0), (70001, 0), (300, 1), (1, 1)])
 def test_cg_sizes_and_row_lengths(n, dense):
     """CG at grid edges (one row, a block, one row more, more rows than lanes of the largest grid) and with
