@@ -102,7 +102,7 @@ __global__ __launch_bounds__(kThreads) void k_diag_inv(int32_t n, const int32_t*
     if (r >= n) return;
     int32_t lo = rp[r], hi = rp[r + 1];
     while (lo < hi) {   // sorted columns: binary search for the diagonal
-        const int32_t m = (lo + hi) >> 1;
+        const int32_t m = lo + ((hi - lo) >> 1);
         if (ci[m] < r) lo = m + 1;
         else hi = m;
     }
@@ -130,18 +130,20 @@ __global__ __launch_bounds__(kThreads) void k_spmv(int32_t n, const int32_t* rp,
     const int64_t row0 = (int64_t)blockIdx.x * G + g, stride = (int64_t)gridDim.x * G;
     int32_t next0 = row0 < n ? rp[row0] : 0, next1 = row0 < n ? rp[row0 + 1] : 0;
     for (int64_t row = row0; row < n; row += stride) {
-        const int32_t r = (int32_t)row, k0 = next0, k1 = next1;
+        const int32_t r = (int32_t)row;
+        const uint32_t k0 = next0, k1 = next1;
         if (row + stride < n) {
             next0 = rp[row + stride];
             next1 = rp[row + stride + 1];
         }
         double s = 0.0;
-        for (int32_t k = k0 + lane; k < k1; k += kSpmvAhead * L) {
+        // (unsigned: an index ahead of the last row's end may pass the largest int32)
+        for (uint32_t k = k0 + lane; k < k1; k += kSpmvAhead * L) {
             double v[kSpmvAhead], xv[kSpmvAhead];
             int32_t c[kSpmvAhead];
 #pragma unroll
             for (int t = 0; t < kSpmvAhead; ++t) {
-                const int32_t kt = min(k + t * L, k1 - 1);
+                const uint32_t kt = min(k + t * L, k1 - 1);
                 v[t] = vals[kt];
                 c[t] = ci[kt];
             }

@@ -81,7 +81,7 @@ __global__ __launch_bounds__(kThreads) void k_gm_dinv(int32_t n, const int32_t* 
     if (r >= n) return;
     int32_t lo = rp[r], hi = rp[r + 1];
     while (lo < hi) {
-        const int32_t mid = (lo + hi) >> 1;
+        const int32_t mid = lo + ((hi - lo) >> 1);
         if (ci[mid] < r) lo = mid + 1;
         else hi = mid;
     }
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(kThreads) void k_gm_spmv(int32_t n, const int32_t* 
     for (int64_t row = (int64_t)blockIdx.x * G + g; row < n; row += (int64_t)gridDim.x * G) {
         const int32_t r = (int32_t)row;
         double s = 0.0;
-        for (int32_t k = rp[r] + lane; k < rp[r + 1]; k += L) {
+        for (int64_t k = (int64_t)rp[r] + lane; k < rp[r + 1]; k += L) {
             const int32_t c = ci[k];
             s += (RESID || !JAC) ? vals[k] * x[c] : vals[k] * (dinv[c] * x[c]);
         }

@@ -135,7 +135,7 @@ __global__ __launch_bounds__(64) void k_ilu_row(const int32_t* rows, const int32
                 const int j = c[q];
                 int lo = u0, hi = u1;
                 while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
+                    const int mid = lo + ((hi - lo) >> 1);
                     if (ci[mid] < j) lo = mid + 1;
                     else hi = mid;
                 }
