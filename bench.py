@@ -175,11 +175,9 @@ def run_hex27(args):
                                                                          P.n_ig))
     S = M.Set(P.desc, keepalive=P)
     t_host = time.time() - t0
-    # sets whose element matrices exceed 2^30 entries assemble in scatter mode (no K_e pool);
-    # MGPU_GENERIC_SCATTER=1 / =0 forces it on / off
+    # how the set sums K: row by row from the K_e pool, by lists, or (large sets) scatter mode without one
     ke_entries = int(np.sum(np.diff(S.topology_offsets()).astype(np.int64) ** 2))
-    force = os.environ.get("MGPU_GENERIC_SCATTER", "")[:1]
-    mode = "scatter" if force == "1" or (ke_entries > 2 ** 30 and force != "0") else "gather"
+    mode = ("stencil", "rows", "lists", "scatter")[S.statistics()[7]]
     log("hex27 setup %.1fs: %d^3, elements %d, cut %d, sub-tets %d, rows %d, nnz %d, %s mode" % (
         time.time() - t0, n, P.n_elements, P.n_cut, P.n_ig, S.n_rows, S.nnz, mode))
     u = np.random.default_rng(SEED + 27).uniform(-1.0, 1.0, S.n_rows)

@@ -258,7 +258,10 @@ mgpu_status mgpu_set_stats(const mgpu_set* set, int64_t stats[5]);
 /* The same statistics and more, the first n_stats of: [0]..[4] as mgpu_set_stats, [5] integration
    points skipped because their sub-cell has detJ < -1e-6 (Element_Bulk::compute_jacobian_and_
    residual, cl_FEM_Element_Bulk.cpp:291 -- a reported statistic, not an error), [6] such
-   sub-cells.  Entries beyond [6] are set to 0.                                                */
+   sub-cells, [7] how K is summed: 0 lattice stencil, 1 row by row from a pool of element
+   matrices, 2 from that pool by lists of entries, 3 by colour classes without a pool (large HEX27
+   sets, also where the pool would take much of the free memory; one order of summation per form,
+   so K agrees between them to rounding).  Entries beyond [7] are set to 0.                    */
 mgpu_status mgpu_set_statistics(const mgpu_set* set, int64_t* stats, int32_t n_stats);
 
 /* Device helpers (so callers need no HIP headers). */

@@ -471,9 +471,10 @@ class Set:
         return list(s)
 
     def statistics(self):
-        """mgpu_set_statistics: stats() plus [5] points and [6] sub-cells skipped for detJ < -1e-6."""
-        s = (ctypes.c_int64 * 7)()
-        _check(load_library().mgpu_set_statistics(self._h, s, 7), "mgpu_set_statistics")
+        """mgpu_set_statistics: stats() plus [5] points and [6] sub-cells skipped for detJ < -1e-6, [7] how K is
+        summed (0 stencil, 1 rows, 2 lists, 3 colour classes)."""
+        s = (ctypes.c_int64 * 8)()
+        _check(load_library().mgpu_set_statistics(self._h, s, 8), "mgpu_set_statistics")
         return list(s)
 
     def close(self):

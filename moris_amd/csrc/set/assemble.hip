@@ -974,15 +974,16 @@ extern "C" mgpu_status mgpu_set_stats(const mgpu_set* set, int64_t stats[5]) {
 
 extern "C" mgpu_status mgpu_set_statistics(const mgpu_set* set, int64_t* stats, int32_t n_stats) {
     if (!set || (!stats && n_stats > 0) || n_stats < 0) return set_error(MGPU_ERR_INVALID_ARG, "bad argument");
-    int64_t all[7];
+    int64_t all[8];
     mgpu_status rc = mgpu_set_stats(set, all);
     if (rc != MGPU_OK) return rc;
     // points of sub-cells with detJ < -1e-6 are skipped in every mode; the learned path skips
     // them only on its fallback elements (its accepted elements use 27 points of the IP cell)
     all[5] = set->h.n_skip_points;
     all[6] = set->h.n_skip_subcells;
-    for (int32_t i = 0; i < n_stats && i < 7; ++i) stats[i] = all[i];
-    for (int32_t i = 7; i < n_stats; ++i) stats[i] = 0;
+    all[7] = !set->h.generic ? 0 : (set->h.scatter ? 3 : (set->h.rows ? 1 : 2));
+    for (int32_t i = 0; i < n_stats && i < 8; ++i) stats[i] = all[i];
+    for (int32_t i = 8; i < n_stats; ++i) stats[i] = 0;
     return MGPU_OK;
 }
 

@@ -285,6 +285,28 @@ __global__ __launch_bounds__(256) void k_generic_rhs(GenView g, const double* va
 mgpu_status generic_upload(mgpu_set* S, const mgpu_set_desc& d) {
     const SetHost& h = S->h;
     GenView& g = S->g;
+    // the K_e pool first: large HEX27 sets do without where the memory is short
+    const size_t n_ke = h.ke_off.empty() ? 0 : (size_t)h.ke_off.back();
+    if (n_ke > 0 && !h.scatter) {
+        void* p = nullptr;
+        const bool optional = h.nb == 27 && h.rows && (int64_t)n_ke > kGatherMaxEntries;
+        bool pool = true;
+        if (optional) {
+            size_t free_bytes = 0, total = 0;
+            pool = hipMemGetInfo(&free_bytes, &total) == hipSuccess &&
+                   !scatter_by_memory(h.nb, h.rows, (int64_t)n_ke, free_bytes) &&
+                   hipMalloc(&p, n_ke * sizeof(double)) == hipSuccess;
+            if (!pool) (void)hipGetLastError();
+        } else {
+            HIP_TRY(hipMalloc(&p, n_ke * sizeof(double)));
+        }
+        if (pool) {
+            S->allocs.push_back(p);
+            g.ke = static_cast<double*>(p);
+        } else {
+            rows_to_scatter(d, S->h);
+        }
+    }
     g.n_el = h.n_el;
     g.N = h.n_adofs_type;
     g.n_rows = h.n_rows;
@@ -380,13 +402,6 @@ mgpu_status generic_upload(mgpu_set* S, const mgpu_set_desc& d) {
                 (rc = gupload(S, order.data(), order.size(), const_cast<int32_t**>(&S->d_els_order))))
                 return rc;
         }
-    }
-    const size_t n_ke = h.ke_off.empty() ? 0 : (size_t)h.ke_off.back();
-    if (n_ke > 0) {
-        void* p = nullptr;
-        HIP_TRY(hipMalloc(&p, n_ke * sizeof(double)));
-        S->allocs.push_back(p);
-        g.ke = static_cast<double*>(p);
     }
     return MGPU_OK;
 }

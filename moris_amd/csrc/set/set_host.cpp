@@ -71,6 +71,56 @@ static void tensor_form(const double* D, int nb, uint8_t* perm) {
     perm[27] = 0;
 }
 
+// Scatter mode: the elements of HEX27 sets in colour classes that share no adof.  a_ptr, a_el: the
+// elements holding each adof.
+static void colour_elements(const mgpu_set_desc& d, SetHost& h, const std::vector<int64_t>& a_ptr,
+                            const std::vector<int32_t>& a_el) {
+    // greedy colouring in element order: the smallest colour that no element sharing an
+    // adof with e already holds
+    std::vector<int32_t> colour((size_t)h.n_el, -1), seen;
+    int32_t n_col = 0;
+    for (int32_t e = 0; e < h.n_el; ++e) {
+        for (int32_t x = 0; x < h.na_t[(size_t)e]; ++x) {
+            const int32_t a = h.topo[(size_t)h.topo_ptr[(size_t)e] + x];   // (field 0: the adof itself)
+            for (int64_t q = a_ptr[(size_t)a]; q < a_ptr[(size_t)a + 1]; ++q) {
+                const int32_t c = colour[(size_t)a_el[(size_t)q]];
+                if (c >= 0) seen[(size_t)c] = e;
+            }
+        }
+        int32_t c = 0;
+        while (c < n_col && seen[(size_t)c] == e) ++c;
+        if (c == n_col) {
+            ++n_col;
+            seen.push_back(-1);
+        }
+        colour[(size_t)e] = c;
+    }
+    h.colour_ptr.assign((size_t)n_col + 1, 0);
+    for (int32_t e = 0; e < h.n_el; ++e) h.colour_ptr[(size_t)colour[(size_t)e] + 1]++;
+    for (int32_t c = 0; c < n_col; ++c) h.colour_ptr[(size_t)c + 1] += h.colour_ptr[(size_t)c];
+    h.colour_el.resize((size_t)h.n_el);
+    {
+        std::vector<int32_t> fill(h.colour_ptr.begin(), h.colour_ptr.end() - 1);
+        for (int32_t e = 0; e < h.n_el; ++e) h.colour_el[(size_t)fill[(size_t)colour[(size_t)e]]++] = e;
+    }
+    // within a colour the elements with most sub-cells first, so that a launch does not end
+    // on one long element
+    for (int32_t c = 0; c < n_col; ++c)
+        std::stable_sort(h.colour_el.begin() + h.colour_ptr[(size_t)c], h.colour_el.begin() + h.colour_ptr[(size_t)c + 1],
+                         [&](int32_t x, int32_t y) {
+                             return d.ig_ptr[x + 1] - d.ig_ptr[x] > d.ig_ptr[y + 1] - d.ig_ptr[y];
+                         });
+}
+
+void rows_to_scatter(const mgpu_set_desc& d, SetHost& h) {
+    colour_elements(d, h, h.adof_ptr, h.adof_el);
+    h.rows = false;
+    h.scatter = true;
+    h.adof_ptr = {};
+    h.adof_el = {};
+    h.adof_x = {};
+}
+
 // Generic path: element topology of any T rows (sorted unique adofs per type), element-local T
 // columns, the CSR pattern as the union of the topologies (Sparse_Matrix_EpetraFECrs::build_graph,
 // cl_Sparse_Matrix_EpetraFECrs.cpp:195-240) and, per adof, the elements whose matrices are summed into
@@ -199,49 +249,15 @@ mgpu_status build_generic(const mgpu_set_desc& d, SetHost& h, std::string* err) 
         }
     const int64_t n_src = h.ke_off[(size_t)h.n_el];
     for (int32_t a = 0; a < N; ++a) h.max_nbr = std::max(h.max_nbr, (int32_t)nbr[(size_t)a].size());
-    h.scatter = nb == 27 && n_src > kGatherMaxEntries;
     h.rows = (int64_t)nf * h.max_nbr * (int64_t)sizeof(double) <= kRowsMaxLds;
+    h.scatter = scatter_by_size(nb, h.rows, n_src);
     if (nb == 27)
         if (const char* env = std::getenv("MGPU_GENERIC_SCATTER")) {
             if (env[0] == '1') h.scatter = true;
             if (env[0] == '0') h.scatter = h.rows = false;
         }
     if (h.scatter) h.rows = false;
-    if (h.scatter) {
-        // greedy colouring in element order: the smallest colour that no element sharing an
-        // adof with e already holds
-        std::vector<int32_t> colour((size_t)h.n_el, -1), seen;
-        int32_t n_col = 0;
-        for (int32_t e = 0; e < h.n_el; ++e) {
-            for (int32_t a : loc[(size_t)e])
-                for (int64_t q = a_ptr[(size_t)a]; q < a_ptr[(size_t)a + 1]; ++q) {
-                    const int32_t c = colour[(size_t)a_el[(size_t)q]];
-                    if (c >= 0) seen[(size_t)c] = e;
-                }
-            int32_t c = 0;
-            while (c < n_col && seen[(size_t)c] == e) ++c;
-            if (c == n_col) {
-                ++n_col;
-                seen.push_back(-1);
-            }
-            colour[(size_t)e] = c;
-        }
-        h.colour_ptr.assign((size_t)n_col + 1, 0);
-        for (int32_t e = 0; e < h.n_el; ++e) h.colour_ptr[(size_t)colour[(size_t)e] + 1]++;
-        for (int32_t c = 0; c < n_col; ++c) h.colour_ptr[(size_t)c + 1] += h.colour_ptr[(size_t)c];
-        h.colour_el.resize((size_t)h.n_el);
-        {
-            std::vector<int32_t> fill(h.colour_ptr.begin(), h.colour_ptr.end() - 1);
-            for (int32_t e = 0; e < h.n_el; ++e) h.colour_el[(size_t)fill[(size_t)colour[(size_t)e]]++] = e;
-        }
-        // within a colour the elements with most sub-cells first, so that a launch does not end
-        // on one long element
-        for (int32_t c = 0; c < n_col; ++c)
-            std::stable_sort(h.colour_el.begin() + h.colour_ptr[(size_t)c], h.colour_el.begin() + h.colour_ptr[(size_t)c + 1],
-                             [&](int32_t x, int32_t y) {
-                                 return d.ig_ptr[x + 1] - d.ig_ptr[x] > d.ig_ptr[y + 1] - d.ig_ptr[y];
-                             });
-    }
+    if (h.scatter) colour_elements(d, h, a_ptr, a_el);
     if (h.scatter || h.rows) {
         // rank tables: both the element's adofs and each adof's neighbours are ascending, so
         // one merge per row finds every column

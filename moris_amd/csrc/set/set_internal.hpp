@@ -21,10 +21,21 @@ constexpr int kHex27Moments = 125;      // moments of degree <= 4 per axis of an
 constexpr int kHex27MomTab = 126;       // and from here the coefficients of its 1D functions (hex27.hip)
 constexpr int kHex27MomStride = 180;    // doubles of an element's record
 constexpr int kHex27PermStride = 28;    // SetHost::t_perm entries of an element
-// HEX27 sets whose element matrices hold more entries than this (a K_e pool of 8 GiB) take the
-// scatter mode, which keeps no pool but is slower: 40^3 elements of 81 x 81 (3.4 GiB), elasticity:
-// 4.1 ms with the pool, 8.0 ms without.  MGPU_GENERIC_SCATTER=1 forces it on, =0 forces it off and the gather lists.
-constexpr int64_t kGatherMaxEntries = (int64_t)1 << 30;
+// Large HEX27 sets take the scatter mode, which keeps no K_e pool but is slower (elasticity: 56000 elements of
+// 81 x 81, a pool of 2.7 GiB, 2.6 ms with the pool and 6.2 without; 109375 elements, 5.3 GiB, 4.9 and 12.3; 50000
+// elements of one THB level, 2.4 GiB, 2.2 and 5.5).  In rows mode, where the pool is all they keep: those with
+// more entries than kRowsMaxEntries (8 GiB), and those with more than kGatherMaxEntries (2 GiB) whose
+// pool would take more than an eighth of the device's free memory, so that many sets held together leave
+// room.  Sets that need gather lists (as much again, and more on the host): those with more than
+// kGatherMaxEntries.  MGPU_GENERIC_SCATTER=1 forces the scatter mode, =0 the pool with gather lists.
+constexpr int64_t kGatherMaxEntries = (int64_t)1 << 28;
+constexpr int64_t kRowsMaxEntries = (int64_t)1 << 30;
+constexpr bool scatter_by_size(int nb, bool rows, int64_t entries) {
+    return nb == 27 && entries > (rows ? kRowsMaxEntries : kGatherMaxEntries);
+}
+constexpr bool scatter_by_memory(int nb, bool rows, int64_t entries, size_t free_bytes) {
+    return nb == 27 && rows && entries > kGatherMaxEntries && (size_t)entries * sizeof(double) > free_bytes / 8;
+}
 // LDS of one row's values in the row-wise sums (k_generic_rows); sets with a longer row keep gather lists
 constexpr int kRowsMaxLds = 32768;
 
@@ -93,5 +104,7 @@ struct SetHost {
 // Build topology, pattern and the lattice maps from a descriptor.  Returns MGPU_OK or an error
 // code with *err set.
 mgpu_status build_set_host(const mgpu_set_desc& d, SetHost& h, std::string* err);
+// A HEX27 set in rows mode turned into one in scatter mode.
+void rows_to_scatter(const mgpu_set_desc& d, SetHost& h);
 
 }  // namespace mgpu

@@ -318,6 +318,38 @@ def test_thb_scatter_mode_chosen_by_size_properties():
     assert rel(vm, vals) <= 1e-6 and rel(Rm, R) <= 1e-6
 
 
+def _device_free():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert M.load_library().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0   # (of its HIP runtime)
+    return free.value
+
+
+@pytest.mark.parametrize("left_gib", [3, 12])
+def test_large_hex27_set_where_memory_is_short(left_gib):
+    """A HEX27 set of 3.7e8 element-matrix entries (a pool of 2.7 GiB) with most of the device's memory
+    taken: it assembles without the pool, whether that would not fit (3 GiB left) or would take more
+    than an eighth of what is left (12 GiB); with the memory free it keeps the pool.  Both sum the same element
+    matrices, up to 27 a value, in another order: 27 x 1.1e-16; R rows of 375 such values."""
+    n = 40
+    spec, keep = M.make_spec(3, (n, n, n), iwg=M.IWG_STRUC_LINEAR_BULK, ls_kind=M.LS_GYROID,
+                             gyroid_scale=2 * np.pi * n / 4.0, bspline_order=2, lagrange_order=2)
+    P = M.Problem(spec, keep)
+    u = np.random.default_rng(SEED + 54).uniform(-1.0, 1.0, 3 * P.n_adofs_per_type)
+    S = M.Set(P.desc, keepalive=P)
+    assert S.statistics()[7] == 1
+    v1, R1 = S.compute_jacobian_and_residual(u)
+    S.close()
+    taken = M.DeviceBuffer(_device_free() - (left_gib << 30))
+    try:
+        S = M.Set(P.desc, keepalive=P)
+        assert S.statistics()[7] == 3
+        v2, R2 = S.compute_jacobian_and_residual(u)
+        S.close()
+    finally:
+        taken.free()
+    assert rel(v2, v1) <= 1e-14 and rel(R2, R1) <= 1e-13
+
+
 @pytest.mark.parametrize("scatter", ["", "0", "1"])
 @pytest.mark.parametrize("order", [1, 2])
 def test_hex27_tensor_and_general_rows(order, scatter, monkeypatch):
