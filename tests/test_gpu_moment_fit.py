@@ -1,22 +1,19 @@
-"""GPU tests of the moment-fitted quadrature of cut HEX27 cells (MGPU_QUAD_MOMENT_FIT): each cut
-cell's TET_35 points replaced by the 5 x 5 x 5 Gauss-Legendre nodes weighted by the cell's degree-4
-Lagrange moments over those points, which gives the subdivision's sum for every integrand of degree
-<= 4 per axis, the box HEX27 stiffness among them.
+"""GPU tests of the moment-fitted quadrature (MGPU_QUAD_MOMENT_FIT).  Generic sets take K from the cells'
+moments over the sub-cells' points (degree 4 per axis on HEX27, 2 on HEX8 / QUAD4) with either quadrature
+and at either precision option; 3D lattice sets have a fitted 27-point rule of their own.
 
-* against the oracle (TET_35 on every sub-tet) at 1e-12 on the FP64 path and 1e-6 on the mixed
-  path: p = 2 B-spline and nodal rows, diffusion and elasticity, one THB level, an enriched set;
-  pattern unchanged; repeated calls bit-identical;
+* against the oracle (TET_35 on every sub-tet) at 1e-12, and bit-identical with the other quadrature and
+  precision options: p = 2 B-spline and nodal rows, diffusion and elasticity, one THB level, an
+  enriched set; pattern unchanged; repeated calls bit-identical;
 * scatter mode (colour classes) to the same bars;
-* size-independent on a 16^3 gyroid HEX27 set and a 12^3-base THB set: within 1e-12 of the
-  subdivision path on the GPU;
-* an element given as 750 sub-tets tiling its box (several staging batches of the weight fit): fit,
+* a 16^3 gyroid HEX27 set and a 12^3-base THB set: bit-identical with all four options;
+* an element given as 750 sub-tets tiling its box (several staging batches of the moments): fit,
   subdivision and oracle within 1e-12, and within 1e-8 of the uncut HEX_3x3x3 element (the TET_35
   sum over the tiling differs from it by 9e-10 on M, computed on the CPU);
 * 3D lattice (hex8) sets: the 27 HEX_3x3x3 weights from the degree-2 Lagrange moments; K and R
   against the oracle at 1e-6 (FP32 MFMA product), every cut element accepted, the weights summing
   to each element's material volume; refused in 2D;
-* generic-path HEX8 / QUAD4 cells (p = 2 and THB rows): 3 nodes per axis, TET_11 / TRI_7 points,
-  against the oracle at 1e-12 (FP64) and 1e-6 (mixed).
+* generic-path HEX8 / QUAD4 cells (p = 2 and THB rows), TET_11 / TRI_7 points: against the oracle at 1e-12.
 """
 import numpy as np
 import pytest
@@ -60,10 +57,11 @@ def _check_against_oracle(S, spec):
     assert rel(vals, vo) <= 1e-12 and rel(R, Ro) <= 1e-12
     v2, R2 = S.compute_jacobian_and_residual(u)
     assert np.array_equal(v2.view(np.uint64), vals.view(np.uint64)) and np.array_equal(R2.view(np.uint64), R.view(np.uint64))
-    S.options(M.PREC_MIXED, M.QUAD_MOMENT_FIT)
-    vm, Rm = S.compute_jacobian_and_residual(u)
-    print("mixed moment fit vs oracle |dK|/|K| %.2e" % rel(vm, vo), flush=True)
-    assert rel(vm, vo) <= 1e-6 and rel(Rm, Ro) <= 1e-6
+    # generic sets: one path, at either precision and with either quadrature option
+    for prec, quad in ((M.PREC_MIXED, M.QUAD_MOMENT_FIT), (M.PREC_FP64, M.QUAD_SUBDIVISION)):
+        S.options(prec, quad)
+        vm, Rm = S.compute_jacobian_and_residual(u)
+        assert np.array_equal(vm.view(np.uint64), vals.view(np.uint64)) and np.array_equal(Rm.view(np.uint64), R.view(np.uint64))
 
 
 @pytest.mark.parametrize("case", sorted(CASES))
@@ -100,10 +98,10 @@ def test_moment_fit_equals_subdivision_on_larger_sets(refine):
     v_fit, R_fit = S.compute_jacobian_and_residual(u)
     S.options(M.PREC_MIXED, M.QUAD_MOMENT_FIT)
     v_mix, _ = S.compute_jacobian_and_residual(u)
-    print("elements", P.n_elements, "fit vs subdivision %.2e, mixed fit %.2e" % (rel(v_fit, v_sub), rel(v_mix, v_sub)),
-          flush=True)
-    assert rel(v_fit, v_sub) <= 1e-12 and rel(R_fit, R_sub) <= 1e-12
-    assert rel(v_mix, v_sub) <= 1e-6
+    print("elements", P.n_elements, flush=True)
+    for v in (v_fit, v_mix):
+        assert np.array_equal(v.view(np.uint64), v_sub.view(np.uint64))
+    assert np.array_equal(R_fit.view(np.uint64), R_sub.view(np.uint64))
 
 
 GENERIC_LINEAR = {
@@ -121,9 +119,8 @@ GENERIC_LINEAR = {
 
 @pytest.mark.parametrize("case", sorted(GENERIC_LINEAR))
 def test_generic_hex8_quad4_moment_fit_matches_oracle(case):
-    """Generic-path HEX8 / QUAD4 cells (p = 2 and THB rows): the 3^dim tensor Gauss points with the
-    degree-2 Lagrange moments of the TET_11 / TRI_7 points as weights; K and R against the oracle at
-    1e-12 (FP64) and 1e-6 (mixed)."""
+    """Generic-path HEX8 / QUAD4 cells (p = 2 and THB rows), their degree-2 moments over the TET_11 / TRI_7
+    points: K and R against the oracle at 1e-12, the same bits with every option."""
     print("case", case, flush=True)
     spec, keep = GENERIC_LINEAR[case]()
     P = M.Problem(spec, keep)
