@@ -52,14 +52,12 @@ def log(*a):
 # with two rocprofv3 --pmc runs (FETCH_SIZE scaled x2.0, WRITE_SIZE x1.0 by the copy-kernel
 # calibration): 97,555 KiB x 2 + 445,915 KiB.
 STENCIL_TRAFFIC_BYTES = (97555 * 2 + 445915) * 1024
-# The same for an earlier HEX27 element kernel, k_generic_hex27<3,double,false>, on the 32^3 gyroid set:
-# 109,644 KiB fetched, 1,470,336 KiB written (the K_e pool, which k_hex27_tensor writes now; its counters
-# have not been taken, so no line reports these bytes).
-HEX27_32_TRAFFIC_BYTES = (109644 * 2 + 1470336) * 1024
-# The same for the earlier k_generic_hex27<3,double,true,false> on the 48^3-base THB gyroid set (scatter mode,
-# FP64 atomic adds), summed over the 42 colour launches of one call: 4,423,474 KiB fetched,
-# 70,966,197 KiB written (the atomics count as write requests only).
-THB48_SCATTER_TRAFFIC_BYTES = (4423474 * 2 + 70966197) * 1024
+# The same for the HEX27 element kernels (k_hex27_moments + k_hex27_tensor) on the 32^3 gyroid set: 45,000 +
+# 35,577 KiB fetched, 40,331 + 1,470,490 KiB written (the moments and the K_e pool).
+HEX27_32_TRAFFIC_BYTES = ((45000 + 35577) * 2 + 40331 + 1470490) * 1024
+# The same on the 48^3-base THB gyroid set (scatter mode, FP64 atomic adds), summed over the 42 colour launches
+# of one call (the atomics count as write requests only).
+THB48_SCATTER_TRAFFIC_BYTES = ((796369 + 2786420) * 2 + 972019 + 63171062) * 1024
 # The same for the FP64 k_stencil<3,1,ROWS,DIRECT,double> of the 128^3 diffusion set, per stencil
 # variant (the autotuner's choice): (FETCH_SIZE, WRITE_SIZE) KiB per launch.
 C2_STENCIL_TRAFFIC_KIB = {0: (100537, 428126), 1: (94277, 433217), 2: (68008, 426869),
@@ -204,7 +202,7 @@ def run_hex27(args):
             (M.PREC_FP64, M.QUAD_MOMENT_FIT, "fp64_moment_fit"), (M.PREC_MIXED, M.QUAD_MOMENT_FIT, "mixed_moment_fit"))
     for prec, quad, name in legs:
         S.options(prec, quad)
-        S.autotune(ub, vb, rb, iters=2)   # element order of the gather mode
+        S.autotune(ub, vb, rb, iters=2)   # element order of the pool's kernels
         per, st = S.time_assemble(ub, vb, rb, max(3, args.steps))
         res[name] = (vb.to_array(np.float64, S.nnz), rb.to_array(np.float64, S.n_rows))
         out[name] = {"value": P.n_elements / (per * 1e-3), "ms_per_call": per,
@@ -225,6 +223,14 @@ def run_hex27(args):
                        "achieved": out["fp64"]["element_kernels_TFLOP/s"], "peak": FP64_PEAK_TFLOPS,
                        "unit": "TFLOP/s", "frac": out["fp64"]["element_kernels_TFLOP/s"] / FP64_PEAK_TFLOPS,
                        "traffic": None}
+    if n == 32 and not args.refine and mode == "rows":
+        out["roofline"]["traffic"] = HEX27_32_TRAFFIC_BYTES
+        out["roofline"]["traffic_source"] = "rocprofv3 --pmc FETCH_SIZE (x2.0) + WRITE_SIZE (x1.0) per call"
+    elif n == 48 and args.refine == 1 and mode == "scatter":
+        out["roofline"]["traffic"] = THB48_SCATTER_TRAFFIC_BYTES
+        out["roofline"]["traffic_source"] = ("rocprofv3 --pmc FETCH_SIZE (x2.0) + WRITE_SIZE (x1.0), summed over "
+                                             "the colour launches of one call; the atomic adds count as write "
+                                             "requests only, so this is a lower bound")
     if not args.refine:
         # the set-up of the same set on the GPU (cut, numbering, T rows at the 27 nodes, pattern)
         from moris_amd import gpu_setup as G

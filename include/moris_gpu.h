@@ -287,8 +287,8 @@ mgpu_status mgpu_set_time_assemble(mgpu_set* set, const double* u_adof, double* 
    (0 natural, 1 longest first by sub-cell count).  Stencil variants differ in rows per workgroup
    and in how a row reaches HBM: the first half of the variants stage the workgroup's CSR range
    in LDS and write it coalesced, the second half (same row counts) store each row directly.
-   Generic-path sets have no stencil: their shape is the order of the element workgroups of the
-   gather mode (0 element order, 1 most sub-cells first; scatter mode orders each colour most
+   Generic-path sets have no stencil: their shape is the order of the element workgroups of sets
+   with an element-matrix pool (0 element order, 1 most sub-cells first; scatter mode orders each colour most
    sub-cells first itself), and the autotuner times only (0, 0) and (0, 1).
    Results are bit-identical for every shape.                                                   */
 mgpu_status mgpu_set_tuning(mgpu_set* set, int32_t stencil_variant, int32_t cut_order);

@@ -37,7 +37,7 @@ TuneKey tune_key(const mgpu_set* S) {
 }
 
 // Generic sets have one launch shape per element order (no stencil); the order applies to the
-// gather mode's element workgroups (scatter mode orders within each colour itself).
+// element workgroups of sets with a K_e pool (scatter mode orders within each colour itself).
 bool order_choice(const mgpu_set* S) {
     if (S->h.generic) return !S->h.scatter && !S->h.cut_elems.empty() && S->d_gen_order;
     return S->v.n_cut > 0;

@@ -102,7 +102,7 @@ struct GenView {
     // scatter mode (HEX27 sets without a K_e pool)
     const int32_t* topo;         // rows of each element, nf * na_t from topo_ptr[e]
     const int64_t* topo_ptr;     // [n_el + 1]
-    // gather mode: the processing order of the element workgroups (most sub-cells first), or
+    // sets with a K_e pool: the processing order of the element workgroups (most sub-cells first), or
     // null for element order; the autotuner picks one
     const int32_t* order;
     const int64_t* rank_off;     // [n_el + 1]

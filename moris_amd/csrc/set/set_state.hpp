@@ -43,7 +43,7 @@ struct mgpu_set {
     int stencil_variant = -1;               // index into the stencil row-block sizes, -1 default
     int cut_order = 0;                      // 1: cut elements longest-first
     const int32_t* d_cut_order = nullptr;   // device permutation (built on first use)
-    const int32_t* d_gen_order = nullptr;   // generic sets, gather mode: elements most sub-cells first
+    const int32_t* d_gen_order = nullptr;   // generic sets with a K_e pool: elements most sub-cells first
     // moments of the elements that keep them (HEX27 cells, HEX8 cells with uniform p = 2 rows)
     double* d_mom = nullptr;
     // elements in launch order.  HEX27: (of each colour in scatter mode, else of the set) those with tensor

@@ -28,9 +28,9 @@ def test_headline_stencil_traffic_matches_its_profile():
 
 
 def test_hex27_traffic_matches_its_profile():
-    f, w = _row("k_generic_hex27_elasticity_p2_gyroid_32_hbm_traffic.md",
-                "k_generic_hex27<3,double,false> (FP64)")
-    assert bench.HEX27_32_TRAFFIC_BYTES == (2 * f + w) * 1024
+    path = "hex27_moments_elasticity_p2_gyroid_32_hbm_traffic.md"
+    (fm, wm), (f, w) = _row(path, "k_hex27_moments"), _row(path, "k_hex27_tensor<3,false>")
+    assert bench.HEX27_32_TRAFFIC_BYTES == (2 * (fm + f) + wm + w) * 1024
     # the writes are the K_e pool of the 32^3 set: 188,116,992 FP64 entries, to within 0.1 %
     assert abs(w * 1024 - 188116992 * 8) < 1e-3 * 188116992 * 8
 
@@ -51,9 +51,9 @@ def test_profiles_name_their_commands():
 
 
 def test_thb48_scatter_traffic_matches_its_profile():
-    f, w = _row("k_generic_hex27_scatter_elasticity_p2_thb_gyroid_48_hbm_traffic.md",
-                "k_generic_hex27<3,double,true,false>, 42 launches (FP64 subdivision)")
-    assert bench.THB48_SCATTER_TRAFFIC_BYTES == (2 * f + w) * 1024
+    path = "hex27_scatter_p2_thb_gyroid_48_hbm_traffic.md"
+    (fm, wm), (f, w) = _row(path, "k_hex27_moments"), _row(path, "k_hex27_tensor<3,true>, 42 launches")
+    assert bench.THB48_SCATTER_TRAFFIC_BYTES == (2 * (fm + f) + wm + w) * 1024
     # the zero fill writes the 949,141,152 FP64 values once (0.11 % over, measured), to within 0.5 %
-    _, wz = _row("k_generic_hex27_scatter_elasticity_p2_thb_gyroid_48_hbm_traffic.md", "k_generic_zero")
+    _, wz = _row(path, "k_generic_zero")
     assert abs(wz * 1024 - 949141152 * 8) < 5e-3 * 949141152 * 8
