@@ -135,6 +135,7 @@ __global__ __launch_bounds__(64) void k_hex8_moments(GenView g, const int32_t* e
         const int i = t / 25, j = (t / 5) % 5, k = t % 5;
         out[t] = i < 3 && j < 3 && k < 3 ? m[(i * 3 + j) * 3 + k] : 0.0;
     }
+    if (threadIdx.x == 0) out[kHex27Moments] = 1.0;
     if (threadIdx.x < 54) {
         const int r = threadIdx.x % 18, al = (r % 9) / 3, k = r % 3;
         out[kHex27MomTab + threadIdx.x] =

@@ -45,10 +45,10 @@ typedef double doublex4_t __attribute__((ext_vector_type(4)));
 // 6e-15, summed point by point 3e-15 .. 2e-11; a fixed basis on [-1, 1] fails either at the corners (Lagrange
 // functions and multiples of x^3 - x: 2e-12 .. 1e-4) or at the centre (Bernstein: 1e-10 .. all digits).
 //
-// A record of kHex27MomStride doubles per element: the moments, then from kHex27MomTab the coefficients
-// [axis][function, derivative][alpha][k].
+// A record of kHex27MomStride doubles per element: the moments, a factor of all of them, then from kHex27MomTab
+// the coefficients [axis][function, derivative][alpha][k].
 // ------------------------------------------------------------------------------------------------
-static_assert(kHex27MomTab + 54 <= kHex27MomStride && kHex27MomTab >= kHex27Moments, "the tables follow the moments");
+static_assert(kHex27MomTab + 54 <= kHex27MomStride && kHex27MomTab > kHex27Moments, "the tables follow the moments and their factor");
 
 // Coefficient k of 1D function alpha (0 .. 2) or its derivative on [lo, hi].  Every function is p q + c with
 // linear p, q, its coefficients p q, p q' + p' q, p' q' of their values at the ends; with u = (1 + x) / 2,
@@ -268,12 +268,15 @@ __global__ __launch_bounds__(64, 3) void k_hex27_moments(GenView g, double* mom)
         hex27_box(g, ig0, nsub, X, lds, lo, hi, sc);
         if ((int)threadIdx.x < nsub) stage_simplex<3>(X, lo, sc, vol6, lds + threadIdx.x * kMomTet);
     }
+    if (role == 0 && threadIdx.x == 0) out[kHex27Moments] = nsub == 0 ? detJ / 27000.0 : 1.0;
     if (role == 0) write_tables(g.t_perm[(size_t)e * kHex27PermStride + 27] == 2, lo, hi, out + kHex27MomTab);
     if (nsub == 0) {
-        // whole cell: products of the 1D integrals 2/5, 1/10, 1/15, 1/10, 2/5 (HEX_3x3x3 is exact for them)
+        // whole cell: products of the 1D integrals 2/5, 1/10, 1/15, 1/10, 2/5 (HEX_3x3x3 is exact for them), as
+        // integers: the contraction is exact until the record's factor is applied.  (Rounded here, the
+        // same error in every whole cell put K of a set with many of them 3.6e-16 off instead of 2.7e-16.)
         auto n30 = [](int m) { return m == 2 ? 2 : (m == 0 || m == 4 ? 12 : 3); };
         for (int t = threadIdx.x; t < kHex27Moments && role == 0; t += 64)
-            out[t] = detJ * ((double)(n30(t / 25) * n30((t / 5) % 5) * n30(t % 5)) / 27000.0);
+            out[t] = (double)(n30(t / 25) * n30((t / 5) % 5) * n30(t % 5));
     } else if (role == 0) {
         hex27_cut_moments<0>(g, ig0, nsub, vol6, lo, sc, lds, out);
     } else {
@@ -345,6 +348,7 @@ __device__ __forceinline__ void sf_moments(const GenView& g, const double* mom, 
     double line[7];
 #pragma unroll
     for (int n = 0; n < 7; ++n) line[n] = tab[8 * n < 54 ? 8 * n : 53];
+    const double factor = rec[kHex27Moments];
     double sc[3];
     for (int d = 0; d < 3; ++d) sc[d] = 2.0 / g.ip_box[(size_t)e * 6 + 3 + d];
     __syncthreads();
@@ -391,7 +395,7 @@ __device__ __forceinline__ void sf_moments(const GenView& g, const double* mom, 
         for (int pp = 0; pp < (NF == 3 ? 1 : 3); ++pp) {
             const int p = NF == 3 ? task >> 1 : pp;
             const int i = NF == 1 ? p : (p >= 3) + (p >= 5), j = NF == 1 ? p : (p < 3 ? p : (p < 5 ? p - 2 : 2));
-            const double s2 = (i == 0 ? sc[0] : (i == 1 ? sc[1] : sc[2])) * (j == 0 ? sc[0] : (j == 1 ? sc[1] : sc[2]));
+            const double s2 = factor * (i == 0 ? sc[0] : (i == 1 ? sc[1] : sc[2])) * (j == 0 ? sc[0] : (j == 1 ? sc[1] : sc[2]));
             double y[5], o[9];
 #pragma unroll
             for (int x = 0; x < 5; ++x) y[x] = s2 * Y[p * 405 + x * 81 + ab12];

@@ -18,7 +18,7 @@ constexpr int kGenericMaxAdofsPerType = 64;
 // truncated hierarchical rows up to about 40.
 constexpr int kHex27MaxAdofsPerType = 64;
 constexpr int kHex27Moments = 125;      // moments of degree <= 4 per axis of an element
-constexpr int kHex27MomTab = 126;       // and from here the coefficients of its 1D functions (hex27.hip)
+constexpr int kHex27MomTab = 126;       // then their factor, and from here the 1D functions' coefficients (hex27.hip)
 constexpr int kHex27MomStride = 180;    // doubles of an element's record
 constexpr int kHex27PermStride = 28;    // SetHost::t_perm entries of an element
 // Large HEX27 sets take the scatter mode, which keeps no K_e pool but is slower (elasticity: 56000 elements of
